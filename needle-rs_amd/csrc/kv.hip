@@ -137,7 +137,9 @@ __global__ __launch_bounds__(64) void kv_write_f32_kernel(Geom g, uint8_t *__res
 }
 
 // ---------------------------------------------------------------------------
-// Decode attention over the int8 ring, flash-decoding style.
+// Decode attention over the int8 ring with one query head a kv head,
+// flash-decoding style: the HBM stream (grouped heads share a K/V row and
+// take the matrix-core kernel below).
 //
 // Block = (query i, kv head g, split s).  It walks its share of the span in
 // chunks of CH positions with an online softmax (running max m, running sum
@@ -147,15 +149,14 @@ __global__ __launch_bounds__(64) void kv_write_f32_kernel(Geom g, uint8_t *__res
 // starts; the next chunk's K loads are issued as soon as the scores are
 // done, and its V loads as soon as the value pass is done.
 //   K: KL = qk/16 lanes per position, one 16-byte int8 vector each, the
-//      lane's 16-wide slice of every query head of the group in registers.
-//   V: VL = vd/VW lanes per position, VW bytes each (16 for up to two query
-//      heads per kv head, else 8), REP x VW accumulators per lane.
+//      lane's 16-wide slice of the query head in registers.
+//   V: VL = vd/16 lanes per position, 16 bytes each, 16 accumulators a lane.
 // Scores, weights and block reductions go through LDS.
-template <int REP, int QK, int VD, int VW>
+template <int QK, int VD>
 struct AttnShape {
     static constexpr int KL = QK / 16;
     static constexpr int KPP = kThreads / KL;                 // positions per K pass
-    static constexpr int VL = VD / VW;
+    static constexpr int VL = VD / 16;
     static constexpr int VPP = kThreads / VL;                 // positions per V pass
     // positions per chunk: 256 keeps the registers at 119 (four waves a
     // SIMD) and two chunks of a 512-long span in flight; 512 took 157
@@ -164,44 +165,29 @@ struct AttnShape {
     // 5.83 / 5.91; 384: 4.43 / 5.47 / 5.73)
     static constexpr int CH = 256;
     static constexpr int KP = (CH + KPP - 1) / KPP;           // K passes per chunk
-    // One query head a kv head, KL a power of two (qk 16 .. 256) and one
-    // pass per lane of a position: the KL partial dots meet through DPP in
-    // registers, no LDS and no barrier.  qk 48 (three lanes a position)
-    // sums them in LDS, and so do grouped heads (their REP dots a pass held
-    // across the passes took 6-55 more VGPRs than the LDS sums)
-    static constexpr bool kLaneSums =
-        REP == 1 && (KL & (KL - 1)) == 0 && KL <= 16 && KP == KL && KPP * KL == kThreads;
+    // KL a power of two (qk 16 .. 256) and one pass per lane of a position:
+    // the KL partial dots meet through DPP in registers, no LDS and no
+    // barrier.  qk 48 (three lanes a position) sums them in LDS
+    static constexpr bool kLaneSums = (KL & (KL - 1)) == 0 && KL <= 16 && KP == KL && KPP * KL == kThreads;
     static constexpr int VP = CH / VPP;                       // V passes per chunk
-};
-
-template <int VW>
-struct VVec;
-template <>
-struct VVec<16> {
-    typedef uint32_t T __attribute__((ext_vector_type(4)));
-};
-template <>
-struct VVec<8> {
-    typedef uint32_t T __attribute__((ext_vector_type(2)));
 };
 
 __device__ inline float i8_at(uint32_t dw, int b) { return float(int32_t(dw << (24 - 8 * b)) >> 24); }
 
-template <int REP, int QK, int VD, int VW>
+template <int QK, int VD>
 __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
     Geom g, const uint8_t *__restrict__ kv, size_t kv_stride, const int32_t *__restrict__ lo_a,
     const int32_t *__restrict__ hi_a, const float *__restrict__ q, float scale, int quant_query,
     int splits, float *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml)
 {
-    using S = AttnShape<REP, QK, VD, VW>;
+    using S = AttnShape<QK, VD>;
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    using VT = typename VVec<VW>::T;
     constexpr int CH = S::CH, NW = kThreads / 64;
-    __shared__ float qs[REP][QK];
-    __shared__ float sp[REP][CH * S::KL];  // lane partial dots
-    __shared__ float wsh[REP][CH];         // scores, then weights
-    __shared__ float red[REP][NW];
-    __shared__ float vred[NW][REP][VD];
+    __shared__ float qs[QK];
+    __shared__ float sp[CH * S::KL];  // lane partial dots
+    __shared__ float wsh[CH];         // scores, then weights
+    __shared__ float red[NW];
+    __shared__ float vred[NW][VD];
 
     const size_t qi = blockIdx.z;
     const int kvh = blockIdx.y;
@@ -212,8 +198,15 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
     const int span = hi - lo + 1;
     const bool bad = lo < 0 || span < 1 || span > g.cap;
     const int nch = bad ? 0 : (span + CH - 1) / CH;
-    const int c_begin = int((long long)nch * split / splits);
-    const int c_end = int((long long)nch * (split + 1) / splits);
+    // nch <= 2^16 chunks and splits <= 2^15: the products fit in 32 bits
+    const int c_begin = int(uint32_t(nch) * uint32_t(split) / uint32_t(splits));
+    const int c_end = int(uint32_t(nch) * uint32_t(split + 1) / uint32_t(splits));
+    // a span is no longer than the ring: positions wrap at most once
+    const int slo = bad ? 0 : lo % g.cap;
+    auto slot_of = [&](int pc) {
+        const int s = slo + pc;
+        return s >= g.cap ? s - g.cap : s;
+    };
 
     const uint8_t *blk = kv + qi * kv_stride;
     const int8_t *kb = reinterpret_cast<const int8_t *>(blk) + size_t(kvh) * g.cap * QK;
@@ -221,37 +214,34 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
     const float *ksb = reinterpret_cast<const float *>(blk + g.ks_off) + size_t(kvh) * g.cap;
     const float *vsb = reinterpret_cast<const float *>(blk + g.vs_off) + size_t(kvh) * g.cap;
 
-    // Query heads kvh*REP .. +REP (fake-quantised per head on request).
-    const float *qg = q + qi * size_t(g.H) * QK + size_t(kvh) * REP * QK;
-    for (int e = t; e < REP * QK; e += kThreads) qs[e / QK][e % QK] = qg[e];
+    // The query head (fake-quantised on request).
+    const float *qg = q + qi * size_t(g.H) * QK + size_t(kvh) * QK;
+    for (int e = t; e < QK; e += kThreads) qs[e] = qg[e];
     __syncthreads();
     if (quant_query) {
-        for (int r = wave; r < REP; r += NW) {
+        if (wave == 0) {
             float sc, inv;
-            quant_scale_wave(qs[r], QK, sc, inv);
-            for (int e = lane; e < QK; e += 64) qs[r][e] = quant_code(qs[r][e], inv) * sc;
+            quant_scale_wave(qs, QK, sc, inv);
+            for (int e = lane; e < QK; e += 64) qs[e] = quant_code(qs[e], inv) * sc;
         }
         __syncthreads();
     }
     const int ksub = t % S::KL;
     const int kpos = t / S::KL;  // position within a K pass
     const bool kact = t < S::KPP * S::KL;
-    float qr[REP][16];
+    float qr[16];
 #pragma unroll
-    for (int r = 0; r < REP; ++r)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) qr[r][e] = qs[r][ksub * 16 + e];
+    for (int e = 0; e < 16; ++e) qr[e] = qs[ksub * 16 + e];
     const int vsub = t % S::VL;
     const int vpos = t / S::VL;
 
-    u4 kr[S::KP];
-    VT vr[S::VP];
+    u4 kr[S::KP], vr[S::VP];
     auto load_k = [&](int c) {
 #pragma unroll
         for (int p = 0; p < S::KP; ++p) {
             const int pl = p * S::KPP + kpos;
             const int pc = min(c * CH + pl, span - 1);  // clamp: read a valid slot
-            const int slot = (lo + pc) % g.cap;
+            const int slot = slot_of(pc);
             kr[p] = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(kb + size_t(slot) * QK) + ksub);
         }
     };
@@ -259,8 +249,8 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 #pragma unroll
         for (int p = 0; p < S::VP; ++p) {
             const int pc = min(c * CH + p * S::VPP + vpos, span - 1);
-            const int slot = (lo + pc) % g.cap;
-            vr[p] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(vb + size_t(slot) * VD) + vsub);
+            const int slot = slot_of(pc);
+            vr[p] = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(vb + size_t(slot) * VD) + vsub);
         }
     };
     if (c_begin < c_end) {
@@ -268,160 +258,97 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
         load_v(c_begin);
     }
 
-    float m_run[REP], l_loc[REP], acc[REP][VW];
+    float m_run = -INFINITY, l_loc = 0.0f, acc[16];
 #pragma unroll
-    for (int r = 0; r < REP; ++r) {
-        m_run[r] = -INFINITY;
-        l_loc[r] = 0.0f;
-#pragma unroll
-        for (int e = 0; e < VW; ++e) acc[r][e] = 0.0f;
-    }
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
 
+    // a lane's partial dot of K pass p
+    auto dot16 = [&](int p) {
+        const uint32_t dw[4] = {kr[p].x, kr[p].y, kr[p].z, kr[p].w};
+        float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 16; e += 2) {
+            a0 += qr[e] * i8_at(dw[e >> 2], e & 3);
+            a1 += qr[e + 1] * i8_at(dw[e >> 2], (e & 3) + 1);
+        }
+        return a0 + a1;
+    };
     for (int c = c_begin; c < c_end; ++c) {
         const int n = min(CH, span - c * CH);
-        float cmax[REP];
-#pragma unroll
-        for (int r = 0; r < REP; ++r) cmax[r] = -INFINITY;
+        float cmax = -INFINITY;
         // the position this lane scores, its score and V scale (lane sums)
         const int own = ksub * S::KPP + kpos;
-        float own_sc[REP], own_vs = 0.0f;
+        float own_sc = 0.0f, own_vs = 0.0f;
         if constexpr (S::kLaneSums) {
             // ---- scores: lane partial dots summed across the position's KL
             // lanes by DPP; lane ksub keeps pass ksub's position, and its
             // K and V scales are requested before the dots ----
-            const int oslot = (lo + c * CH + min(own, n - 1)) % g.cap;
+            const int oslot = slot_of(c * CH + min(own, n - 1));
             const float ks = ksb[oslot];
             own_vs = vsb[oslot];
-            float dot[REP];
-#pragma unroll
-            for (int r = 0; r < REP; ++r) dot[r] = 0.0f;
+            float dot = 0.0f;
 #pragma unroll
             for (int p = 0; p < S::KP; ++p) {
-                const uint32_t dw[4] = {kr[p].x, kr[p].y, kr[p].z, kr[p].w};
-                float kf[16];
-#pragma unroll
-                for (int d = 0; d < 4; ++d)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) kf[4 * d + b] = i8_at(dw[d], b);
-#pragma unroll
-                for (int r = 0; r < REP; ++r) {
-                    float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 16; e += 2) {
-                        a0 += qr[r][e] * kf[e];
-                        a1 += qr[r][e + 1] * kf[e + 1];
-                    }
-                    const float v = ndl::group_sum<S::KL>(a0 + a1);
-                    dot[r] = ksub == p ? v : dot[r];
-                }
+                const float v = ndl::group_sum<S::KL>(dot16(p));
+                dot = ksub == p ? v : dot;
             }
             if (c + 1 < c_end) load_k(c + 1);  // lands during softmax and values
-#pragma unroll
-            for (int r = 0; r < REP; ++r) {
-                own_sc[r] = (dot[r] * ks) * scale;
-                if (own < n) cmax[r] = own_sc[r];
-            }
+            own_sc = (dot * ks) * scale;
+            if (own < n) cmax = own_sc;
         } else {
-        // ---- scores: lane partial dots ----
+            // ---- scores: lane partial dots, then per position ----
 #pragma unroll
-        for (int p = 0; p < S::KP; ++p) {
-            const int pl = p * S::KPP + kpos;
-            if (kact && pl < CH) {
-                const uint32_t dw[4] = {kr[p].x, kr[p].y, kr[p].z, kr[p].w};
-                float kf[16];
-#pragma unroll
-                for (int d = 0; d < 4; ++d)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) kf[4 * d + b] = i8_at(dw[d], b);
-#pragma unroll
-                for (int r = 0; r < REP; ++r) {
-                    float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 16; e += 2) {
-                        a0 += qr[r][e] * kf[e];
-                        a1 += qr[r][e + 1] * kf[e + 1];
-                    }
-                    sp[r][pl * S::KL + ksub] = a0 + a1;
-                }
+            for (int p = 0; p < S::KP; ++p) {
+                const int pl = p * S::KPP + kpos;
+                if (kact && pl < CH) sp[pl * S::KL + ksub] = dot16(p);
             }
-        }
-        if (c + 1 < c_end) load_k(c + 1);  // lands during softmax and values
-        __syncthreads();
-        // ---- per-position score, chunk max ----
-        for (int pl = t; pl < n; pl += kThreads) {
-            const int slot = (lo + c * CH + pl) % g.cap;
-            const float ks = ksb[slot];
-#pragma unroll
-            for (int r = 0; r < REP; ++r) {
+            if (c + 1 < c_end) load_k(c + 1);  // lands during softmax and values
+            __syncthreads();
+            for (int pl = t; pl < n; pl += kThreads) {
+                const int slot = slot_of(c * CH + pl);
                 float a = 0.0f;
 #pragma unroll
-                for (int s2 = 0; s2 < S::KL; ++s2) a += sp[r][pl * S::KL + s2];
-                const float sc = (a * ks) * scale;
-                wsh[r][pl] = sc;
-                cmax[r] = fmaxf(cmax[r], sc);
+                for (int s2 = 0; s2 < S::KL; ++s2) a += sp[pl * S::KL + s2];
+                const float sc = (a * ksb[slot]) * scale;
+                wsh[pl] = sc;
+                cmax = fmaxf(cmax, sc);
             }
         }
-        }
-#pragma unroll
-        for (int r = 0; r < REP; ++r) {
-            const float m = wave_max(cmax[r]);
-            if (lane == 0) red[r][wave] = m;
-        }
+        const float wm = wave_max(cmax);
+        if (lane == 0) red[wave] = wm;
         __syncthreads();
-        float alpha[REP], mnew[REP];
+        float mnew = m_run;
 #pragma unroll
-        for (int r = 0; r < REP; ++r) {
-            float m = m_run[r];
-#pragma unroll
-            for (int w2 = 0; w2 < NW; ++w2) m = fmaxf(m, red[r][w2]);
-            mnew[r] = m;
-            alpha[r] = expf(m_run[r] - m);  // exp(-inf) = 0 on the first chunk
-            m_run[r] = m;
-            l_loc[r] *= alpha[r];
-        }
+        for (int w2 = 0; w2 < NW; ++w2) mnew = fmaxf(mnew, red[w2]);
+        const float alpha = expf(m_run - mnew);  // exp(-inf) = 0 on the first chunk
+        m_run = mnew;
+        l_loc *= alpha;
         // ---- weights e * v_scale; running sum ----
         if constexpr (S::kLaneSums) {
             if (own < n) {
-#pragma unroll
-                for (int r = 0; r < REP; ++r) {
-                    const float e = expf(own_sc[r] - mnew[r]);
-                    l_loc[r] = l_loc[r] + e;
-                    wsh[r][own] = e * own_vs;
-                }
+                const float e = expf(own_sc - mnew);
+                l_loc = l_loc + e;
+                wsh[own] = e * own_vs;
             }
         } else {
             for (int pl = t; pl < n; pl += kThreads) {
-                const int slot = (lo + c * CH + pl) % g.cap;
-                const float vs = vsb[slot];
-#pragma unroll
-                for (int r = 0; r < REP; ++r) {
-                    const float e = expf(wsh[r][pl] - mnew[r]);
-                    l_loc[r] = l_loc[r] + e;
-                    wsh[r][pl] = e * vs;
-                }
+                const int slot = slot_of(c * CH + pl);
+                const float e = expf(wsh[pl] - mnew);
+                l_loc = l_loc + e;
+                wsh[pl] = e * vsb[slot];
             }
         }
         __syncthreads();
         // ---- values ----
 #pragma unroll
-        for (int r = 0; r < REP; ++r)
-#pragma unroll
-            for (int e = 0; e < VW; ++e) acc[r][e] *= alpha[r];
+        for (int e = 0; e < 16; ++e) acc[e] *= alpha;
 #pragma unroll
         for (int p = 0; p < S::VP; ++p) {
             const int pl = p * S::VPP + vpos;
             if (pl < n) {
-                float vf[VW];
+                const float wgt = wsh[pl];
 #pragma unroll
-                for (int d = 0; d < VW / 4; ++d)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) vf[4 * d + b] = i8_at(vr[p][d], b);
-#pragma unroll
-                for (int r = 0; r < REP; ++r) {
-                    const float wgt = wsh[r][pl];
-#pragma unroll
-                    for (int e = 0; e < VW; ++e) acc[r][e] += wgt * vf[e];
-                }
+                for (int e = 0; e < 16; ++e) acc[e] += wgt * i8_at(vr[p][e >> 2], e & 3);
             }
         }
         if (c + 1 < c_end) load_v(c + 1);  // lands during the next scores
@@ -430,108 +357,564 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 
     // ---- reduce over the lanes sharing a V column slice ----
 #pragma unroll
-    for (int r = 0; r < REP; ++r)
-#pragma unroll
-        for (int e = 0; e < VW; ++e)
-            acc[r][e] = ndl::wave_sum_from<S::VL>(acc[r][e]);
+    for (int e = 0; e < 16; ++e) acc[e] = ndl::wave_sum_from<S::VL>(acc[e]);
     if (lane < S::VL) {
 #pragma unroll
-        for (int r = 0; r < REP; ++r)
-#pragma unroll
-            for (int e = 0; e < VW; ++e) vred[wave][r][lane * VW + e] = acc[r][e];
+        for (int e = 0; e < 16; ++e) vred[wave][lane * 16 + e] = acc[e];
     }
-#pragma unroll
-    for (int r = 0; r < REP; ++r) {
-        const float l = wave_sum(l_loc[r]);
-        if (lane == 0) red[r][wave] = l;
-    }
+    const float wl = wave_sum(l_loc);
+    if (lane == 0) red[wave] = wl;
     __syncthreads();
-    for (int o = t; o < REP * VD; o += kThreads) {
-        const int r = o / VD, col = o % VD;
+    for (int col = t; col < VD; col += kThreads) {
         float s = 0.0f, l = 0.0f;
 #pragma unroll
         for (int w2 = 0; w2 < NW; ++w2) {
-            s += vred[w2][r][col];
-            l += red[r][w2];
+            s += vred[w2][col];
+            l += red[w2];
         }
-        const int head = kvh * REP + r;
         if (splits == 1) {
-            out[qi * size_t(g.H) * VD + size_t(head) * VD + col] = bad ? NAN : s / l;
+            out[qi * size_t(g.H) * VD + size_t(kvh) * VD + col] = bad ? NAN : s / l;
         } else {
-            part_o[((qi * g.H + head) * size_t(splits) + split) * VD + col] = s;
+            part_o[((qi * g.H + kvh) * size_t(splits) + split) * VD + col] = s;
             if (col == 0) {
-                float *ml = part_ml + ((qi * g.H + head) * size_t(splits) + split) * 2;
-                ml[0] = bad ? NAN : (c_begin < c_end ? m_run[r] : -INFINITY);
+                float *ml = part_ml + ((qi * g.H + kvh) * size_t(splits) + split) * 2;
+                ml[0] = bad ? NAN : (c_begin < c_end ? m_run : -INFINITY);
                 ml[1] = l;
             }
         }
     }
 }
 
-// Merge chunk partials: out = sum_c o_c e^(m_c - M) / sum_c l_c e^(m_c - M).
-__global__ __launch_bounds__(kThreads) void attn_combine_kernel(Geom g, int nchunks,
+// ---------------------------------------------------------------------------
+// Attention over the int8 cache on the matrix cores: grouped query heads
+// (several queries per K/V row) and prompts (all rows over one block).
+//
+// A wave owns 16 NT query columns -- (row, head) pairs that share a kv head
+// -- and walks chunks of 32 positions with its own online softmax; no barrier
+// until the waves of a block, which take the chunks in turn, merge at the end.
+//   scores  S[pos][col] = K Q^T: v_mfma 16x16, A = 16 positions' int8 rows, as
+//           they lie in the cache, B = the wave's query columns.  With
+//           quant_query the query is int8 codes times one scale a head, so
+//           the dot is an exact integer (i32_16x16x64_i8, no conversion of
+//           K at all); else the fp32 query is three bf16 pieces whose sum is
+//           exactly the query and K's codes are exact in bf16.
+//   values  O^T[v][col] = V^T P^T: a score tile's result layout (lane = column,
+//           four positions a lane) is the B layout the product needs, so the
+//           weights stay in their lanes, as three bf16 pieces whose sum is
+//           exactly the fp32 weight; V's codes are exact in bf16.  MFMA c
+//           takes V columns 4 n + c, so a lane's V bytes come as one dword a
+//           position and no byte is moved between lanes.
+// Every product is exact and the sums are fp32 (or int32): nothing is held in
+// 16 bits.  What bounds it is the VALU work of the softmax (about 22
+// operations a score) and V's conversion (1.5 a byte, shared by the wave's
+// columns); the matrix cores need about a third of the time.
+// Measured, MI355X, against the per-position kernel that took these calls
+// before (K and V converted to fp32 and multiplied in the VALU for each query
+// head; a prompt's rows each walked their own span):
+//   prompt, 12 on 2 heads, qk 48, quant_query: 1000 rows 78 -> 12.7 us, 2000
+//   234 -> 29, 3000 470 -> 53 (12 x 64 MHA: 123 / 384 / 788 -> 13 / 29 / 50)
+//   decode, 12 on 2 heads: 64 sessions x 2048 29.6 -> 11.0 us, 256 x 1024
+//   41.4 -> 12.6, one session x 8192 24.7 -> 10.2; 8 on 4: 64 x 2048 26 -> 14;
+//   16 on 2: 256 x 1024 82 -> 13.8
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef int intx4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+// High halves of two floats: (bf16 of a, bf16 of b) where both are exact.
+__device__ inline uint32_t pack_hi(float a, float b)
+{
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+
+__device__ inline float trunc_hi(float a) { return __uint_as_float(__float_as_uint(a) & 0xffff0000u); }
+
+// fmaxf of three (a NaN loses), without the copies the compiler makes of
+// operands it cannot show to be quiet.
+__device__ inline float max3(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// x0, x1 as three bf16 pairs that sum to them exactly (8 mantissa bits each).
+__device__ inline void split3(float x0, float x1, uint32_t &h, uint32_t &m, uint32_t &l)
+{
+    h = pack_hi(x0, x1);
+    const float r0 = x0 - trunc_hi(x0), r1 = x1 - trunc_hi(x1);
+    m = pack_hi(r0, r1);
+    l = pack_hi(r0 - trunc_hi(r0), r1 - trunc_hi(r1));
+}
+
+template <int QK, bool QQ, int NT, int NW, bool SHARED>
+__global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
+    Geom g, const uint8_t *__restrict__ kv, size_t kv_stride, const int32_t *__restrict__ lo_a,
+    const int32_t *__restrict__ hi_a, const float *__restrict__ q, float scale2, int rows, int splits,
+    float *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml)
+{
+    constexpr int VD = 64, SL = QK / 4;             // a lane's slice of a K row
+    constexpr int KD = SL / 4;                      // its dwords (3 or 4)
+    constexpr int COLS = SHARED ? 16 * NT : kMaxRep;  // merged columns
+    constexpr int LD = VD + 4;
+    static_assert(SHARED || NT == 1, "one query: at most kMaxRep columns");
+    __shared__ __align__(16) float sc_s[NW][64];
+    __shared__ __align__(16) float mo[NW][COLS][LD];
+    __shared__ float mm[NW][COLS], ml[NW][COLS], mf[NW][COLS];
+
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int n = lane & 15, qd = lane >> 4;
+    const int R = g.H / g.KVH;
+    const int kvh = blockIdx.x % g.KVH, split = blockIdx.x / g.KVH;
+    // later tiles of a prompt have the longer spans: they start first
+    const int tile = SHARED ? int(gridDim.y) - 1 - int(blockIdx.y) : int(blockIdx.y);
+    const uint8_t *blk = SHARED ? kv : kv + size_t(tile) * kv_stride;
+    const int8_t *kb = reinterpret_cast<const int8_t *>(blk) + size_t(kvh) * g.cap * QK;
+    const int8_t *vb = reinterpret_cast<const int8_t *>(blk + g.v_off) + size_t(kvh) * g.cap * VD;
+    const float *ksb = reinterpret_cast<const float *>(blk + g.ks_off) + size_t(kvh) * g.cap;
+    const float *vsb = reinterpret_cast<const float *>(blk + g.vs_off) + size_t(kvh) * g.cap;
+    const uint32_t cap = uint32_t(g.cap);
+
+    // ---- the wave's columns: their spans and query operands ----
+    const int ncols = SHARED ? rows * R : R;  // columns of this kv head (and query)
+    // f / R of a column f < 2^20: (f + 1/2) / R is 1/16 or more away from an
+    // integer (R <= 8), and its float error is below 2^20 2^-22 / R
+    const float inv_r = 1.0f / float(R);
+    auto row_of = [&](int f) { return SHARED ? int((float(f) + 0.5f) * inv_r) : tile; };
+    uint32_t lo[NT], hi[NT];
+    bool bad[NT];
+    float cf[NT];                              // column factor of a score, in bits
+    intx4_t qi[NT];                            // QQ: codes
+    uint32_t qp[NT][3][KD == 3 ? 6 : 8];       // else: bf16 pieces
+    uint32_t ulo = 0xffffffffu, uhi = 0;
+    float spans = 0.0f;
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+        const int f0 = (SHARED ? tile * (16 * NT) + 16 * x : 0) + n;
+        const int f = f0 < ncols ? f0 : ncols - 1;  // past the end: a copy, not written
+        const int row = row_of(f);
+        const int head = kvh * R + (SHARED ? f - row * R : f);
+        const int l0 = lo_a[row], h0 = hi_a[row];
+        // h0 - l0 cannot overflow where l0 >= 0 and h0 >= l0
+        bad[x] = l0 < 0 || h0 < l0 || h0 - l0 >= g.cap;
+        lo[x] = bad[x] ? 0xffffffffu : uint32_t(l0);
+        hi[x] = bad[x] ? 0u : uint32_t(h0);
+        if (!bad[x]) {
+            ulo = min(ulo, lo[x]);
+            uhi = max(uhi, hi[x]);
+            spans += float(h0 - l0 + 1);
+        }
+        const float *qh = q + (size_t(row) * g.H + head) * QK + qd * SL;
+        float v[SL];
+#pragma unroll
+        for (int e = 0; e < SL; ++e) v[e] = qh[e];
+        if constexpr (QQ) {
+            // quant_rows (model.rs:289-293): the codes and the head's scale
+            float a = 0.0f;
+#pragma unroll
+            for (int e = 0; e < SL; e += 2) a = max3(a, __builtin_fabsf(v[e]), __builtin_fabsf(v[e + 1]));
+            a = fmaxf(a, ndl::wave_xor<16>(a));
+            a = fmaxf(a, ndl::wave_xor<32>(a));
+            const float qs = a > 0.0f ? a / 127.0f : 1.0f;
+            const float inv = 1.0f / qs;
+            float nan = 0.0f;  // NaN where a code is
+            uint32_t dw[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < SL; ++e) {
+                // quant_code: half away from zero is truncation after adding
+                // the float below a half, for every |y| < 2^22
+                const float y = v[e] * inv;
+                const float r = __builtin_amdgcn_fmed3f(y + copysignf(0.49999997f, y), -128.0f, 127.5f);
+                nan += y * 0.0f;
+                dw[e >> 2] |= (uint32_t(int32_t(r)) & 0xffu) << (8 * (e & 3));
+            }
+            nan += ndl::wave_xor<16>(nan);
+            nan += ndl::wave_xor<32>(nan);
+            qi[x] = intx4_t{int(dw[0]), int(dw[1]), int(dw[2]), int(dw[3])};
+            cf[x] = qs * scale2 + nan;
+        } else {
+#pragma unroll
+            for (int e = 0; e < SL; e += 2) split3(v[e], v[e + 1], qp[x][0][e / 2], qp[x][1][e / 2], qp[x][2][e / 2]);
+            cf[x] = scale2;
+        }
+    }
+    // the union of the columns' spans (the same in all four lane quarters)
+    {
+        auto umin = [&](uint32_t &a, uint32_t b) { a = min(a, b); };
+        auto umax = [&](uint32_t &a, uint32_t b) { a = max(a, b); };
+        umin(ulo, uint32_t(ndl::wave_xor_int<1>(int(ulo)))), umax(uhi, uint32_t(ndl::wave_xor_int<1>(int(uhi))));
+        umin(ulo, uint32_t(ndl::wave_xor_int<2>(int(ulo)))), umax(uhi, uint32_t(ndl::wave_xor_int<2>(int(uhi))));
+        umin(ulo, uint32_t(ndl::wave_xor_int<4>(int(ulo)))), umax(uhi, uint32_t(ndl::wave_xor_int<4>(int(uhi))));
+        umin(ulo, uint32_t(ndl::wave_xor_int<8>(int(ulo)))), umax(uhi, uint32_t(ndl::wave_xor_int<8>(int(uhi))));
+        spans = ndl::group_sum<16>(spans);
+        ulo = __builtin_amdgcn_readfirstlane(ulo);
+        uhi = __builtin_amdgcn_readfirstlane(uhi);
+        spans = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(spans)));
+    }
+    const bool any = uhi >= ulo;
+    // Rows of a prompt overlap, and the wave walks the union of their spans.
+    // Rows that share little (a caller's own lo and hi) would make the union
+    // longer than the rows together: then each chunk starts where some row
+    // still has a position, so no more chunks are walked than the rows have.
+    const bool sparse = SHARED && any && float(uhi - ulo) + 1.0f > spans / float(R) + 64.0f;
+    const uint32_t step = uint32_t(splits) * NW;  // waves that share the walk
+    uint32_t p0 = ulo, s0 = 0;
+    bool more = any;
+    const uint32_t step_mod = (32u * step) % cap;
+    auto next_start = [&](uint32_t from) {  // first position >= from of any column
+        uint32_t c = 0xffffffffu;
+#pragma unroll
+        for (int x = 0; x < NT; ++x)
+            if (!bad[x] && hi[x] >= from) c = min(c, max(lo[x], from));
+        c = min(c, uint32_t(ndl::wave_xor_int<1>(int(c))));
+        c = min(c, uint32_t(ndl::wave_xor_int<2>(int(c))));
+        c = min(c, uint32_t(ndl::wave_xor_int<4>(int(c))));
+        c = min(c, uint32_t(ndl::wave_xor_int<8>(int(c))));
+        return uint32_t(__builtin_amdgcn_readfirstlane(c));
+    };
+    auto advance = [&](uint32_t k, uint32_t mod) {  // k chunks on
+        if (!sparse) {
+            // p0 - ulo < 2^31 and 32 k < 2^31: no wrap
+            p0 += 32u * k;
+            s0 += mod;
+            if (s0 >= cap) s0 -= cap;
+            more = p0 <= uhi && p0 >= ulo;
+        } else {
+            for (uint32_t i = 0; i < k && more; ++i) {
+                p0 = next_start(p0 + 32u);  // positions end below 2^31
+                more = p0 != 0xffffffffu;
+            }
+            if (more) s0 = p0 % cap;
+        }
+    };
+    if (any) {
+        s0 = ulo % cap;
+        const uint32_t first = uint32_t(split) * NW + uint32_t(w);
+        if (first) advance(first, (32u * first) % cap);
+    }
+
+    uint32_t kr[2][KD], vr[8];
+    float scr = 0.0f;
+    // a chunk inside the ring: scalar base, lane and pass offsets; across its
+    // end (or in a ring below a chunk): each position's slot
+    auto slot_of = [&](uint32_t off) { return (s0 + off) % cap; };
+    auto load_k = [&]() {
+        if (s0 + 32u <= cap) {
+            const int8_t *p = kb + size_t(s0) * QK;
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int d = 0; d < KD; ++d)
+                    kr[a][d] = *reinterpret_cast<const uint32_t *>(p + (n * QK + qd * SL) + (16 * a * QK + 4 * d));
+            scr = *(lane < 32 ? ksb + s0 + lane : vsb + s0 + (lane - 32));
+        } else {
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const int8_t *p = kb + size_t(slot_of(16 * a + n)) * QK + qd * SL;
+#pragma unroll
+                for (int d = 0; d < KD; ++d) kr[a][d] = *reinterpret_cast<const uint32_t *>(p + 4 * d);
+            }
+            scr = (lane < 32 ? ksb : vsb)[slot_of(lane & 31)];
+        }
+    };
+    auto load_v = [&]() {
+        if (s0 + 32u <= cap) {
+            const int8_t *p = vb + size_t(s0) * VD;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                vr[j] = *reinterpret_cast<const uint32_t *>(p + (4 * qd * VD + 4 * n) + (16 * (j >> 2) + (j & 3)) * VD);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                vr[j] = *reinterpret_cast<const uint32_t *>(
+                    vb + size_t(slot_of(16 * (j >> 2) + 4 * qd + (j & 3))) * VD + 4 * n);
+        }
+    };
+    // loads are never conditional: past the last chunk they reread a slot
+    load_k();
+    load_v();
+
+    float m_run[NT], l_run[NT];
+    floatx4_t acc[NT][4];
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+        m_run[x] = -INFINITY;
+        l_run[x] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[x][c] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    while (more) {
+        const uint32_t pc = p0;
+        // the chunk's scales, from position order to the score tiles' rows
+        sc_s[w][lane] = scr;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        floatx4_t ks[2], vs[2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            ks[a] = *reinterpret_cast<const floatx4_t *>(&sc_s[w][16 * a + 4 * qd]);
+            vs[a] = *reinterpret_cast<const floatx4_t *>(&sc_s[w][32 + 16 * a + 4 * qd]);
+        }
+        __builtin_amdgcn_wave_barrier();
+        // ---- scores ----
+        float s[NT][8];
+        if constexpr (QQ) {
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const intx4_t kf{int(kr[a][0]), int(kr[a][1]), int(kr[a][2]), KD == 3 ? 0 : int(kr[a][KD - 1])};
+#pragma unroll
+                for (int x = 0; x < NT; ++x) {
+                    const intx4_t d = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qi[x], intx4_t{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s[x][4 * a + i] = (float(d[i]) * ks[a][i]) * cf[x];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                uint32_t kp[2 * KD];
+#pragma unroll
+                for (int d = 0; d < KD; ++d) {
+                    kp[2 * d] = pack_hi(i8_at(kr[a][d], 0), i8_at(kr[a][d], 1));
+                    kp[2 * d + 1] = pack_hi(i8_at(kr[a][d], 2), i8_at(kr[a][d], 3));
+                }
+                const bf16x8_t k0 = __builtin_bit_cast(bf16x8_t, u32x4_t{kp[0], kp[1], kp[2], kp[3]});
+#pragma unroll
+                for (int x = 0; x < NT; ++x) {
+                    floatx4_t d{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int pc3 = 2; pc3 >= 0; --pc3) {  // the small pieces first
+                        const uint32_t *qq = qp[x][pc3];
+                        // qk 48: a lane's last four codes, doubled to the 32-wide
+                        // product's eight against four zeros of the query
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8_t, u32x4_t{kp[4], kp[5], kp[2 * KD - 2], kp[2 * KD - 1]}),
+                            __builtin_bit_cast(bf16x8_t, KD == 3 ? u32x4_t{qq[4], qq[5], 0u, 0u}
+                                                                 : u32x4_t{qq[4], qq[5], qq[2 * KD - 2], qq[2 * KD - 1]}),
+                            d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            k0, __builtin_bit_cast(bf16x8_t, u32x4_t{qq[0], qq[1], qq[2], qq[3]}), d, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s[x][4 * a + i] = (d[i] * ks[a][i]) * cf[x];
+                }
+            }
+        }
+        advance(step, step_mod);
+        load_k();  // lands during the softmax and the values
+        // ---- softmax: each lane its column's eight positions ----
+        bool inside = true;
+#pragma unroll
+        for (int x = 0; x < NT; ++x) inside = inside && !bad[x] && lo[x] <= pc && hi[x] >= pc + 31u;
+        const bool full = __all(inside);
+        if (!full) {
+#pragma unroll
+            for (int x = 0; x < NT; ++x)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t p = pc + uint32_t(16 * (j >> 2) + 4 * qd + (j & 3));
+                    if (p < lo[x] || p > hi[x]) s[x][j] = -INFINITY;
+                }
+        }
+        bool grew = false;
+        float m_new[NT];
+#pragma unroll
+        for (int x = 0; x < NT; ++x) {
+            const float m8 = max3(max3(s[x][0], s[x][1], s[x][2]), max3(s[x][3], s[x][4], s[x][5]),
+                                  max3(s[x][6], s[x][7], m_run[x]));
+            // over the four lane quarters: each swap returns the pair
+            const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(m8), __float_as_uint(m8), false, false);
+            const float m16 = max3(__uint_as_float(s16[0]), __uint_as_float(s16[1]), m8);
+            const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m16), __float_as_uint(m16), false, false);
+            m_new[x] = max3(__uint_as_float(s32[0]), __uint_as_float(s32[1]), m16);
+            grew = grew || m_new[x] > m_run[x];
+        }
+        if (__any(grew)) {
+#pragma unroll
+            for (int x = 0; x < NT; ++x) {
+                const float al = m_new[x] > m_run[x] ? __builtin_amdgcn_exp2f(m_run[x] - m_new[x]) : 1.0f;
+                m_run[x] = m_new[x];
+                l_run[x] *= al;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[x][c] *= al;
+            }
+        }
+        uint32_t pp[NT][3][4];
+#pragma unroll
+        for (int x = 0; x < NT; ++x) {
+            const float mu = m_run[x] == -INFINITY ? 0.0f : m_run[x];
+            float wt[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float e = __builtin_amdgcn_exp2f(s[x][j] - mu);
+                l_run[x] += e;
+                wt[j] = e * vs[j >> 2][j & 3];
+            }
+            if (!full) {
+                // a slot no row reads may hold anything, a NaN scale too
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t p = pc + uint32_t(16 * (j >> 2) + 4 * qd + (j & 3));
+                    if (p < lo[x] || p > hi[x]) wt[j] = 0.0f;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j += 2)
+                split3(wt[j], wt[j + 1], pp[x][0][j / 2], pp[x][1][j / 2], pp[x][2][j / 2]);
+        }
+        // ---- values ----
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            uint32_t vp[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) vp[j] = pack_hi(i8_at(vr[2 * j], c), i8_at(vr[2 * j + 1], c));
+            const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, u32x4_t{vp[0], vp[1], vp[2], vp[3]});
+#pragma unroll
+            for (int x = 0; x < NT; ++x)
+#pragma unroll
+                for (int pc3 = 2; pc3 >= 0; --pc3)
+                    acc[x][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        vf, __builtin_bit_cast(bf16x8_t, u32x4_t{pp[x][pc3][0], pp[x][pc3][1], pp[x][pc3][2], pp[x][pc3][3]}),
+                        acc[x][c], 0, 0, 0);
+        }
+        load_v();  // lands during the next scores
+    }
+
+    // ---- merge the block's waves ----
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+        float l = l_run[x];
+        l += ndl::wave_xor<16>(l);
+        l += ndl::wave_xor<32>(l);
+        const int col = 16 * x + n;
+        if (col < COLS) {
+            if (qd == 0) {
+                mm[w][col] = bad[x] ? NAN : m_run[x];
+                ml[w][col] = l;
+            }
+            // lane (n, qd) holds V columns 16 qd + 4 i + c
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *reinterpret_cast<floatx4_t *>(&mo[w][col][16 * qd + 4 * i]) =
+                    floatx4_t{acc[x][0][i], acc[x][1][i], acc[x][2][i], acc[x][3][i]};
+        }
+    }
+    __syncthreads();
+    for (int o = t; o < NW * COLS; o += NW * 64) {
+        const int i = o / COLS, col = o % COLS;
+        float M = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < NW; ++j) M = fmaxf(M, mm[j][col]);
+        const float m = mm[i][col];
+        // -inf: the wave's sums are 0, or NaN where a score was; NaN: a bad span
+        mf[i][col] = m == -INFINITY ? 1.0f : exp2f(m - M);
+    }
+    __syncthreads();
+    for (int col = w; col < COLS; col += NW) {  // a wave a column, a lane a value
+        const int f = (SHARED ? tile * (16 * NT) : 0) + col;
+        if (f >= ncols) break;
+        const int row = __builtin_amdgcn_readfirstlane(row_of(f));
+        const int head = kvh * R + (SHARED ? f - row * R : f);
+        float O = 0.0f, L = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            O += mo[i][col][lane] * mf[i][col];
+            L += ml[i][col] * mf[i][col];
+        }
+        const size_t oh = size_t(row) * g.H + head;
+        if (splits == 1) {
+            out[oh * VD + lane] = O / L;
+        } else {
+            part_o[(oh * splits + split) * VD + lane] = O;
+            if (lane == 0) {
+                float M = -INFINITY;
+                for (int i = 0; i < NW; ++i) M = fmaxf(M, mm[i][col]);
+                float *p = part_ml + (oh * splits + split) * 2;
+                p[0] = L != L ? NAN : M;
+                p[1] = L;
+            }
+        }
+    }
+}
+
+// Merge chunk partials: out = sum_c o_c e^(m_c - M) / sum_c l_c e^(m_c - M);
+// with BASE2, powers of two (the matrix-core kernel's maxima are in bits).
+template <bool BASE2>
+__global__ __launch_bounds__(64) void attn_combine_kernel(Geom g, int nchunks,
                                                                const float *__restrict__ part_o,
                                                                const float *__restrict__ part_ml,
                                                                float *__restrict__ out)
 {
+    // the partials' factors, 64 at a time in the lanes, then one column a lane
     const size_t qi = blockIdx.y;
-    const int head = blockIdx.x;
+    const int head = blockIdx.x, lane = threadIdx.x;
     const size_t base = (qi * g.H + head) * size_t(nchunks);
+    __shared__ float fs[64], ls[64];
     float M = -INFINITY;
-    for (int c = 0; c < nchunks; ++c) M = fmaxf(M, part_ml[(base + c) * 2]);
-    for (int col = threadIdx.x; col < g.VD; col += blockDim.x) {
+    for (int c = lane; c < nchunks; c += 64) M = fmaxf(M, part_ml[(base + c) * 2]);
+    M = wave_max(M);
+    for (int col = lane; col < g.VD; col += 64) {
         float O = 0.0f, L = 0.0f;
-        for (int c = 0; c < nchunks; ++c) {
-            const float m = part_ml[(base + c) * 2];
-            if (m == -INFINITY) continue;
-            const float f = expf(m - M);
-            O += part_o[(base + c) * g.VD + col] * f;
-            L += part_ml[(base + c) * 2 + 1] * f;
+        for (int c0 = 0; c0 < nchunks; c0 += 64) {
+            const int nc = min(64, nchunks - c0);
+            __syncthreads();
+            if (lane < nc) {
+                const float m = part_ml[(base + c0 + lane) * 2];
+                fs[lane] = m == -INFINITY ? 0.0f : (BASE2 ? exp2f(m - M) : expf(m - M));
+                ls[lane] = m == -INFINITY ? 0.0f : part_ml[(base + c0 + lane) * 2 + 1];
+            }
+            __syncthreads();
+#pragma unroll 4
+            for (int c = 0; c < nc; ++c) {
+                O += part_o[(base + c0 + c) * g.VD + col] * fs[c];
+                L += ls[c] * fs[c];
+            }
         }
         out[qi * size_t(g.H) * g.VD + size_t(head) * g.VD + col] = O / L;
     }
 }
 
+using AttnFn = void (*)(dim3, hipStream_t, Geom, const uint8_t *, size_t, const int32_t *,
+                        const int32_t *, const float *, float, int, int, int, float *, float *, float *);
 
-
-template <int REP, int QK>
+template <int QK>
 void launch_attn(dim3 grid, hipStream_t s, Geom g, const uint8_t *kv, size_t stride,
                  const int32_t *lo, const int32_t *hi, const float *q, float scale, int qq,
-                 int splits, float *out, float *po, float *pml)
+                 int, int splits, float *out, float *po, float *pml)
 {
-    constexpr int VW = REP <= 2 ? 16 : 8;
-    hipLaunchKernelGGL((attn_i8_kernel<REP, QK, 64, VW>), grid, dim3(kThreads), 0, s, g, kv, stride,
-                       lo, hi, q, scale, qq, splits, out, po, pml);
+    hipLaunchKernelGGL((attn_i8_kernel<QK, 64>), grid, dim3(kThreads), 0, s, g, kv, stride, lo, hi, q,
+                       scale, qq, splits, out, po, pml);
 }
 
-using AttnFn = void (*)(dim3, hipStream_t, Geom, const uint8_t *, size_t, const int32_t *,
-                        const int32_t *, const float *, float, int, int, float *, float *, float *);
+template <int QK, int NT, int NW, bool SHARED>
+void launch_mm(dim3 grid, hipStream_t s, Geom g, const uint8_t *kv, size_t stride, const int32_t *lo,
+               const int32_t *hi, const float *q, float scale, int qq, int rows, int splits, float *out,
+               float *po, float *pml)
+{
+    const float scale2 = float(double(scale) * 1.4426950408889634);  // scores in bits: e^s = 2^(s log2 e)
+    if (qq)
+        hipLaunchKernelGGL((attn_mm_kernel<QK, true, NT, NW, SHARED>), grid, dim3(NW * 64), 0, s, g, kv,
+                           stride, lo, hi, q, scale2, rows, splits, out, po, pml);
+    else
+        hipLaunchKernelGGL((attn_mm_kernel<QK, false, NT, NW, SHARED>), grid, dim3(NW * 64), 0, s, g, kv,
+                           stride, lo, hi, q, scale2, rows, splits, out, po, pml);
+}
 
 // Instantiated: qk 48 (the shipped v3 geometry) and 64 (the MHA cache), v 64,
 // query heads per kv head 1, 2, 3, 4, 6, 8.
-template <int REP>
-AttnFn pick_qk(int qk, int vd)
+bool attn_shape(int rep, int qk, int vd)
 {
-    if (vd != 64) return nullptr;
-    switch (qk) {
-    case 48: return launch_attn<REP, 48>;
-    case 64: return launch_attn<REP, 64>;
-    default: return nullptr;
-    }
+    const bool r = rep == 1 || rep == 2 || rep == 3 || rep == 4 || rep == 6 || rep == 8;
+    return r && (qk == 48 || qk == 64) && vd == 64;
 }
 
-AttnFn pick_attn(int rep, int qk, int vd)
-{
-    switch (rep) {
-    case 1: return pick_qk<1>(qk, vd);
-    case 2: return pick_qk<2>(qk, vd);
-    case 3: return pick_qk<3>(qk, vd);
-    case 4: return pick_qk<4>(qk, vd);
-    case 6: return pick_qk<6>(qk, vd);
-    case 8: return pick_qk<8>(qk, vd);
-    default: return nullptr;
-    }
-}
+// The matrix-core kernel takes every prompt, and every decode call with two
+// or more query heads a kv head (figures at the kernel).  One query head a kv
+// head stays with attn_i8_kernel: its column tile would be 1/16 full, and
+// where the caches stream from HBM it is the faster of the two (12 x 64, 256
+// sessions x 1024: 70 against 77-85 us; 64 x 512: 11.5 against 11.6-13.1).
+constexpr int kMmMinRep = 2;
 
 }  // namespace
 
@@ -640,13 +1023,13 @@ int attend_i8(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride
     ND_REQUIRE((reinterpret_cast<uintptr_t>(kv) & 255) == 0 && kv_stride % 256 == 0,
                "kv blocks must be 256-byte aligned");
     const int rep = g->num_heads / g->num_kv_heads;
-    AttnFn fn = pick_attn(rep, g->qk_head_dim, g->v_head_dim);
-    ND_REQUIRE(fn, "no attention kernel for repeat %d, qk %d, v %d", rep, g->qk_head_dim,
-               g->v_head_dim);
+    ND_REQUIRE(attn_shape(rep, g->qk_head_dim, g->v_head_dim),
+               "no attention kernel for repeat %d, qk %d, v %d", rep, g->qk_head_dim, g->v_head_dim);
     // Split each span across blocks only when (query, kv head) pairs cannot
     // give every CU a few blocks; the split partials merge in a second pass.
     const size_t pairs = count * size_t(g->num_kv_heads);
-    const size_t want = size_t(ctx->num_cus > 0 ? ctx->num_cus : 256) * 4;
+    const size_t cus = size_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
+    const size_t want = cus * 4;
     // a split covers at least 512 positions (256 with more than two query
     // heads a kv head): with one query head, splits of one 256-position
     // chunk measured slower at one session (ctx 512: 13.1 against 10.6 us,
@@ -656,16 +1039,60 @@ int attend_i8(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride
     size_t splits = pairs >= want ? 1 : (want + pairs - 1) / pairs;
     if (splits > max_splits) splits = max_splits;
     if (splits > 65535) splits = 65535;
+    if (fixed && splits > 1) {
+        const size_t need = count * size_t(g->num_heads) * splits * (g->v_head_dim + 2);
+        ND_REQUIRE(need <= fixed_floats,
+                   "split-K partials need %zu floats (%zu queries x %d heads x %zu splits x "
+                   "(%d + 2)); the no-allocation scratch holds %zu",
+                   need, count, g->num_heads, splits, g->v_head_dim, fixed_floats);
+    }
+    const bool q48 = g->qk_head_dim == 48;
+    bool base2 = true;
+    AttnFn fn;
+    dim3 grid;
+    if (kv_stride == 0 && count > 1) {
+        // A prompt's rows over one block.  Two column tiles a wave share V's
+        // conversion once that leaves four blocks a CU (3000 rows, 12 on 2:
+        // 53 against 57 us; 2000: 31 against 29); with fewer than two
+        // single-tile blocks a CU, eight waves a block (500 rows: 9.3 against
+        // 14.3 us with four; 1000: 14.7 against 12.8)
+        const size_t cols = count * size_t(rep);
+        const size_t kvh = size_t(g->num_kv_heads);
+        const bool wide = (cols + 31) / 32 * kvh >= 4 * cus;
+        const size_t tiles = wide ? (cols + 31) / 32 : (cols + 15) / 16;
+        const size_t nw = !wide && tiles * kvh < 2 * cus ? 8 : 4;
+        const size_t fill = (cus * 8 + tiles * g->num_kv_heads * nw - 1) / (tiles * g->num_kv_heads * nw);
+        if (splits > fill) splits = fill;
+        grid = dim3(unsigned(g->num_kv_heads * splits), unsigned(tiles));
+        fn = wide      ? (q48 ? launch_mm<48, 2, 4, true> : launch_mm<64, 2, 4, true>)
+             : nw == 4 ? (q48 ? launch_mm<48, 1, 4, true> : launch_mm<64, 1, 4, true>)
+                       : (q48 ? launch_mm<48, 1, 8, true> : launch_mm<64, 1, 8, true>);
+    } else if (rep >= kMmMinRep) {
+        // Two waves a SIMD or more, from one block where it can be: 16-wave
+        // blocks below 8 waves a CU (64 sessions x 2 heads x 512: 7.4 against
+        // 9.7 us with four waves and a merge launch), 4-wave blocks above
+        // (256 x 2 x 1024: 15.3 against 17.3); no split leaves a wave without
+        // a chunk
+        const bool deep = pairs * 4 < cus * 8;
+        const size_t nw = deep ? 16 : 4;
+        const size_t fill = (cus * 8 + pairs * nw - 1) / (pairs * nw);
+        const size_t most = (size_t(g->cap) + 32 * nw - 1) / (32 * nw);
+        if (splits > fill) splits = fill;
+        if (splits > most) splits = most;
+        grid = dim3(unsigned(g->num_kv_heads * splits), unsigned(count));
+        fn = deep ? (q48 ? launch_mm<48, 1, 16, false> : launch_mm<64, 1, 16, false>)
+                  : (q48 ? launch_mm<48, 1, 4, false> : launch_mm<64, 1, 4, false>);
+    } else {
+        grid = dim3(unsigned(splits), unsigned(g->num_kv_heads), unsigned(count));
+        base2 = false;
+        fn = q48 ? launch_attn<48> : launch_attn<64>;
+    }
     float *po = nullptr, *pml = nullptr;
     if (splits > 1) {
         void *wsp = nullptr;
         const size_t n_o = count * size_t(g->num_heads) * splits * g->v_head_dim;
         const size_t n_ml = count * size_t(g->num_heads) * splits * 2;
         if (fixed) {
-            ND_REQUIRE(n_o + n_ml <= fixed_floats,
-                       "split-K partials need %zu floats (%zu queries x %d heads x %zu splits x "
-                       "(%d + 2)); the no-allocation scratch holds %zu",
-                       n_o + n_ml, count, g->num_heads, splits, g->v_head_dim, fixed_floats);
             wsp = fixed;
         } else if (int rc = nd::workspace(ctx, (n_o + n_ml) * sizeof(float), &wsp)) {
             return rc;
@@ -673,13 +1100,17 @@ int attend_i8(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride
         po = static_cast<float *>(wsp);
         pml = po + n_o;
     }
-    dim3 grid(unsigned(splits), unsigned(g->num_kv_heads), unsigned(count));
     fn(grid, ctx->stream, make_geom(g), static_cast<const uint8_t *>(kv), kv_stride, lo, hi, q,
-       scale, quant_query, int(splits), out, po, pml);
+       scale, quant_query, int(count), int(splits), out, po, pml);
     if (int rc = nd::check_launch("attn_i8")) return rc;
     if (splits > 1) {
-        hipLaunchKernelGGL(attn_combine_kernel, dim3(unsigned(g->num_heads), unsigned(count)),
-                           dim3(64), 0, ctx->stream, make_geom(g), int(splits), po, pml, out);
+        const dim3 cg(unsigned(g->num_heads), unsigned(count));
+        if (base2)
+            hipLaunchKernelGGL(attn_combine_kernel<true>, cg, dim3(64), 0, ctx->stream, make_geom(g),
+                               int(splits), po, pml, out);
+        else
+            hipLaunchKernelGGL(attn_combine_kernel<false>, cg, dim3(64), 0, ctx->stream, make_geom(g),
+                               int(splits), po, pml, out);
         return nd::check_launch("attn_combine");
     }
     return ND_OK;

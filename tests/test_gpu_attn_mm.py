@@ -1,0 +1,130 @@
+"""The matrix-core int8 attention (grouped query heads; prompt rows over one
+block) at the sizes where its tiles, masks and ring arithmetic can go wrong,
+against the oracle's attend_step.
+
+Tolerance: a score is a dot of at most 64 products summed in fp32 and two
+products, |score| < 16 for these N(0, 1) draws, so two summation orders
+differ by at most 16 * 66 * 2^-24 = 6.3e-5 in a score in the worst case and
+by its square root's share (8e-6) in any draw; an output is a mean of
+|v| < 5 under weights off by that much, twice (numerator and sum): 2e-5
+bounds the draws with room, against the 1e-4 bar of the entry point.
+"""
+import numpy as np
+import pytest
+import torch
+
+import needle_amd as nd
+import oracle as O
+from conftest import dev, host
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-5
+
+
+def _block(ctx, rng, H, KVH, QK, cap, npos, count=1):
+    """Blocks whose every byte and scale is garbage (NaN) until written."""
+    g = nd.kv_geom(H, KVH, QK, 64, cap)
+    blk, nb = nd.kv_alloc(g, count)
+    blk.fill_(0xff)
+    for i in range(count):
+        k = rng.normal(size=(npos, KVH * QK)).astype(np.float32)
+        v = rng.normal(size=(npos, KVH * 64)).astype(np.float32)
+        # the last `cap` positions only: earlier ones would race for a slot
+        p0 = max(0, npos - cap)
+        pos = torch.arange(p0, npos, dtype=torch.int32, device="cuda")
+        nd.kv_write(ctx, g, blk[i * nb:], 0, pos, dev(k[p0:]), dev(v[p0:]))
+    return g, blk, nb
+
+
+def _want(g, block, q, lo, hi):
+    if lo < 0 or hi < lo or hi - lo >= g.cap:
+        return np.full(g.num_heads * 64, np.nan, np.float32)
+    k, ks, v, vs = nd.kv_unpack(g, block)
+    return O.attend_step_i8(q, k.reshape(-1), ks.reshape(-1), v.reshape(-1), vs.reshape(-1), g.cap, lo, hi,
+                            g.num_heads, g.num_kv_heads, g.qk_head_dim, 64)
+
+
+def _check(ctx, g, blk, nb, lo, hi, q, quant, shared):
+    lo, hi = np.asarray(lo, np.int32), np.asarray(hi, np.int32)
+    got = host(nd.attend_step_i8(ctx, g, blk, 0 if shared else nb, dev(lo), dev(hi), dev(q), quant_query=quant))
+    b = host(blk)
+    qq = O.quant_rows(q, len(lo), g.num_heads, g.qk_head_dim).reshape(q.shape) if quant else q
+    for i in range(len(lo)):
+        want = _want(g, b[:nb] if shared else b[i * nb:(i + 1) * nb], qq[i], int(lo[i]), int(hi[i]))
+        assert np.array_equal(np.isnan(got[i]), np.isnan(want)), i
+        if not np.isnan(want).any():
+            assert np.max(np.abs(got[i] - want)) <= TOL, (i, int(lo[i]), int(hi[i]))
+
+
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("H,KVH,QK", [(12, 2, 48), (16, 2, 64), (6, 2, 64), (8, 2, 48), (4, 2, 48)])
+@pytest.mark.parametrize("cap,spans", [
+    (1, [(0, 0)]), (17, [(0, 16), (20, 36), (3, 3)]), (31, [(40, 70), (69, 70)]), (32, [(33, 64), (64, 64)]),
+    (2048, [(0, 2047), (1, 33), (100, 131), (2040, 2047)]), (1000, [(500, 1499), (999, 1001), (1480, 1499)])])
+def test_decode_grouped(ctx, H, KVH, QK, cap, spans, quant):
+    """One row a block: ragged spans, wrapped rings, rings below a chunk."""
+    rng = np.random.default_rng(cap + H + quant)
+    g, blk, nb = _block(ctx, rng, H, KVH, QK, cap, max(h for _, h in spans) + 1, len(spans))
+    q = rng.normal(size=(len(spans), H * QK)).astype(np.float32)
+    _check(ctx, g, blk, nb, *zip(*spans), q, quant, False)
+
+
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("sessions", [150, 600])
+def test_decode_many_sessions(ctx, sessions, quant):
+    """Enough sessions for both block widths, each its own ragged span."""
+    rng = np.random.default_rng(sessions)
+    g, blk, nb = _block(ctx, rng, 12, 2, 48, 96, 96, sessions)
+    hi = rng.integers(0, 96, sessions)
+    lo = np.array([rng.integers(0, h + 1) for h in hi])
+    q = rng.normal(size=(sessions, 12 * 48)).astype(np.float32)
+    _check(ctx, g, blk, nb, lo, hi, q, quant, False)
+
+
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("H,KVH,QK", [(12, 2, 48), (12, 12, 64), (6, 2, 64), (8, 4, 64)])
+@pytest.mark.parametrize("seq,window", [(2, 0), (15, 4), (33, 0), (257, 64), (1500, 100)])
+def test_prompt_rows(ctx, H, KVH, QK, seq, window, quant):
+    """A prompt's rows over one block, both tile widths (few rows, many)."""
+    rng = np.random.default_rng(seq + H)
+    g, blk, nb = _block(ctx, rng, H, KVH, QK, seq, seq)
+    rows = np.arange(seq) if seq <= 300 else np.arange(seq - 1100, seq)
+    lo = np.maximum(rows + 1 - window, 0) if window else 0 * rows
+    q = rng.normal(size=(len(rows), H * QK)).astype(np.float32)
+    if seq > 300:  # every row runs; the oracle checks some
+        got = host(nd.attend_step_i8(ctx, g, blk, 0, dev(lo.astype(np.int32)), dev(rows.astype(np.int32)),
+                                     dev(q), quant_query=quant))
+        qq = O.quant_rows(q, len(rows), H, QK).reshape(q.shape) if quant else q
+        for i in list(range(0, len(rows), 97)) + [len(rows) - 1]:
+            assert np.max(np.abs(got[i] - _want(g, host(blk), qq[i], int(lo[i]), int(rows[i])))) <= TOL, i
+    else:
+        _check(ctx, g, blk, nb, lo, rows, q, quant, True)
+
+
+@pytest.mark.parametrize("quant", [False, True])
+def test_shared_block_any_spans(ctx, quant):
+    """Rows over one ring in any order with spans that share nothing, among
+    them bad ones (NaN, that row alone) and positions far apart."""
+    H, KVH, QK, cap = 12, 2, 48, 200
+    rng = np.random.default_rng(5)
+    g, blk, nb = _block(ctx, rng, H, KVH, QK, cap, 450)
+    far = 200 * 5_000_000  # a multiple of cap: the same slots
+    spans = [(250, 449), (449, 449), (far + 60, far + 99), (300, 310), (-1, 5), (400, 399), (250, 450),
+             (255, 260), (2 ** 31 - 48, 2 ** 31 - 1), (251, 252), (far, far + 199), (0, 0)]
+    q = rng.normal(size=(len(spans), H * QK)).astype(np.float32)
+    _check(ctx, g, blk, nb, *zip(*spans), q, quant, True)
+
+
+def test_nan_query_stays_with_its_head(ctx):
+    """A NaN in one head's query makes that head's output NaN, no other's."""
+    rng = np.random.default_rng(6)
+    g, blk, nb = _block(ctx, rng, 12, 2, 48, 64, 64)
+    for quant in (False, True):
+        q = rng.normal(size=(3, 12 * 48)).astype(np.float32)
+        q[1, 7 * 48 + 20] = np.nan
+        for shared in (True, False):
+            blks = blk if shared else torch.cat([blk] * 3)
+            out = host(nd.attend_step_i8(ctx, g, blks, 0 if shared else nb, dev(np.zeros(3, np.int32)),
+                                         dev(np.full(3, 63, np.int32)), dev(q), quant_query=quant))
+            bad = np.isnan(out.reshape(3, 12, 64)).all(-1)
+            assert bad[1, 7] and bad.sum() == 1 and np.isnan(out).sum() == 64
