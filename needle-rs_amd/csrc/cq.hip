@@ -17,7 +17,9 @@
 //                conflict on banks; a group's norm multiplies the group dot
 //                as in cq.rs:731.
 //   cq_gemv_generic   any width/group (3-bit, tiny groups): bit reader.
-//   cq_matmul    batched prefill: a 64x64 output tile, the weight tile
+//   cq_matmul_mm batched prefill: fp32 operands as two f16 pieces each on
+//                the f16 matrix cores, groups of 128 columns or more.
+//   cq_matmul    smaller groups: a 64x64 output tile, the weight tile
 //                decoded to fp32 (level * norm) in LDS, fp32 MFMA 16x16x4.
 //   cq_dequant   dequantize_row (cq.rs:763-779), bit-identical.
 #include "nd_internal.h"
@@ -28,6 +30,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -1121,8 +1124,8 @@ __global__ __launch_bounds__(256) void cq_matmul_kernel(
             }
 }
 
-// The same product for the byte-aligned widths (4-bit, 2-bit, ternary), the
-// prefill path: block tile BM (batch) x 64 (rows), K steps of 32.  X is staged
+// The same product for the byte-aligned widths (4-bit, 2-bit, ternary):
+// block tile BM (batch) x 64 (rows), K steps of 32.  X is staged
 // with float4 loads; codes 8 at a time (one 16- or 32-bit load), decoded
 // through the weight's byte LUT and scaled by the group norm; the next step's
 // loads are in flight while the current step's MFMAs run.  Waves 2x2 (BM 64:
@@ -1239,6 +1242,277 @@ __global__ __launch_bounds__(256) void cq_matmul_b_kernel(
                 const int m = m0 + wm + a * 16 + rb + i;
                 const int n = n0 + wn + b * 16 + col;
                 if (m < batch && n < rows) y[size_t(m) * rows + n] = acc[a][b][i];
+            }
+}
+
+// ---------------------------------------------------------------------------
+// Batched matmul on the f16 matrix cores, fp32 in and out: groups that are
+// multiples of 128, any width.
+//
+// An fp32 value times a power of two is h + l, two f16 values, to within
+// 2^-24 of itself (h keeps 11 bits, l the next 11 and its sign one more), so
+// x . lv = xh lh + xh ll + xl lh plus a term below 2^-24 of it: three f16
+// MFMAs in place of sixteen-fold slower fp32 ones, products exact, sums
+// fp32.  The activations are scaled by a power of two per (row, 128 columns)
+// and the levels by one per weight so that h uses f16's top binade; the
+// scales go back exactly, with the norm, once per 128 columns.  Against 64
+// bits the result is closer than the fp32 MFMA kernel's was (1.0e-7 against
+// 5.0e-7 at in 768: a sum of 32-wide dots is a shorter chain).
+//
+// Block: 16 MT batch rows x 16 NL weight rows a wave, NW waves side by side
+// along the weight rows, 128 columns a step.  X is split once per block into
+// LDS (rows 272 bytes apart: fragment reads hit distinct banks).  Codes go
+// straight to the lanes that multiply them: lane (n, q) holds codes 32 q ..
+// 32 q + 31 of row n, and a pair of codes is one 8-byte read of (h pair | l
+// pair) from a table of all pairs in lane replicas.
+// What bounds it (4-bit, 512 x 8192 x 768: 48k cycles a CU): MFMA 18k, LDS
+// 12-22k, VALU 25k (X's split, the lookups' addresses, the norms), which a
+// SIMD's two waves overlap in part.
+// Measured, MI355X, against the fp32 MFMA kernels before: 500 x 768 by 8192
+// rows 4-bit 66.5 -> 26.0 us (157 -> 248 TFLOP/s of the product), 2-bit 63.7
+// -> 24.5, 3-bit 156 -> 25.1; by 768 rows 17.6 -> 9.3; 4 rows by 8192 x 768
+// 14.5 -> 7.3 (3-bit 64.0 -> 7.0).  Four waves of 64 x 64 a block: 30.0.
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t cq_u32x4 __attribute__((ext_vector_type(4)));
+typedef float cq_f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kMmLd = 136;   // halfs between X rows in LDS
+
+// Bits [pos, pos + n) of a lane's slice, constant pos and n <= 8.
+template <int ND>
+__device__ inline uint32_t slice_bits(const uint32_t (&d)[ND], int pos, int n)
+{
+    const int i = pos >> 5, sh = pos & 31;
+    const uint32_t v = sh + n > 32 ? __builtin_amdgcn_alignbit(d[i + 1 < ND ? i + 1 : i], d[i], sh) : d[i] >> sh;
+    return v & ((1u << n) - 1);
+}
+
+// The largest of a half wave's 32 values, in every lane of it: rotations
+// within 16 lanes (folded into the max), then one lane swap.
+__device__ inline uint32_t half_max_u32(uint32_t v)
+{
+    v = max(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x128, 0xf, 0xf, false)));  // row_ror:8
+    v = max(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x124, 0xf, 0xf, false)));  // row_ror:4
+    v = max(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x122, 0xf, 0xf, false)));  // row_ror:2
+    v = max(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x121, 0xf, 0xf, false)));  // row_ror:1
+    const auto sw = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return max(sw[0], sw[1]);
+}
+
+// A barrier for LDS only: global loads stay in flight across it.
+__device__ inline void lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int W, int MT, int NL, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void cq_matmul_mm_kernel(
+    const uint8_t *__restrict__ packed, const float *__restrict__ norms, const float *__restrict__ lv,
+    const float *__restrict__ xh, float *__restrict__ y, int batch, int row_start, int rows, int row_bytes,
+    int num_groups, int group, int in_padded, int ternary, float lv_scale)
+{
+    constexpr int NT = 64 * NW, BM = 16 * MT, BN = 16 * NL * NW, TE = 1 << (2 * W), ND = W;
+    constexpr int XR = BM * 32 / NT;  // X rows a thread stages per step, 4 columns each
+    // the widest tile runs one block a CU: X of the next step is split into a
+    // second buffer between this step's products
+    constexpr bool DB = NW == 8;
+    // lane replicas of the pair table: 32 take no bank conflicts, 16 leave
+    // room for two blocks a CU (conflicts: 42 % of the LDS cycles)
+    constexpr int REP = DB ? 32 : 16;
+    __shared__ __align__(16) uint2 tab[TE * REP];
+    __shared__ __align__(16) _Float16 xs[DB ? 2 : 1][2][BM][kMmLd];  // h, l
+    __shared__ __align__(16) float sx[DB ? 2 : 1][BM];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int n = lane & 15, q = lane >> 4;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN + w * (16 * NL);
+    const int steps = in_padded / 128;
+
+    // ---- loads of one step ----
+    const int xc = (t & 31) * 4, xr0 = t >> 5;
+    float4 xv[XR];
+    uint32_t code[2][NL][ND];  // this step's, the next one's
+    float nrm[2][NL];
+    const uint8_t *crow[NL];
+    const float *nrow[NL];
+#pragma unroll
+    for (int b = 0; b < NL; ++b) {
+        const int r = n0 + 16 * b + n;
+        const size_t rr = size_t(row_start) + (r < rows ? r : rows - 1);
+        crow[b] = packed + rr * row_bytes + q * (4 * W);
+        nrow[b] = norms + rr * num_groups;
+    }
+    auto load_x = [&](int c) {
+#pragma unroll
+        for (int j = 0; j < XR; ++j) {
+            const int m = m0 + xr0 + (NT / 32) * j;
+            xv[j] = *reinterpret_cast<const float4 *>(xh + size_t(m < batch ? m : batch - 1) * in_padded + c * 128 + xc);
+        }
+    };
+    auto load_w = [&](int u, int c) {
+        const int g = c * 128 / group;
+#pragma unroll
+        for (int b = 0; b < NL; ++b) {
+            const uint32_t *p = reinterpret_cast<const uint32_t *>(crow[b] + c * (16 * W));
+#pragma unroll
+            for (int d = 0; d < ND; ++d) code[u][b][d] = p[d];
+            nrm[u][b] = nrow[b][g];
+        }
+    };
+    load_x(0);
+    load_w(0, 0);
+
+    // ---- the pair table: entry e is codes (e & mask, e >> W) ----
+    for (int e = t; e < TE; e += NT) {
+        uint32_t c0 = uint32_t(e) & ((1u << W) - 1), c1 = uint32_t(e) >> W;
+        if (ternary) c0 = ternary_index(c0), c1 = ternary_index(c1);
+        const float a = lv[c0] * lv_scale, b = lv[c1] * lv_scale;
+        const f16x2_t h{_Float16(a), _Float16(b)};
+        const f16x2_t l{_Float16(a - float(h[0])), _Float16(b - float(h[1]))};
+        const uint2 v = make_uint2(__builtin_bit_cast(uint32_t, h), __builtin_bit_cast(uint32_t, l));
+#pragma unroll
+        for (int k = 0; k < REP; ++k) tab[e * REP + ((k + e) & (REP - 1))] = v;
+    }
+
+    bool odd = false;  // a value that is not finite
+    auto store_row = [&](int buf, int j) {
+        const uint32_t ab = 0x7fffffffu;
+        uint32_t mx = max(max(__float_as_uint(xv[j].x) & ab, __float_as_uint(xv[j].y) & ab),
+                          max(__float_as_uint(xv[j].z) & ab, __float_as_uint(xv[j].w) & ab));
+        mx = half_max_u32(mx);
+        odd = odd || mx >= 0x7f800000u;
+        // the row's largest |x| into [2^14, 2^15); at most 2^126
+        const uint32_t eb = min(268u - (mx >> 23), 253u);
+        const float sc = __uint_as_float(eb << 23);
+        const cq_f32x4 v = cq_f32x4{xv[j].x, xv[j].y, xv[j].z, xv[j].w} * sc;
+        const f16x4_t h = __builtin_convertvector(v, f16x4_t);
+        const f16x4_t l = __builtin_convertvector(v - __builtin_convertvector(h, cq_f32x4), f16x4_t);
+        const int r = xr0 + (NT / 32) * j;
+        *reinterpret_cast<f16x4_t *>(&xs[buf][0][r][xc]) = h;
+        *reinterpret_cast<f16x4_t *>(&xs[buf][1][r][xc]) = l;
+        if ((t & 31) == 0) sx[buf][r] = __uint_as_float((254u - eb) << 23);
+    };
+
+    cq_f32x4 acc[MT][NL];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NL; ++b) acc[a][b] = cq_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const float inv_lv = 1.0f / lv_scale;  // a power of two
+    const uint2 *tl = tab + (lane & (REP - 1));
+
+    // step c, its codes in register set u; step c + 1's loads land during its
+    // products (past the last step they repeat it)
+    auto step = [&](auto uc, int c) {
+        constexpr int u = decltype(uc)::value, xb = DB ? u : 0;
+        const int cn = c + 1 < steps ? c + 1 : c;
+        if constexpr (!DB) {
+#pragma unroll
+            for (int j = 0; j < XR; ++j) store_row(0, j);
+            lds_sync();
+            load_x(cn);
+        }
+        load_w(u ^ 1, cn);
+        // The step's 4 NL products of 32 columns by 16 weight rows, each with
+        // its operands read from LDS one product ahead (a wave may be alone
+        // on its SIMD: nothing else hides the lookups).
+        cq_f32x4 part[MT][NL];
+        f16x8_t ah[2][MT], al[2][MT];
+        uint2 e[2][4];
+        auto read_x = [&](int s) {
+#pragma unroll
+            for (int a = 0; a < MT; ++a) {
+                ah[s & 1][a] = *reinterpret_cast<const f16x8_t *>(&xs[xb][0][16 * a + n][32 * q + 8 * s]);
+                al[s & 1][a] = *reinterpret_cast<const f16x8_t *>(&xs[xb][1][16 * a + n][32 * q + 8 * s]);
+            }
+        };
+        auto read_w = [&](int i) {
+            const int s = i / NL, b = i % NL;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) e[i & 1][k] = tl[slice_bits(code[u][b], (4 * s + k) * 2 * W, 2 * W) * REP];
+        };
+        read_x(0);
+        read_w(0);
+#pragma unroll
+        for (int i = 0; i < 4 * NL; ++i) {
+            const int s = i / NL, b = i % NL;
+            if (b == NL - 1 && s < 3) read_x(s + 1);
+            if (i + 1 < 4 * NL) read_w(i + 1);
+            const uint2 *ei = e[i & 1];
+            const f16x8_t bh = __builtin_bit_cast(f16x8_t, cq_u32x4{ei[0].x, ei[1].x, ei[2].x, ei[3].x});
+            const f16x8_t bl = __builtin_bit_cast(f16x8_t, cq_u32x4{ei[0].y, ei[1].y, ei[2].y, ei[3].y});
+            const cq_f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+                part[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s & 1][a], bh, s ? part[a][b] : zero, 0, 0, 0);
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+                part[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s & 1][a], bl, part[a][b], 0, 0, 0);
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+                part[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s & 1][a], bh, part[a][b], 0, 0, 0);
+            if constexpr (DB) {
+                // the next step's rows, one every other product
+                if ((i & 1) == 1) store_row(u ^ 1, i / 2);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        static_assert(!DB || XR == 2 * NL, "a row every other product");
+        if constexpr (DB) load_x(c + 2 < steps ? c + 2 : steps - 1);
+        float nr[NL];
+#pragma unroll
+        for (int b = 0; b < NL; ++b) nr[b] = nrm[u][b] * inv_lv;
+        // the 128 columns' dots times the norm, then unscaled (in this order
+        // nothing overflows that the result does not)
+#pragma unroll
+        for (int a = 0; a < MT; ++a) {
+            const cq_f32x4 sv = *reinterpret_cast<const cq_f32x4 *>(&sx[xb][16 * a + 4 * q]);
+#pragma unroll
+            for (int b = 0; b < NL; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[a][b][i] = __builtin_fmaf(part[a][b][i] * nr[b], sv[i], acc[a][b][i]);
+        }
+        lds_sync();
+    };
+    if constexpr (DB) {
+#pragma unroll
+        for (int j = 0; j < XR; ++j) store_row(0, j);
+        load_x(1 < steps ? 1 : 0);
+        lds_sync();
+    }
+    for (int c = 0; c < steps; c += 2) {
+        step(std::integral_constant<int, 0>{}, c);
+        if (c + 1 < steps) step(std::integral_constant<int, 1>{}, c + 1);
+    }
+    if (__syncthreads_or(odd)) {
+        // infinities and NaN, which the split cannot carry: the plain sums
+        for (int o = t; o < BM * BN; o += NT) {
+            const int m = m0 + o / BN, r = int(blockIdx.x) * BN + o % BN;
+            if (m >= batch || r >= rows) continue;
+            const uint8_t *row = packed + size_t(row_start + r) * row_bytes;
+            const float *x = xh + size_t(m) * in_padded;
+            float total = 0.0f;
+            for (int g = 0; g < num_groups; ++g) {
+                float s = 0.0f;
+                for (int k = g * group; k < (g + 1) * group; ++k)
+                    s += lv[ternary ? ternary_index(read_code(row, k, W, row_bytes)) : int(read_code(row, k, W, row_bytes))] * x[k];
+                total += norms[size_t(row_start + r) * num_groups + g] * s;
+            }
+            y[size_t(m) * rows + r] = total;
+        }
+        return;
+    }
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NL; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = m0 + 16 * a + 4 * q + i, r = n0 + 16 * b + n;
+                if (m < batch && r < rows) y[size_t(m) * rows + r] = acc[a][b][i];
             }
 }
 
@@ -1602,6 +1876,57 @@ int nd_cq_matmul_rows_prepared(nd_ctx *ctx, const nd_cq *w, const float *xh, siz
     if (rows == 0 || batch == 0) return ND_OK;
     ND_REQUIRE(xh && y, "null buffer");
     ND_REQUIRE(batch <= (size_t(1) << 22), "batch too large");
+    // groups of 128 columns or more, finite levels: the f16 matrix cores
+    float top = 0.0f;
+    bool finite = true;
+    for (int i = 0; i < w->n_levels; ++i) {
+        finite = finite && std::isfinite(w->levels[i]);
+        top = std::fmax(top, std::fabs(w->levels[i]));
+    }
+    if (w->group % 128 == 0 && finite && (reinterpret_cast<uintptr_t>(xh) & 15) == 0) {
+        // the largest level into [2^14, 2^15), the scale and its inverse normal
+        int e = 0;
+        std::frexp(top, &e);
+        e = 15 - e;
+        const float lv_scale = std::ldexp(1.0f, top > 0.0f ? (e > 126 ? 126 : e < -126 ? -126 : e) : 0);
+        const size_t cus = size_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
+        // The largest tile that still gives every CU a block: 8 waves of 64 x
+        // 32 (500 rows by 8192: 26.0 us; 4-wave blocks 30), then smaller ones
+        // (128 rows by 8192: 13.5 us at 32 x 32 a wave, 19 at 64 x 32)
+        static const int kTiles[5][3] = {{4, 2, 8}, {4, 2, 4}, {2, 2, 4}, {2, 1, 4}, {1, 1, 4}};  // MT, NL, waves
+        int ti = 0;
+        size_t bx = 0, by = 0;
+        for (; ti < 5; ++ti) {
+            by = (batch + 16 * kTiles[ti][0] - 1) / (16 * kTiles[ti][0]);
+            const size_t bn = 16 * size_t(kTiles[ti][1]) * kTiles[ti][2];
+            bx = (rows + bn - 1) / bn;
+            const bool fits = kTiles[ti][0] == 1 || batch > 8 * size_t(kTiles[ti][0]);
+            if (ti == 4 || (fits && bx * by >= cus)) break;
+        }
+        if (by <= 65535) {
+            const dim3 g2{unsigned(bx), unsigned(by)};
+#define ND_MM(WW, MM, NN, NWV)                                                                                \
+    hipLaunchKernelGGL((cq_matmul_mm_kernel<WW, MM, NN, NWV>), g2, dim3(64 * NWV), 0, ctx->stream, w->packed, w->norms, \
+                       w->lv, xh, y, int(batch), int(row_start), int(rows), int(w->row_bytes),               \
+                       int(w->num_groups), int(w->group), int(w->in_padded), int(w->bits == kTernary), lv_scale)
+#define ND_MM_W(WW)                     \
+    switch (ti) {                       \
+    case 0: ND_MM(WW, 4, 2, 8); break;  \
+    case 1: ND_MM(WW, 4, 2, 4); break;  \
+    case 2: ND_MM(WW, 2, 2, 4); break;  \
+    case 3: ND_MM(WW, 2, 1, 4); break;  \
+    default: ND_MM(WW, 1, 1, 4); break; \
+    }
+            switch (code_width(w)) {
+            case 2: ND_MM_W(2) break;
+            case 3: ND_MM_W(3) break;
+            default: ND_MM_W(4) break;
+            }
+#undef ND_MM_W
+#undef ND_MM
+            return nd::check_launch("cq_matmul_mm");
+        }
+    }
     const bool bytes = (w->per_byte == 2 || w->per_byte == 4) && w->lut && w->in_padded % 8 == 0 &&
                        (reinterpret_cast<uintptr_t>(xh) & 15) == 0;
     if (bytes) {

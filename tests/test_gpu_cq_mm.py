@@ -1,0 +1,91 @@
+"""The f16 matrix-core Cactus-Quants matmul at its tile edges, against the
+same product in 64 bits.
+
+Tolerance: both operands are carried to 2^-24 of themselves and one cross
+term below 2^-24 of the product is left out; a product sum adds at most 96
+fp32 roundings in a step of 32 columns' three products and one a step and a
+group after it.  Rounding errors of either sign add as their square root: 16
+units of 2^-24 of sum |x w| bound every draw here by a factor of ten or more.
+"""
+import numpy as np
+import pytest
+import torch
+
+import needle_amd as nd
+from conftest import dev, host
+from cq_cases import TERNARY, levels_for, random_case
+
+pytestmark = pytest.mark.gpu
+CB = np.concatenate([np.sort(np.random.default_rng(b).normal(0, 0.1, 1 << b)) for b in (2, 3, 4)]).astype(np.float32)
+TOL = 16 * 2.0 ** -24
+
+
+def _weights64(c):
+    lv = levels_for(c.bits, c.group, c.codebook).astype(np.float64)
+    u = lv[c.idx].reshape(c.out, c.num_groups, c.group) * c.norms_f32.astype(np.float64)[:, :, None]
+    return u.reshape(c.out, c.in_pad)
+
+
+def _weight(ctx, c):
+    return nd.CqWeight(ctx, c.blob, c.out, c.in_feat, c.group, c.bits, c.codebook)
+
+
+def _check(ctx, c, gw, xh, r0, rows):
+    got = host(gw.matmul_rows_prepared(dev(xh), xh.shape[0], r0, rows)).reshape(xh.shape[0], rows)
+    w = _weights64(c)[r0:r0 + rows]
+    x = xh.astype(np.float64)
+    want, mag = x @ w.T, np.abs(x) @ np.abs(w).T
+    assert np.all(np.abs(got - want) <= TOL * mag + 1e-37), np.max(np.abs(got - want) / (mag + 1e-300))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, TERNARY])
+@pytest.mark.parametrize("out,inn,group,batch,r0,rows", [
+    (1, 1, 128, 1, 0, 1), (64, 128, 128, 16, 0, 64), (65, 200, 128, 17, 0, 65), (300, 768, 128, 15, 7, 193),
+    (300, 700, 256, 33, 1, 299), (130, 1024, 1024, 65, 0, 130), (520, 512, 512, 9, 3, 517),
+    (4100, 384, 128, 130, 0, 4100), (8192, 256, 128, 520, 0, 8192)])
+def test_tiles(ctx, bits, out, inn, group, batch, r0, rows):
+    """One row to several tiles of every tile shape, ragged in all three."""
+    rng = np.random.default_rng(out + inn + bits)
+    c = random_case(rng, out, inn, group, bits, CB)
+    xh = rng.normal(size=(batch, c.in_pad)).astype(np.float32)
+    _check(ctx, c, _weight(ctx, c), xh, r0, rows)
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, TERNARY])
+def test_scales(ctx, bits):
+    """Rows and 128-column groups whose sizes lie from subnormal to the
+    largest floats, a wide range within a group, and a zero group."""
+    rng = np.random.default_rng(bits)
+    c = random_case(rng, 96, 512, 128, bits, CB)
+    xh = rng.normal(size=(40, 512)).astype(np.float32)
+    scale = np.float32(2.0) ** rng.integers(-140, 118, size=(40, 4, 1)).astype(np.float32)
+    xh = (xh.reshape(40, 4, 128) * scale).astype(np.float32)
+    xh[:, 1, ::3] *= np.float32(2.0 ** -12)
+    xh[5, 2] = 0
+    xh = xh.reshape(40, 512)
+    # a row with one large group: the small groups vanish beside it in fp32 too
+    got = host(_weight(ctx, c).matmul_rows_prepared(dev(xh), 40, 0, 96)).reshape(40, 96)
+    w, x = _weights64(c), xh.astype(np.float64)
+    want, mag = x @ w.T, np.abs(x) @ np.abs(w).T
+    ok = mag < 1e38
+    assert np.all(np.abs(got - want)[ok] <= TOL * mag[ok] + 1e-43)
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_not_finite(ctx, bits):
+    """An infinity or NaN reaches its own row's outputs and no other's."""
+    rng = np.random.default_rng(10 + bits)
+    c = random_case(rng, 200, 300, 128, bits, CB)
+    xh = rng.normal(size=(70, c.in_pad)).astype(np.float32)
+    xh[3, 17], xh[66, 299], xh[20, 5] = np.inf, -np.inf, np.nan
+    got = host(_weight(ctx, c).matmul_rows_prepared(dev(xh), 70, 0, 200)).reshape(70, 200)
+    w = _weights64(c)
+    with np.errstate(invalid="ignore"):
+        want = xh.astype(np.float64) @ w.T
+    for r in range(70):
+        if r == 20:
+            assert np.isnan(got[r]).all()
+        elif r in (3, 66):
+            assert np.array_equal(got[r], want[r].astype(np.float32), equal_nan=True)
+        else:
+            assert np.all(np.abs(got[r] - want[r]) <= TOL * (np.abs(xh[r]).astype(np.float64) @ np.abs(w).T))
