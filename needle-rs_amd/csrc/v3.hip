@@ -38,6 +38,7 @@
 #include <memory>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -851,6 +852,30 @@ __device__ void mhc_gates_phase1(const MhcIn &a, size_t b)
     if (tid < n * n) a.gr[b * n * n + tid] = m;
 }
 
+// The same gates for a prefill pass's rows, on the side stream: all
+// iterations in one launch; with n = 4 a wave takes four rows, 16 lanes each
+// (k_mhc_gates, one row a wave, through shuffles: 37 us for 2048 rows; this
+// one 32).
+__global__ __launch_bounds__(256) void k_mhc_gates_rows(MhcIn a, int rows)
+{
+    const int tid = threadIdx.x, n = a.n, rw = n + n * n;
+    const bool four = n == 4;
+    const int row = four ? int(blockIdx.x) * 16 + (tid >> 4) : int(blockIdx.x) * 4 + (tid >> 6);
+    const int l = four ? tid & 15 : tid & 63;
+    // every lane stays (the lane moves read their partners); rows past the
+    // end repeat the last one
+    const size_t b = row < rows ? row : rows - 1;
+    const float *raw = a.graw + b * rw;
+    float m = l < n * n ? a.a_res * raw[n + l] + a.b_res[l] : 0.0f;
+    m = nd_expf(sinkhorn_iters(m, n, 0, kSinkhornIters));
+    if (row >= rows) return;
+    if (l < n) {
+        const float off = l == a.layer % n ? 0.0f : -4.0f;
+        a.gp[b * n + l] = 2.0f * sigmoidf_(a.a_post * raw[l] + a.b_post[l] + off);
+    }
+    if (l < n * n) a.gr[b * n * n + l] = m;
+}
+
 // ---- after the projections: causal conv step over q/k/v with the retained
 // tails (cache.rs:401-438), ZCRMSNorm + RoPE on q and k
 // (attention.rs:108-150), q to global, and k and v quantised straight into
@@ -909,15 +934,22 @@ __device__ inline float conv_rows(const float *rows, const float *tail, const fl
 
 // After a step of C positions: each session's tail of the last `keep`
 // values of `rows` (row stride `dim`, the session's C rows consecutive),
-// older entries shifted in from the previous tail when C < keep.
-__global__ void k_tails(const float *__restrict__ rows, float *__restrict__ tail, int keep, int C,
-                        int dim)
+// older entries shifted in from the previous tail when C < keep.  Up to
+// three (rows, tail, dim) sets in one launch (q, k and v: 16 us a layer of a
+// 2048-row pass as three launches, 6 as one), blockIdx.z the set.
+struct Tails {
+    const float *rows[3];
+    float *tail[3];
+    int dim[3];
+};
+__global__ void k_tails(Tails a, int keep, int C)
 {
     const size_t s = blockIdx.y;
+    const int z = blockIdx.z, dim = a.dim[z];
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= dim || keep <= 0) return;
-    float *tb = tail + s * size_t(keep) * dim;
-    const float *rb = rows + s * size_t(C) * dim;
+    float *tb = a.tail[z] + s * size_t(keep) * dim;
+    const float *rb = a.rows[z] + s * size_t(C) * dim;
     float old[16];
     for (int k = 0; k < keep && k < 16; ++k) old[k] = tb[size_t(k) * dim + c];
     for (int k = 0; k < keep && k < 16; ++k) {
@@ -1353,6 +1385,8 @@ __device__ inline void kron32(const float *zT, const float *aT, const float *bT,
 
 constexpr int kMaxCondRegs = 8;     // cond_v / cond_u values a thread preloads
 constexpr int kCondProd = 6144;     // conditioning products held in LDS at once
+// rows up to which a pass's k_post_hada has a CU a row
+constexpr int kHadaOneRow = 256;
 
 
 __global__ __launch_bounds__(1024) void k_post_hada(HadaArgs a, MhcIn mhc)
@@ -1519,6 +1553,225 @@ __global__ __launch_bounds__(1024) void k_post_hada(HadaArgs a, MhcIn mhc)
         a.bx[b * d + tid] = nb;
         a.y[b * d + tid] = nb - uv;
     }
+}
+
+// The same for the rows of a prefill pass, RB rows a workgroup.  One row a
+// workgroup is bound by its sequential sums (two norms of d terms and the
+// conditioning chains on one wave, the others idle) and by LDS: every
+// Kronecker term reads both factors from it.  Here the RB rows' chains run
+// side by side on the lanes of one wave; a wave owns two values of k (the
+// factor a[.][k] is uniform: scalar loads) and a lane one l of one of two
+// rows, with b[.][l] in registers, so a term reads LDS once for two products;
+// and t[k][.] never leaves the wave.  The operations of a row and their order
+// are those of k_post_hada.
+// Bound by LDS reads and the VALU; measured (2048 rows, MI355X): 128.8 us a
+// layer in workgroups of one row, 53.7 so.
+typedef const __attribute__((address_space(4))) float *const_f32;
+
+template <int RB>
+__global__ __launch_bounds__(1024) void k_post_hada_rows(HadaArgs a, int rows)
+{
+    constexpr int LD = 1028;  // a row's stride: chain lanes in distinct banks
+    __shared__ __align__(16) float z[RB][32 * kKS], o[RB][LD], x[RB][LD], cvs[kCondProd], tw[16][2][64];
+    __shared__ float tot[RB], proj[RB][8];
+    const int tid = threadIdx.x, d = a.d, r = a.rank;
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row0 = int(blockIdx.x) * RB;
+    const bool ch = tid < d;
+    const int cc = ch ? tid : 0;
+    int base[RB];  // rows past the end repeat the last one, unwritten
+#pragma unroll
+    for (int q = 0; q < RB; ++q) base[q] = (row0 + q < rows ? row0 + q : rows - 1) * d + cc;
+    float nb[RB], xv[RB];
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        xv[q] = a.proj[base[q]];
+        nb[q] = a.bx[base[q]];
+    }
+    const float post_n = a.post_norm[cc];
+#pragma unroll
+    for (int q = 0; q < RB; ++q) o[q][tid] = xv[q] * xv[q];
+    lds_barrier();
+    if (tid < RB) tot[tid] = 1.0f / sqrtf(chain_sum(o[tid], d) / float(d) + 1e-6f);
+    const float pre_n = a.pre_hada[cc];
+    const float d1 = a.d1[tid], d2 = a.d2[tid], b2 = a.b2[tid], d3 = a.d3[tid], d4 = a.d4[tid];
+    const int p1 = a.p1[tid], p2 = a.p2perm[tid];
+    float cu[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) cu[j] = a.cond_u[j < r ? j * 1024 + tid : tid];
+    for (int e = tid; e < d * r; e += 1024) cvs[e] = a.cond_v[e];
+    // which factors hold a zero (their products are skipped, kron_apply)
+    const unsigned zb = unsigned(a.w1a[tid] == 0.0f) | unsigned(a.w2a[tid] == 0.0f) << 1 |
+                        unsigned(a.w3a[tid] == 0.0f) << 2;
+    unsigned zf = 0;
+    if (__syncthreads_or(int(zb & 1u))) zf |= 1u;
+    if (__syncthreads_or(int(zb & 2u))) zf |= 2u;
+    if (__syncthreads_or(int(zb & 4u))) zf |= 4u;
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        const float pn = (1.0f + post_n) * xv[q] * tot[q];
+        nb[q] = nb[q] + a.agate * pn;
+        o[q][tid] = nb[q] * nb[q];
+    }
+    lds_barrier();
+    if (tid < RB) tot[tid] = 1.0f / sqrtf(chain_sum(o[tid], d) / float(d) + 1e-6f);
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        xv[q] = ch ? (1.0f + pre_n) * nb[q] * tot[q] : 0.0f;
+        x[q][tid] = xv[q];
+        z[q][kron_t(tid)] = xv[q] * d1;
+    }
+    lds_barrier();
+    if (tid < 8 * RB) {
+        // cond = 1 + softmax(x . cond_v) . cond_u: lane 8 q + j runs row q's
+        // chain j over the model dim; the operands of sixteen terms are read
+        // while the sixteen before them are added
+        const int q = tid >> 3, j = tid & 7, jc = j < r ? j : 0;
+        const float *xr = x[q], *cv = cvs + jc;
+        float acc = 0.0f;
+        float4 xa[2][4];
+        float ca[2][16];
+        auto read = [&](int u, int i0) {
+            const float *cp = cv + i0 * r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xa[u][e] = *reinterpret_cast<const float4 *>(xr + i0 + 4 * e);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) ca[u][e] = cp[e * r];
+        };
+        auto add = [&](int u) {
+            float pr[16];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v[4] = {xa[u][e].x, xa[u][e].y, xa[u][e].z, xa[u][e].w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) pr[4 * e + k] = v[k] * ca[u][4 * e + k];
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc += pr[e];
+        };
+        int i = 0;
+        if (d >= 32) {
+            __builtin_amdgcn_s_setprio(2);
+            read(0, 0);
+            for (; i + 32 <= d; i += 32) {
+                read(1, i + 16);
+                __builtin_amdgcn_sched_barrier(0);
+                add(0);
+                read(0, i + 48 <= d ? i + 32 : 0);  // past the end: unused
+                __builtin_amdgcn_sched_barrier(0);
+                add(1);
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        for (; i < d; ++i) acc += xr[i] * cv[i * r];
+        // softmax over the r projections: the max is order-free, the sum one
+        // chain in j order
+        const float pj = j < r ? acc : -INFINITY;
+        float m2 = fmaxf(pj, ndl::wave_xor<1>(pj));
+        m2 = fmaxf(m2, ndl::wave_xor<2>(m2));
+        m2 = fmaxf(m2, ndl::wave_xor<4>(m2));
+        const float e = j < r ? nd_expf(pj - m2) : 0.0f;
+        float sum = 0.0f;
+        for (int u = 0; u < r; ++u) sum += __shfl(e, (lane & ~7) + u, 64);
+        if (j < r) proj[q][j] = e / sum;
+    }
+    lds_barrier();
+    float cond[RB];
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        float c = 1.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (j < r && proj[q][j] != 0.0f) c += proj[q][j] * cu[j];
+        cond[q] = c;
+    }
+    // o[row][k * 32 + l] = sum_j (sum_i z[row][i][l] a[i][k]) b[j][l]; with
+    // AZ (TZ) a factor (a t) of zero skips its product
+    auto first = [&](auto az, const float *zr, const const_f32 a0, const const_f32 a1, float &t0, float &t1)
+                     __attribute__((always_inline)) {
+        constexpr bool AZ = decltype(az)::value;
+#pragma unroll
+        for (int i0 = 0; i0 < 32; i0 += 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(zr + i0);
+            const float z4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float f0 = a0[i0 + u], f1 = a1[i0 + u];
+                const float p0 = z4[u] * f0, p1 = z4[u] * f1;
+                t0 = AZ && f0 == 0.0f ? t0 : t0 + p0;
+                t1 = AZ && f1 == 0.0f ? t1 : t1 + p1;
+            }
+        }
+    };
+    auto second = [&](auto tz, const float *ta, const float *tb, const float (&bv)[32], float &s0, float &s1)
+                      __attribute__((always_inline)) {
+        constexpr bool TZ = decltype(tz)::value;
+#pragma unroll
+        for (int j0 = 0; j0 < 32; j0 += 4) {
+            const float4 u0 = *reinterpret_cast<const float4 *>(ta + j0);
+            const float4 u1 = *reinterpret_cast<const float4 *>(tb + j0);
+            const float v0[4] = {u0.x, u0.y, u0.z, u0.w}, v1[4] = {u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float p0 = v0[u] * bv[j0 + u], p1 = v1[u] * bv[j0 + u];
+                s0 = TZ && v0[u] == 0.0f ? s0 : s0 + p0;
+                s1 = TZ && v1[u] == 0.0f ? s1 : s1 + p1;
+            }
+        }
+    };
+    auto pass = [&](auto az, const float *ap, const float *bp) __attribute__((always_inline)) {
+        const int rr = lane >> 5, l = lane & 31;
+        float bv[32];
+#pragma unroll
+        for (int j = 0; j < 32; j += 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(bp + l * 32 + j);
+            bv[j] = v.x, bv[j + 1] = v.y, bv[j + 2] = v.z, bv[j + 3] = v.w;
+        }
+        const const_f32 a0 = (const_f32)(uintptr_t)(ap + w * 32), a1 = (const_f32)(uintptr_t)(ap + (w + 16) * 32);
+#pragma unroll 1
+        for (int q = 0; q < RB; q += 2) {
+            float t0 = 0.0f, t1 = 0.0f, s0 = 0.0f, s1 = 0.0f;
+            first(az, z[q + rr] + l * kKS, a0, a1, t0, t1);
+            wave_lds_sync();  // the rows before have been read
+            tw[w][0][lane] = t0;
+            tw[w][1][lane] = t1;
+            wave_lds_sync();
+            const float *ta = &tw[w][0][32 * rr], *tb = &tw[w][1][32 * rr];
+            if (__any(t0 == 0.0f || t1 == 0.0f))
+                second(std::true_type{}, ta, tb, bv, s0, s1);
+            else
+                second(std::false_type{}, ta, tb, bv, s0, s1);
+            o[q + rr][w * 32 + l] = s0;
+            o[q + rr][(w + 16) * 32 + l] = s1;
+        }
+        lds_barrier();
+    };
+    auto kron = [&](const float *ap, const float *bp, bool a_zero) __attribute__((always_inline)) {
+        if (a_zero)
+            pass(std::true_type{}, ap, bp);
+        else
+            pass(std::false_type{}, ap, bp);
+    };
+    kron(a.w1a, a.w1b, zf & 1u);
+#pragma unroll
+    for (int q = 0; q < RB; ++q) {
+        const float zz = d2 * cond[q] * o[q][p1] + b2;
+        z[q][kron_t(tid)] = zz * sigmoidf_(zz);
+    }
+    lds_barrier();
+    kron(a.w2a, a.w2b, zf & 2u);
+#pragma unroll
+    for (int q = 0; q < RB; ++q) z[q][kron_t(tid)] = o[q][p2] * d3;
+    lds_barrier();
+    kron(a.w3a, a.w3b, zf & 4u);
+#pragma unroll
+    for (int q = 0; q < RB; ++q)
+        if (ch && row0 + q < rows) {
+            const float v = nb[q] + o[q][tid] * d4;
+            a.bx[base[q]] = v;
+            a.y[base[q]] = v - a.u[base[q]];
+        }
 }
 
 // ---- the last layer's scatter up, lane mean, final norm (model.rs:360-368),
@@ -2455,7 +2708,7 @@ struct StepRun {
     hipStream_t st = nullptr;
     float qk_scale = 1.0f;
     int kf = 0;
-    bool gate_fused = false, gates_in = false;
+    bool gate_fused = false, gates_in = false, phi_in = false;
     const nd_cq *phi = nullptr, *fpo = nullptr, *fre = nullptr;
     float *ev_conv = nullptr;  // [sites][Rcap][d], after the conv
     // tokens == nullptr: this step's tokens are b->next on the device (the
@@ -2570,21 +2823,23 @@ int StepRun::begin(const int32_t *tokens)
     gate_fused = c.v_head_dim == 64 && m->pre_attn.group == 128 &&
                  m->pre_attn.in_padded == od && m->layers[0].out->per_byte != 0;
     phi = m->phi_pre;
-    // The scatter-up gates ride in the layer's launches (k_layer_in's phi
-    // rows, second workgroups of k_qkv_kv and k_post_hada) for single
-    // positions when the phi weights fit; else (and for prefill passes)
-    // they run on the side stream, joined by events.
+    // When the phi weights fit, k_layer_in forms the raw scatter-up gates
+    // beside its own phi rows (phi_in; a separate projection launch of 20
+    // rows by 3072 took 185 us for a pass of 2048 rows).  A single position's
+    // gates then ride in the layer's launches (gates_in: second workgroups of
+    // k_qkv_kv and k_post_hada); a prefill pass's run on the side stream,
+    // joined by events, and so does everything where the weights do not fit.
     fpo = m->phi_post;
     fre = m->phi_res;
-    gates_in = (phi->per_byte == 2 || phi->per_byte == 4) && phi->group == 128 &&
+    phi_in = (phi->per_byte == 2 || phi->per_byte == 4) && phi->group == 128 &&
                   fpo->per_byte == phi->per_byte && fre->per_byte == phi->per_byte &&
                   fpo->group == 128 && fre->group == 128 &&
                   fpo->in_padded == phi->in_padded && fre->in_padded == phi->in_padded &&
                   size_t(2 * nl + nl * nl) * phi->num_groups <= size_t(kMaxPhiPairs) &&
                   size_t(2 * nl + nl * nl) * phi->num_groups <=
                       size_t((kMaxPhiPairs + kLayerInThreads - 1) / kLayerInThreads * kLayerInThreads) &&
-                  nl * nl <= 64 && fpo->row_bytes % 16 == 0 && fre->row_bytes % 16 == 0 &&
-                  C == 1;
+                  nl * nl <= 64 && fpo->row_bytes % 16 == 0 && fre->row_bytes % 16 == 0;
+    gates_in = phi_in && C == 1;
     ev_conv = C == 1 ? b->ev : b->evc;
     return ND_OK;
 }
@@ -2689,8 +2944,8 @@ int StepRun::enqueue(int phase, bool argmax)
                                    site.taps, b->et[s], pos_dev, c.e_conv_taps, c.e_conv_dilation, mo,
                                    reach, d, C);
                 LCHK("k_engram_conv_rows");
-                hipLaunchKernelGGL(k_tails, dim3((d + 255) / 256, S), dim3(256), 0, st,
-                                   b->ev + size_t(s) * Rcap * d, b->et[s], reach, C, d);
+                const Tails ta{{b->ev + size_t(s) * Rcap * d}, {b->et[s]}, {d}};
+                hipLaunchKernelGGL(k_tails, dim3((d + 255) / 256, S), dim3(256), 0, st, ta, reach, C);
                 LCHK("k_tails");
             }
         }
@@ -2711,7 +2966,7 @@ int StepRun::enqueue(int phase, bool argmax)
         LayerIn in{b->lanes, b->y, b->gp, b->gr, li > 0, b->nxh, m->pre_nx, phi->packed,
                    phi->norms, phi->lv, phi->row_bytes, int(phi->num_groups), li * nl,
                    int(phi->bits == 5), m->b_pre + size_t(li) * nl, m->a_pre[li], li, nl, d,
-                   gates_in ? 1 : 0, fpo->packed, fre->packed, fpo->norms, fre->norms, fpo->lv, fre->lv,
+                   phi_in ? 1 : 0, fpo->packed, fre->packed, fpo->norms, fre->norms, fpo->lv, fre->lv,
                    fpo->row_bytes, fre->row_bytes, li * nl, li * nl * nl, int(fpo->bits == 5),
                    int(fre->bits == 5), b->graw,
                    site >= 0 ? b->ek + size_t(site) * Rcap * d : nullptr,
@@ -2722,22 +2977,40 @@ int StepRun::enqueue(int phase, bool argmax)
         else
             hipLaunchKernelGGL((k_layer_in<4, kLayerInThreads>), dim3(B), dim3(kLayerInThreads), 0, st, in);
         LCHK("k_layer_in");
+        // this layer's scatter-up gates
+        MhcIn mi{};
+        mi.on = gates_in ? 1 : 0;
+        mi.graw = b->graw;
+        mi.n = nl;
+        mi.layer = li;
+        mi.split = kGateSplit;
+        mi.b_post = m->b_post + size_t(li) * nl;
+        mi.b_res = m->b_res + size_t(li) * nl * nl;
+        mi.a_post = m->a_post[li];
+        mi.a_res = m->a_res[li];
+        mi.gp = b->gp;
+        mi.gr = b->gr;
+        mi.state = b->gstate;
         if (!gates_in) {
             // side stream: this layer's scatter-up gates from the prepared lanes
             ND_HIP(hipEventRecord(b->ev_in[li & 1], st));
             ND_HIP(hipStreamWaitEvent(side, b->ev_in[li & 1], 0));
-            {
+            if (phi_in) {
+                const unsigned per = nl == 4 ? 16 : 4;
+                hipLaunchKernelGGL(k_mhc_gates_rows, dim3((unsigned(B) + per - 1) / per), dim3(256), 0, side,
+                                   mi, B);
+                LCHK("k_mhc_gates_rows");
+            } else {
                 const nd_cq *ws[2] = {m->phi_post, m->phi_res};
                 const size_t r0[2] = {size_t(li) * nl, size_t(li) * nl * nl};
                 const size_t nr[2] = {size_t(nl), size_t(nl) * nl};
                 float *ys[2] = {b->hpost, b->hres};
                 CK(nd_cq_exact_set(ctx, side, 2, ws, b->nxh, size_t(B), r0, nr, ys, "v3 phi post/res"));
+                MhcGates mg{b->hpost, b->hres, mi.b_post, mi.b_res, mi.a_post, mi.a_res, li, nl,
+                            b->gp, b->gr};
+                hipLaunchKernelGGL(k_mhc_gates, dim3(B), dim3(64), 0, side, mg);
+                LCHK("k_mhc_gates");
             }
-            MhcGates mg{b->hpost, b->hres, m->b_post + size_t(li) * nl,
-                        m->b_res + size_t(li) * nl * nl, m->a_post[li], m->a_res[li], li, nl,
-                        b->gp, b->gr};
-            hipLaunchKernelGGL(k_mhc_gates, dim3(B), dim3(64), 0, side, mg);
-            LCHK("k_mhc_gates");
             ND_HIP(hipEventRecord(b->ev_gates[li & 1], side));
         }
         // q, k, v and gate projections of the prepared h, one launch
@@ -2747,22 +3020,6 @@ int StepRun::enqueue(int phase, bool argmax)
             const size_t nr[4] = {size_t(qd), size_t(kd), size_t(vd), size_t(od)};
             float *ys[4] = {b->q, b->k, b->v, b->gate};
             CK(nd_cq_exact_set(ctx, st, 4, ws, b->hh, size_t(B), r0, nr, ys, "v3 qkv/gate"));
-        }
-        // this layer's scatter-up gates, when they ride in the layer's launches
-        MhcIn mi{};
-        if (gates_in) {
-            mi.on = 1;
-            mi.graw = b->graw;
-            mi.n = nl;
-            mi.layer = li;
-            mi.split = kGateSplit;
-            mi.b_post = m->b_post + size_t(li) * nl;
-            mi.b_res = m->b_res + size_t(li) * nl * nl;
-            mi.a_post = m->a_post[li];
-            mi.a_res = m->a_res[li];
-            mi.gp = b->gp;
-            mi.gr = b->gr;
-            mi.state = b->gstate;
         }
         const unsigned gy = gates_in ? 2u : 1u;
         const nd_kv_geom &g = b->geom[li];
@@ -2797,12 +3054,9 @@ int StepRun::enqueue(int phase, bool argmax)
                 LCHK("k_qkv_kv");
                 const int tt = c.qkv_conv_taps - 1;
                 if (tt > 0) {
-                    hipLaunchKernelGGL(k_tails, dim3((qd + 255) / 256, S), dim3(256), 0, st, b->q,
-                                       b->qt[li], tt, C, qd);
-                    hipLaunchKernelGGL(k_tails, dim3((kd + 255) / 256, S), dim3(256), 0, st, b->k,
-                                       b->kt[li], tt, C, kd);
-                    hipLaunchKernelGGL(k_tails, dim3((vd + 255) / 256, S), dim3(256), 0, st, b->v,
-                                       b->vt[li], tt, C, vd);
+                    const Tails ta{{b->q, b->k, b->v}, {b->qt[li], b->kt[li], b->vt[li]}, {qd, kd, vd}};
+                    const int widest = qd > kd ? (qd > vd ? qd : vd) : (kd > vd ? kd : vd);
+                    hipLaunchKernelGGL(k_tails, dim3((widest + 255) / 256, S, 3), dim3(256), 0, st, ta, tt, C);
                     LCHK("k_tails");
                 }
             }
@@ -2860,8 +3114,21 @@ int StepRun::enqueue(int phase, bool argmax)
             ha.sdim[1] = kd;
             ha.sdim[2] = vd;
         }
-        hipLaunchKernelGGL(k_post_hada, dim3(unsigned(B), gy), dim3(1024), 0, st, ha, mi);
-        LCHK("k_post_hada");
+        if (!gates_in && ha.shift_taps <= 1 && l.cond_rank <= 8 && d * l.cond_rank <= kCondProd &&
+            d <= 1024 && B > kHadaOneRow) {
+            // a CU's rows in one workgroup, up to eight
+            const unsigned bu = unsigned(B);
+            if (B <= 2 * kHadaOneRow)
+                hipLaunchKernelGGL((k_post_hada_rows<2>), dim3((bu + 1) / 2), dim3(1024), 0, st, ha, B);
+            else if (B <= 4 * kHadaOneRow)
+                hipLaunchKernelGGL((k_post_hada_rows<4>), dim3((bu + 3) / 4), dim3(1024), 0, st, ha, B);
+            else
+                hipLaunchKernelGGL((k_post_hada_rows<8>), dim3((bu + 7) / 8), dim3(1024), 0, st, ha, B);
+            LCHK("k_post_hada_rows");
+        } else {
+            hipLaunchKernelGGL(k_post_hada, dim3(unsigned(B), gy), dim3(1024), 0, st, ha, mi);
+            LCHK("k_post_hada");
+        }
         return ND_OK;
     }
     // ---- head ---------------------------------------------------------------
