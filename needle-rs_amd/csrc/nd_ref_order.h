@@ -38,6 +38,17 @@ int nd_attend_exact_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_
                          const float *q, float scale, int quant_query, float *out,
                          const float *gate = nullptr, int kv_f32 = 0);
 
+// A prefill pass's attention at the shipped grouping (six query heads a kv
+// head, qk 48, v 64, int8): bit for bit nd_attend_exact_rows with
+// quant_query over q already fake-quantised, with the gated epilogue.
+// `max_span` bounds the spans of the rows.  nd_attend_rows_fit: whether the
+// geometry, the number of rows and the span take it.
+bool nd_attend_rows_fit(nd_ctx *ctx, const nd_kv_geom *g, size_t count, int max_span);
+int nd_attend_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride, size_t count,
+                   int rows_per_block, const int32_t *lo, const int32_t *hi, const float *q, float scale,
+                   float *out, const float *gate, int max_span);
+
+
 // One 128-wide group of a Cactus-Quants row dotted with a prepared
 // activation group in the reference's order (cq.rs:838-873): element e into
 // lane e % 8, each lane a chain over the 16 elements it holds, the lanes

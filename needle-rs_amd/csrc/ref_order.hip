@@ -580,6 +580,225 @@ __global__ __launch_bounds__(kAttn2Threads, 4) void attn_exact2_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// A prefill pass's attention over the int8 ring, six query heads a kv head
+// (attend_step's order, attention.rs:327-377): one wave a (row, kv head).
+// attn_exact2_kernel gives every (row, query head) a workgroup, so each K and
+// V code is converted six times and each weighted value crosses LDS to the
+// wave that adds it; that pays where a decode step has few rows, and a pass has
+// thousands.  Here the wave runs the row's six heads together:
+//   scores  a lane a position; a converted K code feeds six chains, the
+//           query a scalar operand;
+//   sums    six lanes, one chain each;
+//   values  a lane two columns of three heads (the half waves split the six):
+//           a converted V code feeds three chains, products in registers.
+// So a (row, head, position) costs 96 + 128 multiply-adds' operations and about
+// 60 more; nothing waits at a barrier, and the waves of a CU overlap each
+// other's sums.  Every float operation and its order are the reference's.
+// Bound by the VALU.  Measured (64 sessions x 32 rows at 512 positions,
+// MI355X): 253 us a layer as workgroups of one (row, head), 96 so over a
+// prompt (55 with six heads a wave on its short spans, 143 with three on its long).
+constexpr int kRowHeads = 6, kRowQk = 48, kRowVd = 64;
+// Where it pays (ms a pass of all 20 layers, this kernel / the workgroup a
+// (row, head)): a wave takes its spans in sequence, so it needs four of them
+// a CU (512 rows at position 512: 4.85 / 5.55; one session's 256: 4.0 / 3.4),
+// and the scores of six heads in LDS leave too few waves a CU on long spans:
+// three heads a wave above kRowSix (2048 rows at 512: 12.4, six heads 12.9;
+// at 256: 11.0, six heads 10.7), the workgroup kernel above kRowSpan (at 2048:
+// 20.5 / 21.3; at 2304: 21.7 / 21.5).
+constexpr size_t kRowFill = 4;
+constexpr int kRowSix = 352, kRowSpan = 2176;
+typedef const __attribute__((address_space(4))) float *const_f32;
+
+__device__ inline void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+template <int NH>
+__global__ __launch_bounds__(64) void attn_rows_kernel(
+    ndkv::Geom g, const uint8_t *__restrict__ kv, size_t stride, const int32_t *__restrict__ lo,
+    const int32_t *__restrict__ hi, const float *__restrict__ q, float scale, float *__restrict__ out,
+    const float *__restrict__ gate, int groups, int rows_per_block, int sp)
+{
+    extern __shared__ __align__(16) float sc[];  // [NH][sp] scores, exps, weights
+    constexpr int QK = kRowQk, VD = kRowVd, PARTS = kRowHeads / NH, CW = NH == kRowHeads ? 2 : 1;
+    // the rows of a (session, kv head) share an XCD's L2 (dealt round-robin)
+    const int xcd = int(blockIdx.x) & 7, slot8 = int(blockIdx.x) >> 3;
+    const int grp = (slot8 / (rows_per_block * PARTS)) * 8 + xcd;
+    if (grp >= groups) return;
+    const int sess = grp / g.KVH, kvh = grp - sess * g.KVH;
+    const int i = sess * rows_per_block + slot8 / PARTS % rows_per_block;
+    const int h0 = kvh * kRowHeads + slot8 % PARTS * NH;  // the wave's first head
+    const int lane = threadIdx.x;
+    const int p0 = lo[i];
+    const int span = hi[i] - p0 + 1;
+    const size_t orow = (size_t(i) * g.H + h0) * VD;
+    if (p0 < 0 || span < 1 || span > g.cap || (span + 63) / 64 * 64 + 36 > sp) {
+        for (int h = 0; h < NH; ++h) out[orow + size_t(h) * VD + lane] = NAN;
+        return;
+    }
+    const uint8_t *blk = kv + size_t(sess) * stride;
+    const int8_t *kb = reinterpret_cast<const int8_t *>(blk) + size_t(kvh) * g.cap * QK;
+    const int8_t *vb = reinterpret_cast<const int8_t *>(blk + g.v_off) + size_t(kvh) * g.cap * VD;
+    const float *ks = reinterpret_cast<const float *>(blk + g.ks_off) + size_t(kvh) * g.cap;
+    const float *vs = reinterpret_cast<const float *>(blk + g.vs_off) + size_t(kvh) * g.cap;
+    const int base = p0 % g.cap;
+    auto slot_of = [&](int t) {
+        const int s = base + t;
+        return s >= g.cap ? s - g.cap : s;
+    };
+    const const_f32 qv = (const_f32)(uintptr_t)(q + (size_t(i) * g.H + h0) * QK);
+
+    // ---- scores ----
+    float mx[NH];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) mx[h] = -INFINITY;
+    uint4 kw[3];
+    float kscale;
+    auto load_k = [&](int t0) {
+        const int t = t0 + lane, s = slot_of(t < span ? t : span - 1);
+        const uint4 *kr = reinterpret_cast<const uint4 *>(kb + size_t(s) * QK);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) kw[c] = kr[c];
+        kscale = ks[s];
+    };
+    load_k(0);
+    for (int t0 = 0; t0 < span; t0 += 64) {
+        const uint32_t dw[12] = {kw[0].x, kw[0].y, kw[0].z, kw[0].w, kw[1].x, kw[1].y,
+                                 kw[1].z, kw[1].w, kw[2].x, kw[2].y, kw[2].z, kw[2].w};
+        const float kc = kscale;
+        load_k(t0 + 64 < span ? t0 + 64 : t0);
+        float acc[NH];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) acc[h] = 0.0f;
+        // the query four elements of each head at a time, the next four in
+        // flight (all 288 would not fit the scalar registers)
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        typedef const __attribute__((address_space(4))) f4 *const_f4;
+        f4 qn[2][NH];
+        auto load_q = [&](int u, int c) {
+            const_f32 qq = qv;
+            asm volatile("" : "+s"(qq));  // load here, not before the loop
+#pragma unroll
+            for (int h = 0; h < NH; ++h) qn[u][h] = *(const_f4)(qq + h * QK + 4 * c);
+        };
+        load_q(0, 0);
+#pragma unroll
+        for (int c = 0; c < QK / 4; ++c) {
+            if (c + 1 < QK / 4) load_q((c + 1) & 1, c + 1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float kf = i8_lane(dw[c], e);
+#pragma unroll
+                for (int h = 0; h < NH; ++h) acc[h] += qn[c & 1][h][e] * kf;
+            }
+        }
+        const int t = t0 + lane;
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const float s = acc[h] * kc * scale;
+            sc[h * sp + t] = s;  // past the span: not read
+            mx[h] = t < span && s > mx[h] ? s : mx[h];
+        }
+    }
+    // ---- softmax: exps, one chain a head in position order ----
+#pragma unroll
+    for (int h = 0; h < NH; ++h) mx[h] = ndkv::wave_max(mx[h]);
+    for (int t = lane; t < span; t += 64) {
+        float e[NH];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) e[h] = nd_expf(sc[h * sp + t] - mx[h]);
+#pragma unroll
+        for (int h = 0; h < NH; ++h) sc[h * sp + t] = e[h];
+    }
+    wave_lds_sync();
+    float inv = 0.0f;
+    if (lane < NH) inv = 1.0f / lds_chain(0.0f, sc + lane * sp, span);
+    float ih[NH];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) ih[h] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv), h));
+    // weights (e * inv) * v_scale; zeros to the next multiple of 8 (a zero
+    // product leaves a sum that started at +0 as it is)
+    const int padded = (span + 7) & ~7;
+    for (int t = lane; t < padded; t += 64) {
+        const bool on = t < span;
+        const float vsc = vs[slot_of(on ? t : span - 1)];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const float wgt = sc[h * sp + t] * ih[h] * vsc;
+            sc[h * sp + t] = on ? wgt : 0.0f;
+        }
+    }
+    wave_lds_sync();
+    // ---- values: heads 3 hh .. 3 hh + 2 of the wave's, CW columns a lane ----
+    const int hh = CW == 2 ? lane >> 5 : 0, c0 = CW == 2 ? 2 * (lane & 31) : lane;
+    const float *wr = sc + 3 * hh * sp;
+    float acc[3][CW];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int c = 0; c < CW; ++c) acc[j][c] = 0.0f;
+    uint32_t vr[8];
+    auto load_v = [&](int t0) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int8_t *vp = vb + size_t(slot_of(t0 + u < span ? t0 + u : span - 1)) * VD + c0;
+            if constexpr (CW == 2)
+                vr[u] = *reinterpret_cast<const uint16_t *>(vp);
+            else
+                vr[u] = *reinterpret_cast<const uint8_t *>(vp);
+        }
+    };
+    load_v(0);
+    for (int t0 = 0; t0 < span; t0 += 8) {
+        uint32_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = vr[u];
+        load_v(t0 + 8 < span ? t0 + 8 : t0);
+        float4 w0[3], w1[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            w0[j] = *reinterpret_cast<const float4 *>(wr + j * sp + t0);
+            w1[j] = *reinterpret_cast<const float4 *>(wr + j * sp + t0 + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            float vf[CW];
+#pragma unroll
+            for (int c = 0; c < CW; ++c) vf[c] = i8_lane(v[u], c);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const float4 &wq = u < 4 ? w0[j] : w1[j];
+                const float wv = (u & 3) == 0 ? wq.x : (u & 3) == 1 ? wq.y : (u & 3) == 2 ? wq.z : wq.w;
+#pragma unroll
+                for (int c = 0; c < CW; ++c) acc[j][c] += wv * vf[c];
+            }
+        }
+    }
+    // ---- gate, then the butterfly stages inside each head: with two columns
+    // a lane, stage 1 pairs them and stage 2 h lanes h apart ----
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const size_t oh = orow + size_t(3 * hh + j) * VD + c0;
+        if constexpr (CW == 2) {
+            const float a = acc[j][0] * nd_sigmoidf(gate[oh]), c = acc[j][1] * nd_sigmoidf(gate[oh + 1]);
+            float x0 = a + c, x1 = a - c;
+            x0 = ndl::wave_butterfly<1>(x0), x1 = ndl::wave_butterfly<1>(x1);
+            x0 = ndl::wave_butterfly<2>(x0), x1 = ndl::wave_butterfly<2>(x1);
+            x0 = ndl::wave_butterfly<4>(x0), x1 = ndl::wave_butterfly<4>(x1);
+            x0 = ndl::wave_butterfly<8>(x0), x1 = ndl::wave_butterfly<8>(x1);
+            x0 = ndl::wave_butterfly<16>(x0), x1 = ndl::wave_butterfly<16>(x1);
+            out[oh] = x0;
+            out[oh + 1] = x1;
+        } else {
+            out[oh] = gate_half_fwht(acc[j][0], gate + oh - c0, lane);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Row sums in the reference's order: ((0 + x[0]) + x[1]) + ... per row, one
 // workgroup a row, the row staged in LDS.  Rows of terms >= +0 (sums of
 // squares, softmax sums) take the exact parallel fold of nd_fold.h; any
@@ -684,7 +903,7 @@ int nd_attend_exact_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_
         hipLaunchKernelGGL((attn_exact2_kernel<CW, QC, true>), dim3(unsigned(blocks)),            \
                            dim3(kAttn2Threads), lds, ctx->stream, kg,                             \
                            static_cast<const uint8_t *>(kv), kv_stride, lo, hi, q, scale, 0, out, \
-                           int(groups), rows_per_block, gate);                                    \
+                           int(groups), rows_per_block, gate);                               \
     else                                                                                          \
         hipLaunchKernelGGL((attn_exact2_kernel<CW, QC, false>), dim3(unsigned(blocks)),           \
                            dim3(kAttn2Threads), lds, ctx->stream, kg,                             \
@@ -713,4 +932,42 @@ int nd_attend_exact_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_
                        ndkv::make_geom(g), static_cast<const uint8_t *>(kv), kv_stride,
                        rows_per_block, lo, hi, q, scale, quant_query, out, gate);
     return nd::check_launch("attn_exact");
+}
+
+bool nd_attend_rows_fit(nd_ctx *ctx, const nd_kv_geom *g, size_t count, int max_span)
+{
+    return g->num_heads == kRowHeads * g->num_kv_heads && g->qk_head_dim == kRowQk &&
+           g->v_head_dim == kRowVd && max_span >= 1 && max_span <= kRowSpan &&
+           count * size_t(g->num_kv_heads) >= kRowFill * size_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
+}
+
+int nd_attend_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride, size_t count,
+                   int rows_per_block, const int32_t *lo, const int32_t *hi, const float *q, float scale,
+                   float *out, const float *gate, int max_span)
+{
+    ND_ENTER(ctx);
+    if (int rc = ndkv::check_geom(g)) return rc;
+    ND_REQUIRE(nd_attend_rows_fit(ctx, g, count, max_span),
+               "attend_rows: not the shipped grouping, too few rows, or span %d above %d", max_span,
+               kRowSpan);
+    ND_REQUIRE(kv && lo && hi && q && out && gate, "null buffer");
+    ND_REQUIRE(rows_per_block >= 1 && count % size_t(rows_per_block) == 0, "rows_per_block %d", rows_per_block);
+    const size_t groups = count / size_t(rows_per_block) * size_t(g->num_kv_heads);
+    const size_t blocks = 8 * size_t(rows_per_block) * ((groups + 7) / 8);
+    ND_REQUIRE(blocks <= 0x3fffffffu, "count %zu too large", count);
+    // a head's row: whole runs of 64 scores, and the chain reads 32 floats
+    // past its span; 4 mod 32 floats apart, so the chains' reads fall in
+    // different banks
+    const int sp = (max_span + 63) / 64 * 64 + 36;
+    const ndkv::Geom kg = ndkv::make_geom(g);
+    const uint8_t *kvb = static_cast<const uint8_t *>(kv);
+    if (max_span <= kRowSix)
+        hipLaunchKernelGGL(attn_rows_kernel<6>, dim3(unsigned(blocks)), dim3(64), size_t(6) * sp * 4,
+                           ctx->stream, kg, kvb, kv_stride, lo, hi, q, scale, out, gate, int(groups),
+                           rows_per_block, sp);
+    else
+        hipLaunchKernelGGL(attn_rows_kernel<3>, dim3(unsigned(2 * blocks)), dim3(64), size_t(3) * sp * 4,
+                           ctx->stream, kg, kvb, kv_stride, lo, hi, q, scale, out, gate, int(groups),
+                           rows_per_block, sp);
+    return nd::check_launch("attn_rows");
 }

@@ -898,6 +898,7 @@ struct QkvKv {
     // tails, which this kernel does not change; the normed q goes to q_out.
     int C;
     float *q_out;
+    int fq = 0;  // (prefill, int8) q_out takes the fake-quantised query (quant_rows, model.rs:289-293)
 };
 
 // cache.rs:401-438 for one channel: the conv output, with the tail shifted
@@ -1108,12 +1109,12 @@ __global__ __launch_bounds__(NTH) void k_qkv_kv(QkvKv a, MhcIn mhc)
         const float x2 = (1.0f + rn2[k]) * x[half + i] / r;
         const float c = rc[k], s = rs[k];
         const float o1 = x1 * c - x2 * s, o2 = x2 * c + x1 * s;
-        if (hh < a.H) {
+        if (hh < a.H && !(CHUNK && a.fq)) {
             float *o = (CHUNK ? a.q_out : a.q) + b * a.qd + hh * hd;
             o[i] = o1;
             o[half + i] = o2;
         } else {
-            sq[hh * hd + i] = o1;  // the roped k, reusing the squares' space
+            sq[hh * hd + i] = o1;  // the roped k (and q), reusing the squares' space
             sq[hh * hd + half + i] = o2;
         }
     }
@@ -1133,6 +1134,13 @@ __global__ __launch_bounds__(NTH) void k_qkv_kv(QkvKv a, MhcIn mhc)
         }
         return;
     }
+    if (CHUNK && a.fq)
+        for (int h = wave; h < a.H; h += NTH / 64) {
+            float scale, inv;
+            ndkv::quant_scale_wave(sq + h * hd, hd, scale, inv);
+            for (int e = lane; e < hd; e += 64)
+                a.q_out[b * a.qd + h * hd + e] = ndkv::quant_code(sq[h * hd + e], inv) * scale;
+        }
     for (int vec = wave; vec < 2 * a.KVH; vec += NTH / 64) {
         const bool isv = vec >= a.KVH;
         const int h = isv ? vec - a.KVH : vec;
@@ -2711,6 +2719,7 @@ struct StepRun {
     bool gate_fused = false, gates_in = false, phi_in = false;
     const nd_cq *phi = nullptr, *fpo = nullptr, *fre = nullptr;
     float *ev_conv = nullptr;  // [sites][Rcap][d], after the conv
+    std::vector<int> max_span;  // longest span of any row, per layer
     // tokens == nullptr: this step's tokens are b->next on the device (the
     // previous step's choices); the greedy choices are also written here
     int32_t *argmax_also = nullptr;
@@ -2732,6 +2741,7 @@ int StepRun::begin(const int32_t *tokens)
     B = S * C;
     Rcap = b->R;
     L = c.num_layers;
+    max_span.assign(size_t(L), 0);
     nl = c.mhc_lanes;
     d = c.d_model;
     qd = c.num_heads * c.qk_head_dim;
@@ -2792,7 +2802,9 @@ int StepRun::begin(const int32_t *tokens)
             const int window = is_global(c, li) ? 0 : c.sliding_window;
             int lo = (window && pos + 1 > window) ? pos + 1 - window : 0;
             const int clamp = pos + 1 > slots ? pos + 1 - slots : 0;
-            h_lo[size_t(li) * B + i] = lo > clamp ? lo : clamp;
+            lo = lo > clamp ? lo : clamp;
+            h_lo[size_t(li) * B + i] = lo;
+            if (pos - lo + 1 > max_span[li]) max_span[li] = pos - lo + 1;
         }
     }
     // this step's rows only: the buffer is sized for a full pass of max_chunk
@@ -3029,6 +3041,10 @@ int StepRun::enqueue(int phase, bool argmax)
                  b->kv[li], b->kv_stride[li], nd_kv_v_offset(&g), nd_kv_ks_offset(&g),
                  nd_kv_vs_offset(&g), g.cap, C, b->qn};
         if (kf) qk.v_off = nd_kv_f32_v_offset(&g);
+        // a pass over the int8 ring at the shipped grouping: a wave a (row,
+        // kv head) for all its query heads, which takes the query quantised
+        const bool rows_attn = C > 1 && !kf && gate_fused && nd_attend_rows_fit(ctx, &g, size_t(B), max_span[li]);
+        qk.fq = rows_attn ? 1 : 0;
         // a decode step over the int8 ring with the gated epilogue forms its
         // q, k and v inside the attention launch (k_attn_step)
         const bool step_attn = C == 1 && !kf && gate_fused && c.qk_head_dim % 16 == 0 &&
@@ -3080,6 +3096,13 @@ int StepRun::enqueue(int phase, bool argmax)
             default: hipLaunchKernelGGL((k_attn_step<4>), ag, dim3(ndattn::kAttn2Threads), lds, st, as, mi); break;
             }
             LCHK("k_attn_step");
+            const size_t r0 = 0, nr = size_t(d);
+            CK(nd_cq_exact_set(ctx, st, 1, &l.out, b->attn, size_t(B), &r0, &nr, &b->proj,
+                               "v3 out projection", m->pre_attn.inv));
+        } else if (rows_attn) {
+            CK(nd_attend_rows(ctx, &b->geom[li], b->kv[li], b->kv_stride[li], size_t(B), C,
+                              lo_dev + size_t(li) * B, hi_dev, b->qn, qk_scale, b->attn, b->gate,
+                              max_span[li]));
             const size_t r0 = 0, nr = size_t(d);
             CK(nd_cq_exact_set(ctx, st, 1, &l.out, b->attn, size_t(B), &r0, &nr, &b->proj,
                                "v3 out projection", m->pre_attn.inv));
