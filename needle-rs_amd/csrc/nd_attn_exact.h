@@ -303,19 +303,20 @@ __device__ inline float lds_chain(float acc, const float *v, int n)
 // 1 <= span <= cap); output column c goes to out_row[c], gated and half
 // transformed when gate_row is set.  Every thread of the workgroup calls it.
 // NEW: the span's last position is nr's row (int8 view, QC > 0).
+// score_floats: LDS floats of the scores (a multiple of 4, at least the span).
 // KF: the cache is the f32 view (F32View, attention.rs:166-189): f32 K/V
 // rows at the f32 block's offsets, no scales, weights e * inv.
 template <int CW, int QC, bool KF, bool NEW>
 __device__ __forceinline__ void attn_exact2_run(const ndkv::Geom &g, const uint8_t *blk, int kvh,
                                                 int p0, int span, float scale, float *sm,
                                                 AttnLds &L, const AttnNewRow *nr, float *out_row,
-                                                const float *gate_row)
+                                                const float *gate_row, int score_floats)
 {
     static_assert(!NEW || !KF, "the launch's own row is int8");
     constexpr int NT = kAttn2Threads;
     const int tid = threadIdx.x;
     float *sc = sm;                         // [span] scores, then exps
-    float *prod = sm + ((g.cap + 3) & ~3);  // [2][kProdBuf] products
+    float *prod = sm + score_floats;        // [2][kProdBuf] products
     const int base = p0 % g.cap;
     float mx;
     if constexpr (KF) {

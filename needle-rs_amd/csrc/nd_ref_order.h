@@ -32,11 +32,12 @@ int nd_cq_exact_multi(nd_ctx *ctx, hipStream_t stream, int n, const nd_cq *const
 // of its 128-wide group applied: the input nd_cq_exact_set finishes with
 // half_inv (v3/model.rs:309-313, hadamard.rs:24-55).  kv_f32: the blocks
 // are f32 KV blocks (nd_kv_f32_block_bytes) read through the f32 view, as
-// nd_attend_step_f32_exact.
+// nd_attend_step_f32_exact.  max_span: the longest span of the rows where the
+// caller knows it (0: the ring's); a row beyond it is NaN.
 int nd_attend_exact_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride,
                          size_t count, int rows_per_block, const int32_t *lo, const int32_t *hi,
                          const float *q, float scale, int quant_query, float *out,
-                         const float *gate = nullptr, int kv_f32 = 0);
+                         const float *gate = nullptr, int kv_f32 = 0, int max_span = 0);
 
 // A prefill pass's attention at the shipped grouping (six query heads a kv
 // head, qk 48, v 64, int8): bit for bit nd_attend_exact_rows with

@@ -545,7 +545,8 @@ template <int CW, int QC, bool KF>
 __global__ __launch_bounds__(kAttn2Threads, 4) void attn_exact2_kernel(
     ndkv::Geom g, const uint8_t *__restrict__ kv, size_t stride, const int32_t *__restrict__ lo,
     const int32_t *__restrict__ hi, const float *__restrict__ q, float scale, int quant_query,
-    float *__restrict__ out, int groups, int rows_per_block, const float *__restrict__ gate)
+    float *__restrict__ out, int groups, int rows_per_block, const float *__restrict__ gate,
+    int score_floats)
 {
     extern __shared__ __align__(16) float sm[];
     __shared__ AttnLds L;
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(kAttn2Threads, 4) void attn_exact2_kernel(
     const int p0 = lo[i];
     const int span = hi[i] - p0 + 1;
     float *orow = out + (size_t(i) * g.H + h) * g.VD;
-    if (p0 < 0 || span < 1 || span > g.cap) {
+    if (p0 < 0 || span < 1 || span > g.cap || span > score_floats) {
         for (int j = tid; j < g.VD; j += kAttn2Threads) orow[j] = NAN;
         return;
     }
@@ -576,7 +577,8 @@ __global__ __launch_bounds__(kAttn2Threads, 4) void attn_exact2_kernel(
     }
     __syncthreads();
     attn_exact2_run<CW, QC, KF, false>(g, blk, kvh, p0, span, scale, sm, L, nullptr, orow,
-                                       gate ? gate + (size_t(i) * g.H + h) * g.VD : nullptr);
+                                       gate ? gate + (size_t(i) * g.H + h) * g.VD : nullptr,
+                                       score_floats);
 }
 
 // ---------------------------------------------------------------------------
@@ -870,7 +872,7 @@ int nd_attend_step_f32_exact(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, s
 int nd_attend_exact_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride,
                          size_t count, int rows_per_block, const int32_t *lo, const int32_t *hi,
                          const float *q, float scale, int quant_query, float *out,
-                         const float *gate, int kv_f32)
+                         const float *gate, int kv_f32, int max_span)
 {
     ND_ENTER(ctx);
     ND_REQUIRE(rows_per_block >= 1, "rows_per_block %d", rows_per_block);
@@ -893,7 +895,10 @@ int nd_attend_exact_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_
         const size_t groups = count * size_t(g->num_kv_heads);
         const size_t blocks = 8 * size_t(R) * ((groups + 7) / 8);
         ND_REQUIRE(blocks <= 0x7fffffffu, "count %zu too large", count);
-        const size_t lds = size_t((g->cap + 3) & ~3) * 4 + 2 * kProdBuf * sizeof(float);
+        // scores of the longest span the caller knows of, else of the ring
+        const int most = max_span > 0 && max_span < g->cap ? max_span : g->cap;
+        const int score_floats = (most + 3) & ~3;
+        const size_t lds = size_t(score_floats) * 4 + 2 * kProdBuf * sizeof(float);
         const int cw = g->v_head_dim <= 64 ? 1 : 2;
         const int qc = g->qk_head_dim <= 64 ? g->qk_head_dim / 16 : 0;
         ndkv::Geom kg = ndkv::make_geom(g);
@@ -903,12 +908,12 @@ int nd_attend_exact_rows(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_
         hipLaunchKernelGGL((attn_exact2_kernel<CW, QC, true>), dim3(unsigned(blocks)),            \
                            dim3(kAttn2Threads), lds, ctx->stream, kg,                             \
                            static_cast<const uint8_t *>(kv), kv_stride, lo, hi, q, scale, 0, out, \
-                           int(groups), rows_per_block, gate);                               \
+                           int(groups), rows_per_block, gate, score_floats);                 \
     else                                                                                          \
         hipLaunchKernelGGL((attn_exact2_kernel<CW, QC, false>), dim3(unsigned(blocks)),           \
                            dim3(kAttn2Threads), lds, ctx->stream, kg,                             \
                            static_cast<const uint8_t *>(kv), kv_stride, lo, hi, q, scale,         \
-                           quant_query, out, int(groups), rows_per_block, gate)
+                           quant_query, out, int(groups), rows_per_block, gate, score_floats)
 #define ND_ATTN2_QC(CW)                    \
     switch (qc) {                          \
     case 1: ND_ATTN2(CW, 1); break;        \

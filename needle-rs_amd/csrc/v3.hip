@@ -1175,6 +1175,7 @@ struct AttnStep {
     const float *gate;   // [B][H * 64]
     int groups;          // B * KVH
     int attn_blocks;     // 8 * R * ceil(groups / 8)
+    int score_floats;    // LDS floats of a workgroup's scores
 };
 
 template <int QC>
@@ -1283,12 +1284,12 @@ __global__ __launch_bounds__(ndattn::kAttn2Threads, 4) void k_attn_step(AttnStep
     const int span = hi - p0 + 1;
     float *orow = s.out + (size_t(i) * g.H + h) * g.VD;
     // the span must end at the step's own position
-    if (p0 < 0 || span < 1 || span > g.cap || hi != p) {
+    if (p0 < 0 || span < 1 || span > g.cap || span > s.score_floats || hi != p) {
         for (int j = tid; j < g.VD; j += kAttn2Threads) orow[j] = NAN;
         return;
     }
     attn_exact2_run<1, QC, false, true>(g, blk, kvh, p0, span, s.scale, sm, L, &nr, orow,
-                                        s.gate + (size_t(i) * g.H + h) * g.VD);
+                                        s.gate + (size_t(i) * g.H + h) * g.VD, s.score_floats);
 }
 
 // attn *= sigmoid(gate) (model.rs:309-312), then prepare_input for out_proj.
@@ -3041,6 +3042,12 @@ int StepRun::enqueue(int phase, bool argmax)
                  b->kv[li], b->kv_stride[li], nd_kv_v_offset(&g), nd_kv_ks_offset(&g),
                  nd_kv_vs_offset(&g), g.cap, C, b->qn};
         if (kf) qk.v_off = nd_kv_f32_v_offset(&g);
+        // LDS for the scores of this step's longest span, not of the ring: a
+        // global layer of 8192 slots held a CU to four workgroups (64 sessions'
+        // step at 512 positions 1.66 -> 1.62 ms, at 2048 1.95 -> 1.88; one
+        // session's prompt passes of 256 rows 64.0 -> 60.8 ms up to 4096).  A
+        // captured step is replayed at later positions and keeps the ring's.
+        const int spans = b->graphs ? g.cap : max_span[li];
         // a pass over the int8 ring at the shipped grouping: a wave a (row,
         // kv head) for all its query heads, which takes the query quantised
         const bool rows_attn = C > 1 && !kf && gate_fused && nd_attend_rows_fit(ctx, &g, size_t(B), max_span[li]);
@@ -3085,9 +3092,10 @@ int StepRun::enqueue(int phase, bool argmax)
             const int R = c.num_heads / c.num_kv_heads;
             const size_t groups = size_t(B) * c.num_kv_heads;
             const size_t ablocks = 8 * size_t(R) * ((groups + 7) / 8);
-            const size_t lds = size_t((g.cap + 3) & ~3) * 4 + 2 * ndattn::kProdBuf * sizeof(float);
+            const int score_floats = (spans + 3) & ~3;
+            const size_t lds = size_t(score_floats) * 4 + 2 * ndattn::kProdBuf * sizeof(float);
             AttnStep as{qk, ndkv::make_geom(&g), lo_dev + size_t(li) * B, hi_dev, qk_scale,
-                        b->attn, b->gate, int(groups), int(ablocks)};
+                        b->attn, b->gate, int(groups), int(ablocks), score_floats};
             const dim3 ag(unsigned(ablocks + (gates_in ? size_t(B) : 0)));
             switch (c.qk_head_dim / 16) {
             case 1: hipLaunchKernelGGL((k_attn_step<1>), ag, dim3(ndattn::kAttn2Threads), lds, st, as, mi); break;
@@ -3109,14 +3117,14 @@ int StepRun::enqueue(int phase, bool argmax)
         } else if (gate_fused) {
             CK(nd_attend_exact_rows(ctx, &b->geom[li], b->kv[li], b->kv_stride[li], size_t(B), C,
                                     lo_dev + size_t(li) * B, hi_dev, C == 1 ? b->q : b->qn,
-                                    qk_scale, kf ? 0 : 1, b->attn, b->gate, kf));
+                                    qk_scale, kf ? 0 : 1, b->attn, b->gate, kf, spans));
             const size_t r0 = 0, nr = size_t(d);
             CK(nd_cq_exact_set(ctx, st, 1, &l.out, b->attn, size_t(B), &r0, &nr, &b->proj,
                                "v3 out projection", m->pre_attn.inv));
         } else {
             CK(nd_attend_exact_rows(ctx, &b->geom[li], b->kv[li], b->kv_stride[li], size_t(B), C,
                                     lo_dev + size_t(li) * B, hi_dev, C == 1 ? b->q : b->qn,
-                                    qk_scale, kf ? 0 : 1, b->attn, nullptr, kf));
+                                    qk_scale, kf ? 0 : 1, b->attn, nullptr, kf, spans));
             hipLaunchKernelGGL(k_gate_prep, dim3(B), dim3(kT), 0, st, b->attn, b->gate, b->ah, od,
                                m->pre_attn);
             LCHK("k_gate_prep");

@@ -20,14 +20,14 @@ def _bits(a):
 
 @pytest.fixture(scope="module")
 def small(ctx):
-    g, recs = S.build_records(S.small_geometry(4), seed=33)
+    g, recs = S.build_records({**S.small_geometry(4), "max_seq_len": 4096}, seed=33)
     return nd.V3Model(ctx, g, recs, S.CODEBOOK)
 
 
 @pytest.mark.parametrize("kv_int8", [True, False])
 @pytest.mark.parametrize("sessions,passes", [
     (1, [1, 5]), (16, [16]), (1, [256, 3]), (3, [86, 2]), (2, [255, 1, 40]), (4, [129]), (7, [101, 7]),
-    (5, [205, 30]), (13, [79, 33])])
+    (5, [205, 30]), (13, [79, 33]), (8, [64] * 35)])
 def test_pass_equals_stepping(small, sessions, passes, kv_int8):
     n = sum(passes)
     prompts = np.stack([S.prompt_tokens(n, 90 + i) for i in range(sessions)]).astype(np.int32)
