@@ -14,7 +14,7 @@
 //     not conflict on banks;
 //   * code loads split in two halves so the second half is in flight while
 //     the first computes; nontemporal loads, since codes are read once.
-// Other widths fall back to a kernel with the activations in LDS.
+// Other widths take a kernel with the activations in LDS and part steps.
 // GEMM (prefill) converts X to bf16 once, dequantises weight tiles to bf16 in
 // LDS through the bf16-rounded codebook and feeds v_mfma_f32_16x16x32_bf16
 // with fp32 accumulation: 64x64 tiles below M = 96, 128x128 tiles, and
@@ -31,8 +31,6 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kTileRows = 64;      // rows sharing one codebook
 constexpr int kThreads = 256;      // 4 waves
-constexpr int kLanesPerRow = 16;
-constexpr int kRowsPerPass = kThreads / kLanesPerRow;  // 16
 
 // Fast path, in = 256*M (M = 1..4; config 1's 768 is M = 3).  One 256-thread
 // block owns one 64-row tile.  32 lanes share a row: lane j reads M/2
@@ -168,62 +166,108 @@ __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_kernel(
     if ((j & 3) == 0 && r < out) y[r] = s;
 }
 
-// Any `in` (multiple of 16): activations staged in LDS instead of registers.
-template <int REP>
-__global__ __launch_bounds__(kThreads) void cb8_gemv_generic_kernel(
+// Any `in` (multiple of 16).  Eight lanes share a row (128 contiguous bytes a
+// load; a wave's 16 rows take P = 2 passes), a step is U = 4 vectors of 16
+// codes a lane and row: eight loads of 16 bytes in flight, and the next step's
+// are issued before the current one's gathers.  The part step at a row's end
+// goes first, its loads together with the first full step's: a vector past the
+// end is read as the last one and left out of the sum.  The activations sit in
+// LDS, the quads of a vector rotated by its index so that the lanes' reads of
+// one quad fall on different banks; eight lanes a row read each once for two
+// rows.
+// Bound by HBM on stacks of wide rows, by filling the table for a tile on
+// narrow ones.  Measured, MI355X, stacks of 300 MB, codes' GB/s (before: one
+// load in flight a lane; 16 lanes a row): in = 64: 2289 (1122), 128: 3960
+// (1671), 272: 3997 (1704), 528: 4989 (1869), 1040: 5000 (1922), 2048: 6087
+// (1996), 4096: 5509 (1750).  Four lanes a row gain on 64 (2753) and lose
+// elsewhere (4124 at 1040); 16 gain on 208 to 400 (12 % at most) and lose
+// elsewhere (3701 at 4096).
+__global__ __launch_bounds__(kThreads, 4) void cb8_gemv_any_kernel(
     const uint8_t *__restrict__ w, size_t w_stride, const float *__restrict__ cb,
     size_t cb_stride, const float *__restrict__ x, size_t x_stride, float *__restrict__ y,
     size_t y_stride, int out, int in)
 {
-    __shared__ float4 rep4[256 * REP / 4];
-    __shared__ float stage[256];
-    extern __shared__ float xs[];
-    float *rep = reinterpret_cast<float *>(rep4);
-    const int tile = blockIdx.x;
+    constexpr int L = 8, P = 2, U = 4, R = 64 / L;
+    __shared__ float4 rep4[256 * 32 / 4];  // 32 KB
+    extern __shared__ float4 xs4[];        // [in / 4]
     const size_t prob = blockIdx.y;
     w += prob * w_stride;
-    cb += prob * cb_stride + size_t(tile) * 256;
+    cb += prob * cb_stride + size_t(blockIdx.x) * 256;
     x += prob * x_stride;
     y += prob * y_stride;
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int j = t & (kLanesPerRow - 1);
-    const int rg = t / kLanesPerRow;
+    const int t = threadIdx.x, lane = t & 63, j = lane & (L - 1);
+    const int row0 = blockIdx.x * kTileRows + (t >> 6) * 16 + lane / L;
     const int nvec = in >> 4;
-    stage[t] = cb[t];
-    for (int k = t; k < in; k += kThreads) xs[k] = x[k];
-    __syncthreads();
-    for (int i = 0; i < REP / 4; ++i) {
-        const int f4 = i * kThreads + t;
-        const float v = stage[(f4 * 4) / REP];
-        rep4[f4] = make_float4(v, v, v, v);
-    }
-    __syncthreads();
-    const float *cbl = rep + (lane & (REP - 1));
-    const int row0 = tile * kTileRows;
-    for (int p = 0; p < kTileRows / kRowsPerPass; ++p) {
-        const int r = row0 + rg + kRowsPerPass * p;
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (r < out) {
-            const uint4 *wr = reinterpret_cast<const uint4 *>(w + size_t(r) * in);
-            for (int c = j; c < nvec; c += kLanesPerRow) {
-                const uint4 cv = wr[c];
-                const uint32_t dw[4] = {cv.x, cv.y, cv.z, cv.w};
+
+    const u32x4_t *wr[P];
 #pragma unroll
-                for (int d = 0; d < 4; ++d)
+    for (int p = 0; p < P; ++p)
+        wr[p] = reinterpret_cast<const u32x4_t *>(w + size_t(min(row0 + R * p, out - 1)) * in);
+    constexpr int kStep = U * L;
+    const int tail = nvec / kStep * kStep;  // first vector of the part step
+    u32x4_t cur[P][U], nxt[P][U];
+    auto fetch = [&](u32x4_t (&c)[P][U], int v0) {
 #pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        const uint32_t e = (dw[d] >> (8 * b)) & 0xffu;
-                        acc[b] += cbl[e * REP] * xs[c * 16 + 4 * d + b];
-                    }
-            }
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int p = 0; p < P; ++p) c[p][u] = __builtin_nontemporal_load(wr[p] + v0 + u * L + j);
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (tail + u * L < nvec) {
+            const int v = min(tail + u * L + j, nvec - 1);
+#pragma unroll
+            for (int p = 0; p < P; ++p) nxt[p][u] = __builtin_nontemporal_load(wr[p] + v);
         }
-        float s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        s += ndl::wave_xor<8>(s);
+    if (tail > 0) fetch(cur, 0);
+    // float4 slot f4 = i*256 + t of the replica array holds entry f4 / 8.
+    float cbv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) cbv[i] = cb[(i * kThreads + t) >> 3];
+    for (int f = t; f < in >> 2; f += kThreads) {
+        const int v = f >> 2;
+        xs4[4 * v + ((f ^ (v >> 2)) & 3)] = reinterpret_cast<const float4 *>(x)[f];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) rep4[i * kThreads + t] = make_float4(cbv[i], cbv[i], cbv[i], cbv[i]);
+    __syncthreads();
+
+    const float *cbl = reinterpret_cast<const float *>(rep4) + (lane & 31);
+    float acc[P][8] = {};  // 64 partial sums a row
+    auto block = [&](const u32x4_t (&c)[P][U], int u, int v) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const float4 xq = xs4[4 * v + ((d ^ (v >> 2)) & 3)];
+            const float xv[4] = {xq.x, xq.y, xq.z, xq.w};
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    acc[p][4 * (d & 1) + b] += cbl[((c[p][u][d] >> (8 * b)) & 0xffu) * 32] * xv[b];
+        }
+    };
+    auto step = [&](const u32x4_t (&c)[P][U], int v0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) block(c, u, v0 + u * L + j);
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (tail + u * L < nvec && tail + u * L + j < nvec) block(nxt, u, tail + u * L + j);
+    for (int v0 = 0; v0 < tail; v0 += 2 * kStep) {
+        if (v0 + kStep < tail) fetch(nxt, v0 + kStep);
+        step(cur, v0);
+        if (v0 + kStep >= tail) break;
+        if (v0 + 2 * kStep < tail) fetch(cur, v0 + 2 * kStep);
+        step(nxt, v0 + kStep);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        float s = ((acc[p][0] + acc[p][1]) + (acc[p][2] + acc[p][3])) +
+                  ((acc[p][4] + acc[p][5]) + (acc[p][6] + acc[p][7]));
         s += ndl::wave_xor<4>(s);
         s += ndl::wave_xor<2>(s);
         s += ndl::wave_xor<1>(s);
-        if (j == 0 && r < out) y[r] = s;
+        if (j == 0 && row0 + R * p < out) y[row0 + R * p] = s;
     }
 }
 
@@ -845,8 +889,6 @@ __global__ __launch_bounds__(256, 2) void cb8_gemm_m64_kernel(const unsigned sho
             }
 }
 
-constexpr int kRep = 32;
-
 int launch_gemv(nd_ctx *ctx, size_t count, const uint8_t *w, size_t w_stride, const float *cb,
                 size_t cb_stride, const float *x, size_t x_stride, float *y, size_t y_stride,
                 size_t out, size_t in)
@@ -876,9 +918,8 @@ int launch_gemv(nd_ctx *ctx, size_t count, const uint8_t *w, size_t w_stride, co
         }
     } else {
         ND_REQUIRE(in * sizeof(float) <= 64 * 1024, "in (%zu) too large", in);
-        hipLaunchKernelGGL((cb8_gemv_generic_kernel<kRep>), grid, dim3(kThreads),
-                           in * sizeof(float), ctx->stream, w, w_stride, cb, cb_stride, x,
-                           x_stride, y, y_stride, int(out), int(in));
+        hipLaunchKernelGGL(cb8_gemv_any_kernel, grid, dim3(kThreads), in * sizeof(float), ctx->stream, w,
+                           w_stride, cb, cb_stride, x, x_stride, y, y_stride, int(out), int(in));
     }
 #undef ND_GEMV
     return nd::check_launch("cb8_gemv");

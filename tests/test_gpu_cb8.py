@@ -40,6 +40,33 @@ def test_gemv_ragged(ctx, out, inn):
     assert np.max(np.abs(y - O.cb8_gemv(w, cb, x))) <= 1e-4
 
 
+@pytest.mark.parametrize("count,out,inn", [(3, 1, 16), (2, 64, 112), (5, 65, 128), (2, 81, 496),
+                                           (1, 130, 512), (2, 17, 528), (1, 100, 1008), (1, 64, 1536),
+                                           (2, 33, 2064), (1, 3, 16384)])
+def test_gemv_part_steps(ctx, count, out, inn):
+    """Widths around the steps of 512 columns and their parts of 128, ragged
+    rows, padded strides; within inn rounding errors of the sum's magnitude
+    of the 64-bit result, and an infinite entry of an unused code stays out."""
+    rng = np.random.default_rng(out + inn)
+    tiles = (out + 63) // 64
+    W = rng.integers(0, 255, size=(count, out * inn + 48), dtype=np.uint8)
+    CB = rng.normal(0, 0.02, size=(count, tiles, 256)).astype(np.float32)
+    CB[:, :, 255] = np.inf
+    X = rng.normal(size=(count, inn + 8)).astype(np.float32)
+    w, cb, x = dev(W), dev(CB), dev(X)
+    y = torch.full((count, out + 5), 7.0, device="cuda")
+    nd._check(nd.lib().nd_cb8_gemv_batched(
+        ctx.h, count, w.data_ptr(), W.shape[1], cb.data_ptr(), tiles * 256, x.data_ptr(), inn + 8,
+        y.data_ptr(), out + 5, out, inn))
+    Y = host(y)
+    for i in range(count):
+        v = CB[i].astype(np.float64)[np.arange(out)[:, None] // 64, W[i, :out * inn].reshape(out, inn)]
+        xi = X[i, :inn].astype(np.float64)
+        bound = (np.abs(v) @ np.abs(xi)) * inn * 2.0 ** -24
+        assert np.all(np.abs(Y[i, :out] - v @ xi) <= bound)
+    assert np.all(Y[:, out:] == 7.0)
+
+
 def test_gemv_extreme_codes(ctx):
     """All-0 and all-255 codes pick the first and last codebook entries."""
     out, inn = 128, 768
