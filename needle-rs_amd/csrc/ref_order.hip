@@ -19,9 +19,11 @@
 //                  LUT (one LDS read per byte) and dotted with up to 8
 //                  activation rows held in LDS; the group sums meet in LDS
 //                  and one thread per (row, batch row) chains them.
-//   cq_exact_serial   any other width or group: one thread per output, the
-//                  reference's loop verbatim (3-bit bit reader, 8-lane
-//                  groups with a serial tail).
+//                  3-bit weights of groups of 32 take it too (cq.rs:914-925,
+//                  one chain a group): codes decoded in pairs.
+//   cq_exact_serial   any other group: one thread per output, the reference's
+//                  loop verbatim (3-bit bit reader, 8-lane groups with a
+//                  serial tail).
 //   attn_exact     attend_step over the int8 view (attention.rs:327-377):
 //                  per (query, head) a workgroup computes every score with
 //                  its own 16..256-long dot chain, the maximum, exp, the
@@ -45,6 +47,9 @@ constexpr size_t kLdsBudget = 64 * 1024;
 constexpr int kVChunk = 16384;        // bytes of V rows staged per pass
 constexpr int kAttnMaxCap = 12288;    // one span's scores + a V chunk fit 64 KB of LDS
 constexpr uint8_t kTernary = 5;
+
+// LDS floats of the decode table: a byte's levels, or a 3-bit pair's
+__host__ __device__ constexpr int lut_floats(int per_byte) { return per_byte ? 256 * per_byte : 128; }
 
 struct CqExact {
     const uint8_t *packed;
@@ -72,8 +77,14 @@ struct CqExactSet {
 // cq.rs:948-958
 __device__ inline int ternary_index(int code) { return code == 3 ? 0 : (code == 1 ? 2 : 1); }
 
-// GR: the group size when it is 128 (codes preloaded into registers), or 0
-// for any other multiple of 8 (codes read as the loop needs them).
+// P: codes a byte, or 0 for 3-bit codes.  GR: the group size when it is 128
+// (codes preloaded into registers), or 0 for any other multiple of 8 (3-bit: of
+// 32; codes read as the loop needs them).
+// A 3-bit group is one chain of products; BT of them run side by side, bound by
+// the VALU (two operations a product) and for one row by the chain's latency.
+// Measured, MI355X, against a thread an output reading the codes bit by bit:
+// 1 row by 768 x 768 208 -> 15 us (a call's host time), 64 rows 218 -> 15, 117
+// by 1727 x 768 574 -> 25, 478 by 5131 x 768 7747 -> 165.
 template <int P, int BT, int GR>
 __global__ __launch_bounds__(kThreads) void cq_exact_kernel(CqExactSet set)
 {
@@ -81,16 +92,16 @@ __global__ __launch_bounds__(kThreads) void cq_exact_kernel(CqExactSet set)
     while (wk > 0 && int(blockIdx.x) < set.tile0[wk]) --wk;
     const CqExact &a = set.w[wk];
     const int tile = int(blockIdx.x) - set.tile0[wk];
-    constexpr int W = 8 / P;                // bits per code
+    constexpr int W = P ? 8 / (P ? P : 1) : 3;  // bits per code
     constexpr uint32_t MASK = (1u << W) - 1;
-    constexpr int PER_DW = 32 / W;          // codes per dword (8 or 16)
-    constexpr int NDW = GR ? GR / PER_DW : 1;
+    constexpr int PER_DW = 32 / W;          // codes per dword (8 or 16), P > 0
+    constexpr int NDW = GR ? GR * W / 32 : 1;
     extern __shared__ __align__(16) float sm[];
     // activations in LDS with each group padded by 4 floats, so that the
     // groups a wave reads at once fall in different banks
     const int gstride = a.group + 4, xstride = a.G * gstride;
-    float *lut = sm;                        // [256][P] byte -> its P levels (build_lut)
-    float *ns = sm + 256 * P;               // [kThreads] this block's norms
+    float *lut = sm;                        // [256][P] byte -> its P levels (build_lut); [64][2]
+    float *ns = sm + lut_floats(P);         // [kThreads] this block's norms
     float *xs = ns + kThreads;              // [BT][G][group + 4]
     float *gs = xs + BT * xstride;          // [BT][rpb * G] group sums
     const int tid = threadIdx.x;
@@ -107,6 +118,8 @@ __global__ __launch_bounds__(kThreads) void cq_exact_kernel(CqExactSet set)
         const int c = int((uint32_t(tid) >> (k * W)) & MASK);
         lut[tid * P + k] = a.lv[a.ternary ? ternary_index(c) : c];
     }
+    // 3 bits: the levels of a pair of codes
+    if (P == 0 && tid < 128) lut[tid] = a.lv[(tid & 1) ? tid >> 4 : (tid >> 1) & 7];
     if (tid < nrows * a.G) ns[tid] = a.norms[size_t(r0) * a.G + tid];
     for (int bb = 0; bb < nb; ++bb) {
         const float4 *src = reinterpret_cast<const float4 *>(a.xh + size_t(b0 + bb) * a.in_padded);
@@ -128,7 +141,7 @@ __global__ __launch_bounds__(kThreads) void cq_exact_kernel(CqExactSet set)
     const int r = r0 + rl;
     const bool active = tid < pairs && rl < nrows;
     const uint32_t *cw = reinterpret_cast<const uint32_t *>(
-        a.packed + size_t(active ? r : a.row_start) * a.row_bytes + size_t(g) * (a.group / P));
+        a.packed + size_t(active ? r : a.row_start) * a.row_bytes + size_t(g) * (a.group * W / 8));
     uint32_t code[NDW];
     if (GR && active) {
 #pragma unroll
@@ -148,6 +161,35 @@ __global__ __launch_bounds__(kThreads) void cq_exact_kernel(CqExactSet set)
 #pragma unroll
             for (int k = 0; k < 8; ++k) lanes[bb][k] = 0.0f;
         const float *xg = xs + g * gstride;
+        // 32 codes in three dwords, 16 pairs; one chain in lanes[bb][0]
+        auto step3 = [&](int i, uint32_t d0, uint32_t d1, uint32_t d2) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                float v[4];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int bit = 6 * (2 * q + h);
+                    const uint32_t f = bit == 30   ? (d0 >> 30) | (d1 << 2)
+                                       : bit == 60 ? (d1 >> 28) | (d2 << 4)
+                                       : bit < 30  ? d0 >> (bit & 31)
+                                       : bit < 60  ? d1 >> (bit & 31)
+                                                   : d2 >> (bit & 31);
+                    const float2 l2 = *reinterpret_cast<const float2 *>(lut + (f & 63u) * 2);
+                    v[2 * h] = l2.x;
+                    v[2 * h + 1] = l2.y;
+                }
+#pragma unroll
+                for (int bb = 0; bb < BT; ++bb) {
+                    if (bb < nb) {
+                        const float4 xa = *reinterpret_cast<const float4 *>(xg + bb * xstride + i * 32 + q * 4);
+                        lanes[bb][0] += v[0] * xa.x;
+                        lanes[bb][0] += v[1] * xa.y;
+                        lanes[bb][0] += v[2] * xa.z;
+                        lanes[bb][0] += v[3] * xa.w;
+                    }
+                }
+            }
+        };
         // iteration i: elements 8i..8i+7 of the group, element 8i+k into lane k
         auto step = [&](int i, uint32_t dw) {
             const int sh = (i * 8 * W) & 31;
@@ -185,7 +227,14 @@ __global__ __launch_bounds__(kThreads) void cq_exact_kernel(CqExactSet set)
                 }
             }
         };
-        if constexpr (GR != 0) {
+        if constexpr (P == 0) {
+            if constexpr (GR != 0) {
+#pragma unroll
+                for (int i = 0; i < GR / 32; ++i) step3(i, code[3 * i], code[3 * i + 1], code[3 * i + 2]);
+            } else {
+                for (int i = 0; i < a.group / 32; ++i) step3(i, cw[3 * i], cw[3 * i + 1], cw[3 * i + 2]);
+            }
+        } else if constexpr (GR != 0) {
 #pragma unroll
             for (int i = 0; i < GR / 8; ++i) step(i, code[(i * 8) / PER_DW]);
         } else {
@@ -196,6 +245,7 @@ __global__ __launch_bounds__(kThreads) void cq_exact_kernel(CqExactSet set)
             float acc = 0.0f;
 #pragma unroll
             for (int k = 0; k < 8; ++k) acc += lanes[bb][k];
+            if (P == 0) acc = lanes[bb][0];
             if (bb < nb) gs[bb * pairs + tid] = acc;
         }
     }
@@ -274,7 +324,7 @@ __global__ __launch_bounds__(kThreads) void cq_exact_serial_kernel(CqSerial a)
 size_t exact_lds(int bt, int per_byte, size_t in_padded, size_t group, size_t pairs)
 {
     const size_t padded = in_padded / group * (group + 4);
-    return 4 * (256 * size_t(per_byte) + size_t(kThreads) + size_t(bt) * padded + size_t(bt) * pairs);
+    return 4 * (size_t(lut_floats(per_byte)) + size_t(kThreads) + size_t(bt) * padded + size_t(bt) * pairs);
 }
 
 template <int P, int BT>
@@ -352,8 +402,9 @@ int nd_cq_exact_multi(nd_ctx *ctx, hipStream_t stream, int n, const nd_cq *const
     ND_REQUIRE(batch <= 65535u * kMaxBt, "%s: batch too large", what);
     const size_t G = w0->num_groups;
     const int P = int(w0->per_byte);
-    const bool fast = same && (P == 2 || P == 4) && w0->group % 8 == 0 && (w0->group / P) % 4 == 0 &&
-                      G <= kThreads && w0->row_bytes % 4 == 0 && aligned;
+    const bool fast = same && G <= kThreads && w0->row_bytes % 4 == 0 && aligned &&
+                      (P ? (P == 2 || P == 4) && w0->group % 8 == 0 && (w0->group / P) % 4 == 0
+                         : w0->bits == 3 && w0->group % 32 == 0 && half_inv == 0.0f);
     if (fast) {
         const int rpb = int(kThreads / G);
         const size_t pairs = size_t(rpb) * G;
@@ -386,6 +437,8 @@ int nd_cq_exact_multi(nd_ctx *ctx, hipStream_t stream, int n, const nd_cq *const
             set.tile0[set.n] = tiles;
             if (P == 4)
                 launch_bt<4>(set, bt, stream);
+            else if (P == 0)
+                launch_bt<0>(set, bt, stream);
             else
                 launch_bt<2>(set, bt, stream);
             return nd::check_launch(what);

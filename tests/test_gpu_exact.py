@@ -65,6 +65,25 @@ def test_cq_exact_bits(ctx, shape, batch):
         assert _same_bits(got, o.matvec_rows_prepared(xh[0], r0, rows))
 
 
+@pytest.mark.parametrize("out,inn,group,r0,rows", [
+    (1, 128, 128, 0, 1), (300, 768, 128, 7, 290), (257, 2400, 128, 0, 257), (70, 96, 32, 0, 70),
+    (129, 500, 64, 3, 120), (20, 512, 256, 0, 20), (9, 3072, 32, 0, 9), (40, 96, 16, 0, 40)])
+@pytest.mark.parametrize("batch", [1, 2, 5, 77, 1030])
+def test_cq_exact_three_bits(ctx, out, inn, group, r0, rows, batch):
+    """3-bit weights: groups that are multiples of 32, every number of
+    activation rows a workgroup takes, ragged ends; groups of 16 keep the
+    thread an output."""
+    rng = np.random.default_rng(out + inn + batch)
+    c = random_case(rng, out, inn, group, 3, REAL_CB)
+    g = nd.CqWeight(ctx, c.blob, out, inn, group, 3, REAL_CB)
+    o = O.CqWeight(c.blob, out, inn, group, 3, REAL_CB)
+    x = rng.normal(size=(batch, inn)).astype(np.float32)
+    x[:, ::7] *= 30.0
+    xh = o.prepare_batch(x)
+    got = host(g.matmul_rows_prepared(dev(xh), batch, r0, rows, exact=True))
+    assert _same_bits(got, o.matmul_rows_prepared(xh, batch, r0, rows))
+
+
 def test_cq_exact_rejects_bad_band(ctx):
     rng = np.random.default_rng(0)
     c = random_case(rng, 16, 128, 128, 2, REAL_CB)
