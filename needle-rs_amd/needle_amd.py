@@ -156,22 +156,34 @@ def _arg(t, dtype, name, numel=0, rows=False):
         raise ValueError(f"{name}: a device tensor is required")
     if t.dtype != dtype:
         raise ValueError(f"{name}: dtype {t.dtype}, expected {dtype}")
-    ok = (t.dim() == 0 or all(t[i].is_contiguous() for i in range(min(t.shape[0], 1)))) \
-        if rows else t.is_contiguous()
-    if rows and t.dim() > 1:
-        ok = ok and t.stride(0) >= t[0].numel()
-    if not ok:
-        raise ValueError(f"{name}: layout {tuple(t.shape)} strides {t.stride()} is not contiguous")
-    if t.numel() < numel:
+    # A contiguous tensor of two slices or more has contiguous slices that do
+    # not overlap (one slice: by its stride); a slice itself (1 us to form) is
+    # looked at only where that does not settle it.
+    if not (t.is_contiguous() and (not rows or t.dim() < 2 or t.size(0) > 1 or
+                                   (t.size(0) == 1 and t.stride(0) >= t.numel()))):
+        ok = (t.dim() == 0 or all(t[i].is_contiguous() for i in range(min(t.shape[0], 1)))) \
+            if rows else t.is_contiguous()
+        if rows and t.dim() > 1:
+            ok = ok and t.stride(0) >= t[0].numel()
+        if not ok:
+            raise ValueError(f"{name}: layout {tuple(t.shape)} strides {t.stride()} is not contiguous")
+    if numel and t.numel() < numel:
         raise ValueError(f"{name}: {t.numel()} elements, at least {numel} needed")
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+_torch_module = None
 
 
 def _torch():
-    import torch
-    if not torch.cuda.is_available():
-        raise RuntimeError("no GPU visible: the HIP path has no CPU fallback")
-    return torch
+    """torch, once it has been seen to have a GPU (0.6 us a call to ask)."""
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        if not torch.cuda.is_available():
+            raise RuntimeError("no GPU visible: the HIP path has no CPU fallback")
+        _torch_module = torch
+    return _torch_module
 
 
 class Ctx:
@@ -279,7 +291,7 @@ class CqWeight:
 
     def prepare_input(self, x, xh=None):
         torch = _torch()
-        x2 = x.reshape(-1, self.in_feat)
+        x2 = x if x.dim() == 2 and x.size(1) == self.in_feat else x.reshape(-1, self.in_feat)
         if xh is None:
             xh = torch.empty(x2.shape[0], self.in_padded, dtype=torch.float32, device=x.device)
         n = x2.shape[0]
@@ -557,13 +569,18 @@ def attend_i8_prefill(ctx, num_heads, num_kv_heads, qk, vd, q, k, v, window=0, q
     seq = q.shape[0]
     g = kv_geom(num_heads, num_kv_heads, qk, vd, max(seq, 1))
     blk, _ = kv_alloc(g, 1, q.device.index or 0)
-    pos = torch.arange(seq, dtype=torch.int32, device=q.device)
-    kv_write(ctx, g, blk, 0, pos, k.contiguous(), v.contiguous())
-    hi = pos
-    lo = torch.clamp(pos + 1 - window, min=0) if window else torch.zeros_like(pos)
+    if window >= 0 and seq > 0:
+        # both ends of the spans in two operations: 1 - w .. seq - 1 clamped to
+        # 0 holds every row's first position, then, w - 1 on, its last (its own)
+        w = min(window, seq) if window else seq
+        ends = torch.arange(1 - w, seq, dtype=torch.int32, device=q.device).clamp_(min=0)
+        lo, hi = ends[:seq], ends[w - 1:]
+    else:
+        hi = torch.arange(seq, dtype=torch.int32, device=q.device)
+        lo = torch.clamp(hi + 1 - window, min=0) if window else torch.zeros_like(hi)
+    kv_write(ctx, g, blk, 0, hi, k.contiguous(), v.contiguous())
     scale = float(np.float32(1.0) / np.float32(math.sqrt(qk)))
-    return attend_step_i8(ctx, g, blk, 0, lo.to(torch.int32), hi, q.contiguous(), scale,
-                          quant_query)
+    return attend_step_i8(ctx, g, blk, 0, lo, hi, q.contiguous(), scale, quant_query)
 
 
 # ---- Needle-3 forward on the device ----------------------------------------
