@@ -15,10 +15,11 @@
 //   * code loads split in two halves so the second half is in flight while
 //     the first computes; nontemporal loads, since codes are read once.
 // Other widths take a kernel with the activations in LDS and part steps.
-// GEMM (prefill) converts X to bf16 once, dequantises weight tiles to bf16 in
-// LDS through the bf16-rounded codebook and feeds v_mfma_f32_16x16x32_bf16
-// with fp32 accumulation: 64x64 tiles below M = 96, 128x128 tiles, and
-// 256x256 tiles with two waves per SIMD once a launch has a tile per CU.
+// GEMM (prefill) rounds X to bf16, dequantises weights to bf16 through the
+// bf16-rounded codebook and feeds v_mfma_f32_16x16x32_bf16 with fp32
+// accumulation: up to 64 rows codes go from memory to fragments, 128 columns a
+// block; above, weight tiles go through LDS, 64x64 below M = 96, 128x128, and
+// 256x256 with two waves per SIMD once a launch has a tile per CU.
 #include "nd_internal.h"
 #include "nd_lanes.h"
 
@@ -730,163 +731,163 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
             }
 }
 
-// M <= 64 (e.g. the rows of 64 sessions at once): each code feeds only 64
+// M <= 64 (e.g. the rows of 64 sessions at once): each code feeds at most 64
 // rows, so the launch streams codes and the decode, not the MFMAs, sets the
-// pace.  A 256-thread block owns 128 output columns (two codebook groups)
-// and all M rows; the codes skip LDS entirely.  Lane (r16, q) of wave w
-// loads 16 consecutive codes of rows n0 + 32w + 16t + r16 (t = 0, 1) per
-// 64-wide K step -- four lanes cover a row's 64 bytes in one load -- and
-// decodes them through a lane-replicated codebook table (entry e, replica r
-// in bank r: conflict-free gathers; both groups' bf16 in one word) straight
-// into MFMA B fragments.  X is staged in LDS 128 columns at a time, double
-// buffered.  Both operands use physical k 16q..16q+7 for the first MFMA of
-// a step and 16q+8..+15 for the second, so the K order differs from the
-// other tile shapes' (results agree to fp32 rounding, not bit for bit).
+// pace.  A block of eight waves owns 128 output columns (two codebook groups)
+// and all M rows in 16 MT; the codes skip LDS.  Wave w takes columns 16 w ..
+// 16 w + 15 through K steps of 128: lane (r16, q) loads codes 16q..16q+15 and
+// 64+16q..64+16q+15 of row r16, the wave both halves of each 128-byte line
+// (through the caches: with nontemporal loads the line came from memory twice,
+// 43 us against 27 for 24 x 3 rows by 2624 x 2208), and decodes them through a
+// lane-replicated codebook table (entry e, replica r in bank r: conflict-free
+// gathers; both groups' bf16 in one word) straight into MFMA B fragments; a
+// byte dot product forms an entry's address in one operation.  X is rounded to
+// bf16 as it is staged in LDS, double buffered.  Codes are loaded two steps
+// ahead, X three.  Both operands use physical k 16q..16q+7 for the first MFMA
+// of a half step and 16q+8..+15 for the second.  Past K (a last step of 32, 64
+// or 96), X is zero and the codes are a zero entry behind the codebook.
+// Bound by LDS (gathers and X fragments) at 64 rows, by memory at few.
+// Measured, MI355X, a call (before: four waves of 32 columns, X rounded by a
+// launch of its own; widths not a multiple of 128 in 64x64 tiles): 20 problems
+// of 3072 x 768, 64 rows 23.8 -> 20.8 us, 16 rows 23.5 -> 12.6, 3 rows 22.9 ->
+// 11.9; 24 x 3 rows by 2624 x 2208 62.6 -> 25.3 (5.6 TB/s); 8 x 50 by 768 x
+// 3072 47.4 -> 31.3.  32 columns and half the step a wave: 21.2 and 14.7 for
+// 64 and 16 rows.
 constexpr int kRN = 128;          // output columns (N) per block: two codebook groups
-constexpr int kRC = 128;          // K per staged X chunk
+constexpr int kRC = 128;          // K per step
 constexpr int kRXS = kRC + 8;     // padded X row in LDS (bf16)
 
-__global__ __launch_bounds__(256, 2) void cb8_gemm_m64_kernel(const unsigned short *__restrict__ Xb,
-                                                              const uint8_t *__restrict__ W,
-                                                              const float *__restrict__ cb,
-                                                              float *__restrict__ Y, int M, int N,
-                                                              int K, size_t ws, size_t cs, size_t ys,
-                                                              int tiles_n, int xcd_run)
+template <int MT>
+__global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__restrict__ X, size_t xstride,
+                                                               const uint8_t *__restrict__ W,
+                                                               const float *__restrict__ cb,
+                                                               float *__restrict__ Y, int M, int N, int K,
+                                                               size_t ws, size_t cs, size_t ys, int tiles_n,
+                                                               int xcd_run)
 {
-    __shared__ __align__(16) uint32_t tab[256 * 32];
-    __shared__ __align__(16) unsigned short xs[2][64 * kRXS];
+    __shared__ __align__(16) uint32_t tab[257 * 32];  // a zero entry behind the codebook
+    __shared__ __align__(16) unsigned short xs[2][16 * MT * kRXS];
     // the column tiles of one problem are consecutive in u and land on one
     // XCD (workgroups are dealt to the 8 XCDs round-robin), sharing X in L2
     const int id = blockIdx.x;
     const int u = xcd_run ? (id % 8) * xcd_run + id / 8 : id;
     const int z = u / tiles_n, tn = u - z * tiles_n;
-    Xb += size_t(z) * M * K;
+    X += size_t(z) * xstride;
     W += z * ws;
     cb += z * cs;
     Y += z * ys;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int r16 = lane & 15, q = lane >> 4;
-    const int n0 = tn * kRN;
-    const uint8_t *wp0 = W + size_t(n0 + 32 * w + r16) * K + 16 * q;
-    const uint8_t *wp1 = wp0 + size_t(16) * K;
-    const int nc = K / kRC;
-    // codes of chunk c: two 64-wide steps x two row groups.  Past the last
-    // chunk the load reads X instead (L2-resident, unused), so every chunk
-    // issues the same loads and the waits count them exactly.
-    uint4 cw[2][2][2];
+    const int n0 = tn * kRN, col = n0 + 16 * w + r16;
+    const uint8_t *wp0 = W + size_t(min(col, N - 1)) * K;
+    const int k0 = 16 * q;
+    const int nc = (K + kRC - 1) / kRC;
+    // every step issues the same loads (addresses clamped), so the waits
+    // count them exactly
+    u32x4_t cw[2][2];
     auto cload = [&](int slot, int c) {
-        const bool in = c < nc;
-        const uint8_t *p0 = in ? wp0 + c * kRC : reinterpret_cast<const uint8_t *>(Xb);
-        const uint8_t *p1 = in ? wp1 + c * kRC : reinterpret_cast<const uint8_t *>(Xb);
+        const int k = min(c * kRC + k0, K - 16), k1 = min(c * kRC + 64 + k0, K - 16);
+        cw[slot][0] = *(reinterpret_cast<const u32x4_t *>(wp0 + k));
+        cw[slot][1] = *(reinterpret_cast<const u32x4_t *>(wp0 + k1));
+    };
+    // X of step c: 16 MT rows x 128, four columns a thread and piece
+    float4 xr[2][MT];
+    const int xrow = t >> 5, xcol = (t & 31) * 4;
+    auto xload = [&](int slot, int c) {
 #pragma unroll
-        for (int kp = 0; kp < 2; ++kp) {
-            const u32x4_t c0 = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p0 + kp * 64));
-            const u32x4_t c1 = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p1 + kp * 64));
-            cw[slot][kp][0] = make_uint4(c0.x, c0.y, c0.z, c0.w);
-            cw[slot][kp][1] = make_uint4(c1.x, c1.y, c1.z, c1.w);
+        for (int i = 0; i < MT; ++i)
+            xr[slot][i] = *reinterpret_cast<const float4 *>(X + size_t(min(xrow + 16 * i, M - 1)) * K +
+                                                            min(c * kRC + xcol, K - 4));
+    };
+    auto xstore = [&](int slot, int buf, int c) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const float4 v = xr[slot][i];
+            uint2 h = make_uint2(f32x2_to_bf16x2_rne(v.x, v.y), f32x2_to_bf16x2_rne(v.z, v.w));
+            if (xrow + 16 * i >= M || c * kRC + xcol >= K) h = make_uint2(0, 0);
+            *reinterpret_cast<uint2 *>(&xs[buf][(xrow + 16 * i) * kRXS + xcol]) = h;
         }
     };
-    // X chunk c: 64 rows x 128 bf16, 16-byte pieces; rows past M are zero
-    uint4 xr[4];
-    auto xload = [&](int c) {
-        const int cc = c < nc ? c : nc - 1;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = t + 256 * i, row = idx >> 4, col = (idx & 15) * 8;
-            xr[i] = *reinterpret_cast<const uint4 *>(Xb + size_t(row < M ? row : M - 1) * K + cc * kRC + col);
-            if (row >= M) xr[i] = make_uint4(0, 0, 0, 0);
-        }
-    };
-    auto xstore = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = t + 256 * i, row = idx >> 4, col = (idx & 15) * 8;
-            *reinterpret_cast<uint4 *>(&xs[buf][row * kRXS + col]) = xr[i];
-        }
-    };
+    xload(0, 0);
     cload(0, 0);
-    xload(0);
+    xload(1, 1);
+    cload(1, 1);
     {
         // the table, through a staging row in xs[1] so every write is
-        // conflict-free: word e of the staging row, then 8 x 16 bytes a thread
+        // conflict-free: word e of the staging row, then 4 x 16 bytes a thread
         uint32_t *vals = reinterpret_cast<uint32_t *>(&xs[1][0]);
-        vals[t] = f32_to_bf16_rne(cb[size_t(n0 / 64) * 256 + t]) |
-                  (uint32_t(f32_to_bf16_rne(cb[size_t(n0 / 64 + 1) * 256 + t])) << 16);
+        const int ng = N / 64 - 1;
+        if (t < 256)
+            vals[t] = f32_to_bf16_rne(cb[size_t(n0 / 64) * 256 + t]) |
+                      (uint32_t(f32_to_bf16_rne(cb[size_t(min(n0 / 64 + 1, ng)) * 256 + t])) << 16);
         __syncthreads();
         uint4 *t4 = reinterpret_cast<uint4 *>(tab);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t v = vals[(i * 256 + t) >> 3];
-            t4[i * 256 + t] = make_uint4(v, v, v, v);
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t v = vals[(i * 512 + t) >> 3];
+            t4[i * 512 + t] = make_uint4(v, v, v, v);
         }
     }
-    xstore(0);
+    if (t < 32) tab[256 * 32 + t] = 0;
+    xstore(0, 0, 0);
+    xload(0, 2);
     __syncthreads();
     // waves 0-1 hold rows of the first group (low halves), 2-3 the second
-    const uint32_t sel = w >= 2 ? 0x07060302u : 0x05040100u;
-    const uint32_t *tl = tab + (lane & 31);
-    floatx4_t acc[4][2];
+    const uint32_t sel = w >= 4 ? 0x07060302u : 0x05040100u;
+    typedef __attribute__((address_space(3))) uint32_t *lds_u32;
+    const uint32_t base = uint32_t(reinterpret_cast<uintptr_t>((lds_u32)(tab + (lane & 31))));
+    floatx4_t acc[MT];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    auto decode = [&](const uint4 &c, bf16x8_t &f0, bf16x8_t &f1) {
-        const uint32_t d[4] = {c.x, c.y, c.z, c.w};
+    for (int a = 0; a < MT; ++a) acc[a] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    // one dot product of bytes makes an entry's address; 16 codes past the end
+    // are the zero entry
+    auto decode = [&](const u32x4_t &d, bool in, bf16x8_t &f0, bf16x8_t &f1) {
+        const uint32_t at = in ? base : base + 256 * 128;
         uint32_t h[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const uint32_t v0 = tl[((d[k >> 1] >> (16 * (k & 1))) & 0xffu) * 32];
-            const uint32_t v1 = tl[((d[k >> 1] >> (16 * (k & 1) + 8)) & 0xffu) * 32];
+            const uint32_t dw = in ? d[k >> 1] : 0u;
+            const uint32_t v0 = *(lds_u32)(__builtin_amdgcn_udot4(dw, 0x80u << (16 * (k & 1)), at, false));
+            const uint32_t v1 = *(lds_u32)(__builtin_amdgcn_udot4(dw, 0x8000u << (16 * (k & 1)), at, false));
             h[k] = __builtin_amdgcn_perm(v1, v0, sel);
         }
         f0 = __builtin_bit_cast(bf16x8_t, make_uint4(h[0], h[1], h[2], h[3]));
         f1 = __builtin_bit_cast(bf16x8_t, make_uint4(h[4], h[5], h[6], h[7]));
     };
-    auto compute = [&](int buf, int slot) {
-#pragma unroll
-        for (int kp = 0; kp < 2; ++kp) {
-            bf16x8_t b[2][2];
-            decode(cw[slot][kp][0], b[0][0], b[0][1]);
-            decode(cw[slot][kp][1], b[1][0], b[1][1]);
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt) {
-                const unsigned short *xa = &xs[buf][(16 * mt + r16) * kRXS + kp * 64 + 16 * q];
-                const bf16x8_t a0 = *reinterpret_cast<const bf16x8_t *>(xa);
-                const bf16x8_t a1 = *reinterpret_cast<const bf16x8_t *>(xa + 8);
-#pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
-                    acc[mt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[tt][0], acc[mt][tt], 0, 0, 0);
-                    acc[mt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[tt][1], acc[mt][tt], 0, 0, 0);
-                }
-            }
-        }
-    };
-    // chunk c: X of chunk c + 1 and the codes of chunk c + 1 in flight while
-    // chunk c is multiplied.  X is issued first, so storing it waits for X
-    // only and the code loads stay in flight across the barrier.
     for (int c0 = 0; c0 < nc; c0 += 2) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int c = c0 + s;
             if (c < nc) {
-                xload(c + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                cload(s ^ 1, c + 1);
-                compute(c & 1, s);
-                if (c + 1 < nc) xstore((c + 1) & 1);
+                // X of step c + 1 into the buffer that step c - 1 read
+                xstore(s ^ 1, s ^ 1, c + 1);
+                xload(s ^ 1, c + 3);
+                bf16x8_t b[2][2];
+                decode(cw[s][0], c * kRC + k0 < K, b[0][0], b[0][1]);
+                decode(cw[s][1], c * kRC + 64 + k0 < K, b[1][0], b[1][1]);
+                cload(s, c + 2);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+                    for (int kp = 0; kp < 2; ++kp) {
+                        const unsigned short *xa = &xs[s][(16 * mt + r16) * kRXS + 64 * kp + k0];
+                        const bf16x8_t a0 = *reinterpret_cast<const bf16x8_t *>(xa);
+                        const bf16x8_t a1 = *reinterpret_cast<const bf16x8_t *>(xa + 8);
+                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[kp][0], acc[mt], 0, 0, 0);
+                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[kp][1], acc[mt], 0, 0, 0);
+                    }
+                }
                 __syncthreads();
             }
         }
     }
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 16 * mt + 4 * q + i;
-                if (m < M) Y[size_t(m) * N + n0 + 32 * w + 16 * tt + r16] = acc[mt][tt][i];
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int m = 16 * mt + 4 * q + i;
+            if (m < M && col < N) Y[size_t(m) * N + col] = acc[mt][i];
+        }
 }
 
 int launch_gemv(nd_ctx *ctx, size_t count, const uint8_t *w, size_t w_stride, const float *cb,
@@ -962,16 +963,17 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
                "x must be 16-byte and w 8-byte aligned, problem by problem");
     const size_t big_tiles = (out / kPN) * ((m + kPM - 1) / kPM) * count;
     const size_t cus = size_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
-    const size_t m64_tiles = (out / kRN) * count;
-    const bool use_m64 = m <= 64 && out % kRN == 0 && in % kRC == 0 &&
-                         (reinterpret_cast<uintptr_t>(w) & 15) == 0 && w_stride % 16 == 0 &&
-                         m64_tiles <= 0x7fffffff;
-    const bool use_256 = !use_m64 && m >= 96 && out % kPN == 0 && big_tiles >= cus && big_tiles <= 0x7fffffff;
+    const size_t row_tiles = ((out + kRN - 1) / kRN) * count;
+    // up to 64 rows: codes of 16 at a time, so 16-byte aligned
+    const bool use_rows = m <= 64 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && w_stride % 16 == 0 &&
+                          row_tiles <= 0x7fffffff;
+    const bool use_256 = m >= 96 && out % kPN == 0 && big_tiles >= cus && big_tiles <= 0x7fffffff;
     // X to bf16 once per call, into the context workspace, for the kernels
-    // that stage bf16 X; the 256x256 kernel rounds fp32 X as it stages it
+    // that stage bf16 X; the 256x256 and the row kernel round fp32 X as they
+    // stage it
     const size_t mk = m * in;
     unsigned short *xb = nullptr;
-    if (!use_256) {
+    if (!use_256 && !use_rows) {
         void *wsp = nullptr;
         if (int rc = nd::workspace(ctx, count * mk * sizeof(unsigned short), &wsp)) return rc;
         xb = static_cast<unsigned short *>(wsp);
@@ -979,12 +981,20 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
                            dim3(256), 0, ctx->stream, x, x_stride, xb, mk);
         if (int rc = nd::check_launch("x_to_bf16")) return rc;
     }
-    if (use_m64) {
+    if (use_rows) {
         // codes streamed into registers, 128 columns a block
-        const int run = m64_tiles % 8 == 0 ? int(m64_tiles / 8) : 0;
-        hipLaunchKernelGGL(cb8_gemm_m64_kernel, dim3(unsigned(m64_tiles)), dim3(256), 0, ctx->stream, xb, w,
-                           cb, y, int(m), int(out), int(in), w_stride, cb_stride, y_stride,
-                           int(out / kRN), run);
+        const int run = row_tiles % 8 == 0 ? int(row_tiles / 8) : 0;
+#define ND_GEMM_ROWS(MT)                                                                            \
+    hipLaunchKernelGGL((cb8_gemm_rows_kernel<MT>), dim3(unsigned(row_tiles)), dim3(512), 0, ctx->stream, x, \
+                       x_stride, w, cb, y, int(m), int(out), int(in), w_stride, cb_stride, y_stride,    \
+                       int((out + kRN - 1) / kRN), run)
+        if (m <= 16)
+            ND_GEMM_ROWS(1);
+        else if (m <= 32)
+            ND_GEMM_ROWS(2);
+        else
+            ND_GEMM_ROWS(4);
+#undef ND_GEMM_ROWS
     } else if (use_256) {
         // at least one 256x256 tile per CU: below that the 128x128 tiles fill
         // the chip better

@@ -225,3 +225,36 @@ def test_gemm_bf16_rounding_is_round_to_nearest_even(ctx, count, m, out, inn):
     nd.cb8_gemm_batched(ctx, dev(X), dev(W), dev(CB), Y)
     got = host(Y)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("count,out,inn", [(1, 64, 32), (3, 64, 128), (2, 192, 96), (1, 128, 160), (9, 320, 416),
+                                           (8, 256, 1024)])
+def test_gemm_rows(ctx, count, m, out, inn):
+    """Up to 64 rows: an odd group of columns, K steps that are not full,
+    padded strides.  bf16 operands are exact in the reference, so the bound is
+    inn roundings of the fp32 sums; an infinite entry of an unused code stays
+    out, and one that is used reaches its column only."""
+    rng = np.random.default_rng(m * 7 + out + inn)
+    W = rng.integers(0, 255, size=(count, out * inn + 32), dtype=np.uint8)
+    CB = rng.normal(0, 0.02, size=(count, out // 64, 256)).astype(np.float32)
+    CB[:, :, 255] = np.inf
+    X = rng.normal(size=(count, m * inn + 4)).astype(np.float32)
+    w, cb, x = dev(W), dev(CB), dev(X)
+    y = torch.full((count, m * out + 3), 7.0, device="cuda")
+    run = lambda: nd._check(nd.lib().nd_cb8_gemm_batched(
+        ctx.h, count, x.data_ptr(), X.shape[1], w.data_ptr(), W.shape[1], cb.data_ptr(), out // 64 * 256,
+        y.data_ptr(), m * out + 3, m, out, inn))
+    run()
+    Y = host(y)
+    bf = lambda a: dev(a).bfloat16().double().cpu().numpy()
+    for i in range(count):
+        v = bf(CB[i])[np.arange(out)[:, None] // 64, W[i, :out * inn].reshape(out, inn)]
+        xi = bf(X[i, :m * inn]).reshape(m, inn)
+        bound = (np.abs(xi) @ np.abs(v).T) * inn * 2.0 ** -23
+        assert np.all(np.abs(Y[i, :m * out].reshape(m, out) - xi @ v.T) <= bound)
+    assert np.all(Y[:, m * out:] == 7.0)
+    w[0, (out - 1) * inn] = 255
+    run()
+    Z = host(y)[0, :m * out].reshape(m, out)
+    assert np.all(np.isinf(Z[:, -1])) and np.isfinite(Z[:, :-1]).all()
