@@ -17,9 +17,10 @@
 // Other widths take a kernel with the activations in LDS and part steps.
 // GEMM (prefill) rounds X to bf16, dequantises weights to bf16 through the
 // bf16-rounded codebook and feeds v_mfma_f32_16x16x32_bf16 with fp32
-// accumulation: up to 64 rows codes go from memory to fragments, 128 columns a
-// block; above, weight tiles go through LDS, 64x64 below M = 96, 128x128, and
-// 256x256 with two waves per SIMD once a launch has a tile per CU.
+// accumulation: up to 64 rows, and for launches too small to fill the chip,
+// codes go from memory to fragments in 64x128 tiles; above, weight tiles go
+// through LDS, 128x128, and 256x256 with two waves per SIMD once a launch has a
+// tile per CU.
 #include "nd_internal.h"
 #include "nd_lanes.h"
 
@@ -274,8 +275,6 @@ __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_any_kernel(
 
 // ---------------------------------------------------------------------------
 // GEMM: Y[m][o] = sum_k bf16(X[m][k]) * bf16(cb[o/64][W[o][k]]), fp32 accumulate.
-// Block tile 64 (M) x 64 (N, one codebook) with K steps of 32; 4 waves in a
-// 2x2 grid, each wave a 32x32 output = 2x2 MFMA 16x16x32 tiles.
 // ---------------------------------------------------------------------------
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
@@ -297,7 +296,7 @@ __device__ inline unsigned short f32_to_bf16_rne(float f)
     return static_cast<unsigned short>(f32x2_to_bf16x2_rne(f, 0.0f));
 }
 
-constexpr int kGM = 64, kGN = 64, kGK = 128;
+constexpr int kGN = 64;     // columns sharing a codebook
 constexpr int kLdsPad = 8;  // bf16 elements of padding per LDS row
 
 // X (f32) to bf16, round to nearest even; problem blockIdx.y of a batch at
@@ -343,125 +342,13 @@ __global__ __launch_bounds__(256) void x_to_bf16_kernel(const float *__restrict_
     }
 }
 
-// Y[M][N] = X[M][K] . decode(W[N][K])^T, X already bf16.  A 256-thread block
-// owns a 64x64 output tile (4 waves of 32x32, 2x2 MFMA 16x16x32 tiles each)
-// and walks K 128 at a time: the next step's X rows and codes are loaded
-// into registers while the current step's 16 MFMAs per wave run from LDS.
-// The block's codebook sits in LDS already rounded to bf16, so decoding a
-// code is one LDS read.
-__global__ __launch_bounds__(256) void cb8_gemm_kernel(const unsigned short *__restrict__ Xb,
-                                                       const uint8_t *__restrict__ W,
-                                                       const float *__restrict__ cb,
-                                                       float *__restrict__ Y, int M, int N,
-                                                       int K, size_t ws, size_t cs, size_t ys)
-{
-    __shared__ unsigned short cbh[256];
-    __shared__ __align__(16) unsigned short As[kGM][kGK + kLdsPad];
-    __shared__ __align__(16) unsigned short Bs[kGN][kGK + kLdsPad];
-
-    // problem blockIdx.z of a batch: X at M*K, the rest at element strides
-    Xb += blockIdx.z * size_t(M) * K;
-    W += blockIdx.z * ws;
-    cb += blockIdx.z * cs;
-    Y += blockIdx.z * ys;
-
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = t >> 6;
-    const int n0 = blockIdx.x * kGN;
-    const int m0 = blockIdx.y * kGM;
-    const int wm = (wave >> 1) * 32;  // wave's row offset within the tile
-    const int wn = (wave & 1) * 32;   // wave's column offset
-
-    cbh[t] = f32_to_bf16_rne(cb[size_t(n0 / 64) * 256 + t]);
-
-    floatx4_t acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-    const int sr = t >> 2;          // staged row 0..63 (of A and of B)
-    const int sc = (t & 3) * 32;    // staged columns sc..sc+31 of the K step
-    const bool mrow = m0 + sr < M;
-    const unsigned short *xrow = Xb + size_t(mrow ? m0 + sr : 0) * K;
-    const uint8_t *wrow = W + size_t(n0 + sr) * K;  // N is a multiple of 64
-    uint4 xa[4];
-    uint2 wc[4];
-    auto load = [&](int k0) {
-        const bool on = k0 + sc < K;  // K is a multiple of 32: a 32-column run is all in or out
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            xa[q] = on && mrow ? *reinterpret_cast<const uint4 *>(xrow + k0 + sc + 8 * q)
-                               : make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            wc[q] = on ? *reinterpret_cast<const uint2 *>(wrow + k0 + sc + 8 * q) : make_uint2(0, 0);
-        return on;
-    };
-    auto store = [&](bool on) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) *reinterpret_cast<uint4 *>(&As[sr][sc + 8 * q]) = xa[q];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t d[2] = {wc[q].x, wc[q].y};
-            uint32_t h[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t lo = cbh[(d[e >> 1] >> (16 * (e & 1))) & 0xffu];
-                const uint32_t hi = cbh[(d[e >> 1] >> (16 * (e & 1) + 8)) & 0xffu];
-                h[e] = on ? lo | (hi << 16) : 0u;
-            }
-            *reinterpret_cast<uint4 *>(&Bs[sr][sc + 8 * q]) = make_uint4(h[0], h[1], h[2], h[3]);
-        }
-    };
-    __syncthreads();  // codebook in LDS
-    bool on = load(0);
-    // MFMA 16x16x32 bf16: lane l supplies A[row l%16][k 8*(l/16) .. +8]
-    // and B[k 8*(l/16) .. +8][col l%16].
-    const int r16 = lane & 15;
-    const int kq = (lane >> 4) * 8;
-    for (int k0 = 0; k0 < K; k0 += kGK) {
-        store(on);
-        __syncthreads();
-        if (k0 + kGK < K) on = load(k0 + kGK);
-        const int steps = (K - k0 < kGK ? K - k0 : kGK) / 32;
-        for (int kk = 0; kk < steps; ++kk) {
-            bf16x8_t afrag[2], bfrag[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-                afrag[a] = *reinterpret_cast<const bf16x8_t *>(&As[wm + a * 16 + r16][kk * 32 + kq]);
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                bfrag[b] = *reinterpret_cast<const bf16x8_t *>(&Bs[wn + b * 16 + r16][kk * 32 + kq]);
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag[a], bfrag[b],
-                                                                        acc[a][b], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    // C layout: lane l holds C[4*(l/16) + i][l%16], i < 4.
-    const int col = lane & 15;
-    const int rb = (lane >> 4) * 4;
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = m0 + wm + a * 16 + rb + i;
-                const int n = n0 + wn + b * 16 + col;
-                if (m < M) Y[size_t(m) * N + n] = acc[a][b][i];
-            }
-}
-
-// The same product with 128x128 tiles for M >= 96: 4 waves of 64x64 (4x4
-// MFMA tiles each), K steps of 64, each thread staging half a row of A
-// (32 bf16) and of B (32 codes).  A decoded code strip serves twice the
-// rows of the 64x64 kernel, halving the decode work per MFMA.
+// Y[M][N] = X[M][K] . decode(W[N][K])^T, X already bf16, on 128x128 tiles: 4
+// waves of 64x64 (4x4 MFMA tiles each), K steps of 64, each thread staging half
+// a row of A (32 bf16) and of B (32 codes): the next step's are loaded into
+// registers while the current step's MFMAs run from LDS.  The codebooks sit in
+// LDS already rounded to bf16, so decoding a code is one LDS read.  With an odd
+// number of 64-column groups the last tile's second half repeats the last row
+// and is not stored.
 constexpr int kBM = 128, kBN = 128, kBK = 64;
 
 __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *__restrict__ Xb,
@@ -489,7 +376,7 @@ __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *
 
     // the tile's two 64-row codebooks, rounded to bf16
     cbh[0][t] = f32_to_bf16_rne(cb[size_t(n0 / 64) * 256 + t]);
-    cbh[1][t] = f32_to_bf16_rne(cb[size_t(n0 / 64 + 1) * 256 + t]);
+    cbh[1][t] = f32_to_bf16_rne(cb[size_t(min(n0 / 64 + 1, N / 64 - 1)) * 256 + t]);
 
     floatx4_t acc[4][4];
 #pragma unroll
@@ -501,7 +388,7 @@ __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *
     const int sc = (t & 1) * 32;    // staged columns sc..sc+31 of the K step
     const bool mrow = m0 + sr < M;
     const unsigned short *xrow = Xb + size_t(mrow ? m0 + sr : 0) * K;
-    const uint8_t *wrow = W + size_t(n0 + sr) * K;  // N is a multiple of 128 here
+    const uint8_t *wrow = W + size_t(min(n0 + sr, N - 1)) * K;  // N is a multiple of 64
     const unsigned short *cbr = cbh[sr >> 6];
     uint4 xa[4];
     uint2 wc[4];
@@ -568,7 +455,7 @@ __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *
             for (int i = 0; i < 4; ++i) {
                 const int m = m0 + wm + a * 16 + rb + i;
                 const int n = n0 + wn + b * 16 + col;
-                if (m < M) Y[size_t(m) * N + n] = acc[a][b][i];
+                if (m < M && n < N) Y[size_t(m) * N + n] = acc[a][b][i];
             }
 }
 
@@ -731,10 +618,10 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
             }
 }
 
-// M <= 64 (e.g. the rows of 64 sessions at once): each code feeds at most 64
-// rows, so the launch streams codes and the decode, not the MFMAs, sets the
-// pace.  A block of eight waves owns 128 output columns (two codebook groups)
-// and all M rows in 16 MT; the codes skip LDS.  Wave w takes columns 16 w ..
+// Tiles of 16 MT rows (all of them up to M = 64, e.g. the rows of 64 sessions
+// at once) by 128 columns (two codebook groups), eight waves a block: each code
+// feeds at most 64 rows, so the launch streams codes and the decode, not the
+// MFMAs, sets the pace; the codes skip LDS.  Wave w takes columns 16 w ..
 // 16 w + 15 through K steps of 128: lane (r16, q) loads codes 16q..16q+15 and
 // 64+16q..64+16q+15 of row r16, the wave both halves of each 128-byte line
 // (through the caches: with nontemporal loads the line came from memory twice,
@@ -744,7 +631,9 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
 // byte dot product forms an entry's address in one operation.  X is rounded to
 // bf16 as it is staged in LDS, double buffered.  Codes are loaded two steps
 // ahead, X three.  Both operands use physical k 16q..16q+7 for the first MFMA
-// of a half step and 16q+8..+15 for the second.  Past K (a last step of 32, 64
+// of a half step and 16q+8..+15 for the second.  Without LINES a lane's codes
+// come eight at a time, at 8q of each 32 k: for codes aligned to 8 bytes, and
+// with the larger tiles' K order, bit for bit.  Past K (a last step of 32, 64
 // or 96), X is zero and the codes are a zero entry behind the codebook.
 // Bound by LDS (gathers and X fragments) at 64 rows, by memory at few.
 // Measured, MI355X, a call (before: four waves of 32 columns, X rounded by a
@@ -757,13 +646,13 @@ constexpr int kRN = 128;          // output columns (N) per block: two codebook 
 constexpr int kRC = 128;          // K per step
 constexpr int kRXS = kRC + 8;     // padded X row in LDS (bf16)
 
-template <int MT>
+template <int MT, bool LINES>
 __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__restrict__ X, size_t xstride,
                                                                const uint8_t *__restrict__ W,
                                                                const float *__restrict__ cb,
                                                                float *__restrict__ Y, int M, int N, int K,
                                                                size_t ws, size_t cs, size_t ys, int tiles_n,
-                                                               int xcd_run)
+                                                               int tiles_m, int xcd_run)
 {
     __shared__ __align__(16) uint32_t tab[257 * 32];  // a zero entry behind the codebook
     __shared__ __align__(16) unsigned short xs[2][16 * MT * kRXS];
@@ -771,8 +660,10 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     // XCD (workgroups are dealt to the 8 XCDs round-robin), sharing X in L2
     const int id = blockIdx.x;
     const int u = xcd_run ? (id % 8) * xcd_run + id / 8 : id;
-    const int z = u / tiles_n, tn = u - z * tiles_n;
-    X += size_t(z) * xstride;
+    const int z = u / (tiles_n * tiles_m), tm = u % tiles_m, tn = (u / tiles_m) % tiles_n;
+    X += size_t(z) * xstride + size_t(tm) * (16 * MT) * K;
+    Y += size_t(tm) * (16 * MT) * N;
+    M = min(M - tm * (16 * MT), 16 * MT);
     W += z * ws;
     cb += z * cs;
     Y += z * ys;
@@ -780,15 +671,24 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     const int r16 = lane & 15, q = lane >> 4;
     const int n0 = tn * kRN, col = n0 + 16 * w + r16;
     const uint8_t *wp0 = W + size_t(min(col, N - 1)) * K;
-    const int k0 = 16 * q;
+    const int k0 = LINES ? 16 * q : 8 * q;
     const int nc = (K + kRC - 1) / kRC;
     // every step issues the same loads (addresses clamped), so the waits
     // count them exactly
     u32x4_t cw[2][2];
     auto cload = [&](int slot, int c) {
-        const int k = min(c * kRC + k0, K - 16), k1 = min(c * kRC + 64 + k0, K - 16);
-        cw[slot][0] = *(reinterpret_cast<const u32x4_t *>(wp0 + k));
-        cw[slot][1] = *(reinterpret_cast<const u32x4_t *>(wp0 + k1));
+        if constexpr (LINES) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                cw[slot][h] = *reinterpret_cast<const u32x4_t *>(wp0 + min(c * kRC + 64 * h + k0, K - 16));
+        } else {
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const u32x2_t v = *reinterpret_cast<const u32x2_t *>(wp0 + min(c * kRC + 32 * h + k0, K - 8));
+                cw[slot][h >> 1][2 * (h & 1)] = v.x;
+                cw[slot][h >> 1][2 * (h & 1) + 1] = v.y;
+            }
+        }
     };
     // X of step c: 16 MT rows x 128, four columns a thread and piece
     float4 xr[2][MT];
@@ -841,19 +741,22 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     for (int a = 0; a < MT; ++a) acc[a] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
     // one dot product of bytes makes an entry's address; 16 codes past the end
     // are the zero entry
-    auto decode = [&](const u32x4_t &d, bool in, bf16x8_t &f0, bf16x8_t &f1) {
+    // one dot product of bytes makes an entry's address; codes past the end
+    // are the zero entry
+    auto decode = [&](uint32_t d0, uint32_t d1, bool in) {
         const uint32_t at = in ? base : base + 256 * 128;
-        uint32_t h[8];
+        const uint32_t dw[2] = {in ? d0 : 0u, in ? d1 : 0u};
+        uint32_t h[4];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint32_t dw = in ? d[k >> 1] : 0u;
-            const uint32_t v0 = *(lds_u32)(__builtin_amdgcn_udot4(dw, 0x80u << (16 * (k & 1)), at, false));
-            const uint32_t v1 = *(lds_u32)(__builtin_amdgcn_udot4(dw, 0x8000u << (16 * (k & 1)), at, false));
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t v0 = *(lds_u32)(__builtin_amdgcn_udot4(dw[k >> 1], 0x80u << (16 * (k & 1)), at, false));
+            const uint32_t v1 = *(lds_u32)(__builtin_amdgcn_udot4(dw[k >> 1], 0x8000u << (16 * (k & 1)), at, false));
             h[k] = __builtin_amdgcn_perm(v1, v0, sel);
         }
-        f0 = __builtin_bit_cast(bf16x8_t, make_uint4(h[0], h[1], h[2], h[3]));
-        f1 = __builtin_bit_cast(bf16x8_t, make_uint4(h[4], h[5], h[6], h[7]));
+        return __builtin_bit_cast(bf16x8_t, make_uint4(h[0], h[1], h[2], h[3]));
     };
+    // piece h of a step, eight codes: where its k start for this lane
+    auto piece = [&](int h) { return LINES ? 64 * (h >> 1) + 8 * (h & 1) + k0 : 32 * h + k0; };
     for (int c0 = 0; c0 < nc; c0 += 2) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -862,21 +765,19 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
                 // X of step c + 1 into the buffer that step c - 1 read
                 xstore(s ^ 1, s ^ 1, c + 1);
                 xload(s ^ 1, c + 3);
-                bf16x8_t b[2][2];
-                decode(cw[s][0], c * kRC + k0 < K, b[0][0], b[0][1]);
-                decode(cw[s][1], c * kRC + 64 + k0 < K, b[1][0], b[1][1]);
+                bf16x8_t b[4];
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    b[h] = decode(cw[s][h >> 1][2 * (h & 1)], cw[s][h >> 1][2 * (h & 1) + 1],
+                                  c * kRC + piece(h) < K);
                 cload(s, c + 2);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
+                for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                    for (int kp = 0; kp < 2; ++kp) {
-                        const unsigned short *xa = &xs[s][(16 * mt + r16) * kRXS + 64 * kp + k0];
-                        const bf16x8_t a0 = *reinterpret_cast<const bf16x8_t *>(xa);
-                        const bf16x8_t a1 = *reinterpret_cast<const bf16x8_t *>(xa + 8);
-                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[kp][0], acc[mt], 0, 0, 0);
-                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[kp][1], acc[mt], 0, 0, 0);
-                    }
-                }
+                    for (int h = 0; h < 4; ++h)
+                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            *reinterpret_cast<const bf16x8_t *>(&xs[s][(16 * mt + r16) * kRXS + piece(h)]), b[h],
+                            acc[mt], 0, 0, 0);
                 __syncthreads();
             }
         }
@@ -963,11 +864,19 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
                "x must be 16-byte and w 8-byte aligned, problem by problem");
     const size_t big_tiles = (out / kPN) * ((m + kPM - 1) / kPM) * count;
     const size_t cus = size_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
-    const size_t row_tiles = ((out + kRN - 1) / kRN) * count;
-    // up to 64 rows: codes of 16 at a time, so 16-byte aligned
-    const bool use_rows = m <= 64 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && w_stride % 16 == 0 &&
-                          row_tiles <= 0x7fffffff;
-    const bool use_256 = m >= 96 && out % kPN == 0 && big_tiles >= cus && big_tiles <= 0x7fffffff;
+    // 64-row tiles where m has no more, and where two a CU hold them all: a
+    // launch that does not fill the chip waits for one tile's steps, which are
+    // shorter there (us, rows / 128x128 tiles: 192 tiles of 1 x 512 by 3072 x
+    // 768 14.0 / 22.1, 384 of 8 x 500 by 768 x 768 23.9 / 29.2, 512 of 4 x 1000
+    // by 1024 x 256 14.5 / 15.6, 720 of 6 x 300 by 3072 x 768 34.7 / 33.1, 960
+    // of 20 x 80 by 3072 x 768 46.2 / 32.7).  Whole lines of codes need them
+    // 16-byte aligned.  Above 64 rows the K order is the larger tiles', so a
+    // problem's bits do not depend on how many share its launch.
+    const size_t row_tiles_m = (m + 63) / 64;
+    const size_t row_tiles = ((out + kRN - 1) / kRN) * row_tiles_m * count;
+    const bool lines = m <= 64 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && w_stride % 16 == 0;
+    const bool use_rows = (m <= 64 || row_tiles <= 2 * cus) && row_tiles <= 0x7fffffff;
+    const bool use_256 = !use_rows && m >= 96 && out % kPN == 0 && big_tiles >= cus && big_tiles <= 0x7fffffff;
     // X to bf16 once per call, into the context workspace, for the kernels
     // that stage bf16 X; the 256x256 and the row kernel round fp32 X as they
     // stage it
@@ -982,18 +891,19 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
         if (int rc = nd::check_launch("x_to_bf16")) return rc;
     }
     if (use_rows) {
-        // codes streamed into registers, 128 columns a block
         const int run = row_tiles % 8 == 0 ? int(row_tiles / 8) : 0;
-#define ND_GEMM_ROWS(MT)                                                                            \
-    hipLaunchKernelGGL((cb8_gemm_rows_kernel<MT>), dim3(unsigned(row_tiles)), dim3(512), 0, ctx->stream, x, \
+#define ND_GEMM_ROWS(MT, LINES)                                                                     \
+    hipLaunchKernelGGL((cb8_gemm_rows_kernel<MT, LINES>), dim3(unsigned(row_tiles)), dim3(512), 0, ctx->stream, x, \
                        x_stride, w, cb, y, int(m), int(out), int(in), w_stride, cb_stride, y_stride,    \
-                       int((out + kRN - 1) / kRN), run)
-        if (m <= 16)
-            ND_GEMM_ROWS(1);
+                       int((out + kRN - 1) / kRN), int(row_tiles_m), run)
+        if (!lines)
+            ND_GEMM_ROWS(4, false);
+        else if (m <= 16)
+            ND_GEMM_ROWS(1, true);
         else if (m <= 32)
-            ND_GEMM_ROWS(2);
+            ND_GEMM_ROWS(2, true);
         else
-            ND_GEMM_ROWS(4);
+            ND_GEMM_ROWS(4, true);
 #undef ND_GEMM_ROWS
     } else if (use_256) {
         // at least one 256x256 tile per CU: below that the 128x128 tiles fill
@@ -1002,16 +912,11 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
         hipLaunchKernelGGL(cb8_gemm256_kernel, dim3(unsigned(big_tiles)), dim3(512), 0, ctx->stream, x,
                            x_stride, w, cb, y, int(m), int(out), int(in), w_stride, cb_stride, y_stride,
                            int(out / kPN), int((m + kPM - 1) / kPM), run);
-    } else if (m >= 96 && out % kBN == 0) {
-        dim3 grid(static_cast<unsigned>(out / kBN), static_cast<unsigned>((m + kBM - 1) / kBM),
+    } else {
+        dim3 grid(static_cast<unsigned>((out + kBN - 1) / kBN), static_cast<unsigned>((m + kBM - 1) / kBM),
                   static_cast<unsigned>(count));
         hipLaunchKernelGGL(cb8_gemm128_kernel, grid, dim3(256), 0, ctx->stream, xb, w, cb, y,
                            int(m), int(out), int(in), w_stride, cb_stride, y_stride);
-    } else {
-        dim3 grid(static_cast<unsigned>(out / kGN), static_cast<unsigned>((m + kGM - 1) / kGM),
-                  static_cast<unsigned>(count));
-        hipLaunchKernelGGL(cb8_gemm_kernel, grid, dim3(256), 0, ctx->stream, xb, w, cb, y, int(m),
-                           int(out), int(in), w_stride, cb_stride, y_stride);
     }
     return nd::check_launch("cb8_gemm");
 }

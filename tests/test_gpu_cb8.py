@@ -258,3 +258,40 @@ def test_gemm_rows(ctx, count, m, out, inn):
     run()
     Z = host(y)[0, :m * out].reshape(m, out)
     assert np.all(np.isinf(Z[:, -1])) and np.isfinite(Z[:, :-1]).all()
+
+
+@pytest.mark.parametrize("one,many,m,out,inn", [(1, 30, 65, 2048, 96), (2, 33, 130, 704, 224), (1, 9, 200, 3072, 128),
+                                                (1, 20, 513, 192, 64), (3, 70, 96, 192, 1056)])
+def test_gemm_problem_bits_do_not_depend_on_the_launch(ctx, one, many, m, out, inn):
+    """Few problems take 64-row tiles, many 128x128 or 256x256 ones (an odd
+    number of column groups among them): the same bits above 64 rows, and
+    within inn roundings of the products of the bf16 operands."""
+    rng = np.random.default_rng(m + out)
+    W = dev(rng.integers(0, 256, size=(many, out, inn), dtype=np.uint8))
+    CB = dev(rng.normal(0, 0.02, size=(many, out // 64, 256)).astype(np.float32))
+    X = dev(rng.normal(size=(many, m, inn)).astype(np.float32))
+    Y = torch.empty(many, m, out, device="cuda")
+    nd.cb8_gemm_batched(ctx, X, W, CB, Y)
+    for i in (0, many - one):
+        Z = torch.empty(one, m, out, device="cuda")
+        nd.cb8_gemm_batched(ctx, X[i:i + one], W[i:i + one], CB[i:i + one], Z)
+        assert torch.equal(Z, Y[i:i + one])
+    v = torch.gather(CB[0].bfloat16().double().repeat_interleave(64, 0), 1, W[0].long())
+    x = X[0].bfloat16().double()
+    assert torch.all((Y[0].double() - x @ v.T).abs() <= (x.abs() @ v.abs().T) * inn * 2.0 ** -23)
+
+
+def test_gemm_codes_aligned_to_eight_bytes(ctx):
+    """Codes at an address that is a multiple of 8 only are taken."""
+    rng = np.random.default_rng(8)
+    m, out, inn = 40, 192, 160
+    raw = torch.zeros(out * inn + 8, dtype=torch.uint8, device="cuda")
+    W = raw[8:].view(out, inn)
+    W.copy_(dev(rng.integers(0, 256, size=(out, inn), dtype=np.uint8)))
+    CB = dev(rng.normal(0, 0.02, size=(out // 64, 256)).astype(np.float32))
+    X = dev(rng.normal(size=(m, inn)).astype(np.float32))
+    assert W.data_ptr() % 16 == 8
+    y = nd.cb8_gemm(ctx, X, W, CB).double()
+    v = torch.gather(CB.bfloat16().double().repeat_interleave(64, 0), 1, W.long())
+    x = X.bfloat16().double()
+    assert torch.all((y - x @ v.T).abs() <= (x.abs() @ v.abs().T) * inn * 2.0 ** -23)
