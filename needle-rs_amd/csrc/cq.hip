@@ -307,6 +307,11 @@ __global__ __launch_bounds__(kThreads) void cq_gemv_stream_kernel(
 // nontemporal) every CAP tiles and at the end: a global store inside the
 // loop would put its write round trip under the next wait.  Rows past the
 // end reread the last row; the loop body has no branches.
+// A launch of one or two tiles a workgroup (rows up to 16384 at 2 bits, 16384
+// and 32768 at 4) holds just those: the pipeline of four computed and reread
+// the last tile for each it did not have.  With the table of the 4-bit kernel
+// filled from one load a thread, one row by 8192 x 768 took 7.4 -> 5.0 us at 2
+// bits and 8.6 -> 5.0 at 4, by 16384 x 768 7.6 -> 5.2 and 13.0 -> 7.3.
 
 // Batch-1 GEMV on 2-bit (and ternary) rows of 16 * ND code dwords, ND <= 3
 // (in <= 768), by product lookup.  Each workgroup first builds, from the
@@ -387,14 +392,14 @@ __device__ inline void flush_stage(const float *stage, int cap, int rpt, int it_
     lds_barrier();
 }
 
-template <int ND>
+template <int ND, int D>
 __global__ __launch_bounds__(kNibThreads, 2) void cq_gemv_nib_kernel(
     const uint8_t *__restrict__ packed, const float *__restrict__ norms,
     const float *__restrict__ lut, const float *__restrict__ xh, float *__restrict__ y,
     int row_start, int rows, int row_bytes, int num_groups, int group, int iters)
 {
     constexpr int NI = 8 * ND;  // nibble positions per lane
-    constexpr int D = kNibDepth;
+    constexpr bool kOnce = D < kNibDepth;  // iters <= D: no loop, nothing to refill
     __shared__ float tab[16384];  // 64 KiB
     __shared__ float stage[kNibStage * kNibRows];
     const int t = threadIdx.x;
@@ -447,7 +452,7 @@ __global__ __launch_bounds__(kNibThreads, 2) void cq_gemv_nib_kernel(
 
     const uint32_t lb = uint32_t(((rg & 1) * kLanesPerRow + j) * 4);
     const char *tb = reinterpret_cast<const char *>(tab);
-    for (int it0 = 0; it0 < iters; it0 += D) {
+    for (int it0 = 0; it0 < (kOnce ? 1 : iters); it0 += D) {
 #pragma unroll
         for (int k = 0; k < D; ++k) {
             const int it = it0 + k;
@@ -469,9 +474,11 @@ __global__ __launch_bounds__(kNibThreads, 2) void cq_gemv_nib_kernel(
             }
             total = row16_sum(total);
             stage[(it % kNibStage) * kNibRows + rg] = total;  // the row's 16 lanes agree
-            __builtin_amdgcn_sched_barrier(0);
-            load(it + D, k);
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!kOnce) {
+                __builtin_amdgcn_sched_barrier(0);
+                load(it + D, k);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if ((it + 1) % kNibStage == 0) flush_stage<kNibThreads>(stage, kNibStage, kNibRows, it + 1, kNibStage, iters, rows, y);
         }
     }
@@ -496,21 +503,23 @@ __global__ __launch_bounds__(kNibThreads, 2) void cq_gemv_nib_kernel(
 constexpr int kQ4Threads = 512;
 constexpr int kQ4Rows = kQ4Threads / kLanesPerRow;  // 32 rows per tile
 constexpr int kQ4Repl = 32;                        // 256 B an entry
+static_assert(kQ4Threads == 512, "two threads fill an entry");
 static_assert(kQ4Repl * 8 == 256, "a lookup address puts the code byte at bit 8");
 constexpr int kQ4Depth = 4;
 constexpr int kQ4Stage = 32;                        // staged tiles (4 KiB)
 
-template <int ND>
+template <int ND, int D>
 __global__ __launch_bounds__(kQ4Threads) void cq_gemv_q4_kernel(
     const uint8_t *__restrict__ packed, const float *__restrict__ norms,
     const float *__restrict__ lut, const float *__restrict__ xh, float *__restrict__ y,
     int row_start, int rows, int row_bytes, int num_groups, int group, int iters)
 {
     constexpr int B = ND - 4;  // dwords of the second part
-    constexpr int D = kQ4Depth;
-    __shared__ float2 rep[256 * kQ4Repl];  // 64 KiB
+    constexpr bool kOnce = D < kQ4Depth;  // iters <= D: no loop, nothing to refill
+    __shared__ __align__(16) float2 rep[256 * kQ4Repl];  // 64 KiB
     __shared__ float stage[kQ4Stage * kQ4Rows];
     const int t = threadIdx.x, lane = t & 63, j = t & (kLanesPerRow - 1), rg = t / kLanesPerRow;
+    const float2 lv2 = *reinterpret_cast<const float2 *>(lut + (t >> 1) * 2);
     // the lane's activations: part A elements 32 j + 8 i + e (i < 4), part B
     // 512 + 8 B j + 8 (i - 4) + e
     float xr[ND][8];
@@ -531,10 +540,12 @@ __global__ __launch_bounds__(kQ4Threads) void cq_gemv_q4_kernel(
     // the activations are loop invariants: an empty asm reading them puts
     // the wait for their loads here, so the loop's waits do not count them
     // as pending on every pass
+    if constexpr (!kOnce) {
 #pragma unroll
-    for (int i = 0; i < ND; ++i)
+        for (int i = 0; i < ND; ++i)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) asm volatile("" ::"v"(xr[i][q]) : "memory");
+            for (int q = 0; q < 8; ++q) asm volatile("" ::"v"(xr[i][q]) : "memory");
+    }
     const int ga = (32 * j) / group, gb = B > 0 ? (512 + 8 * B * j) / group : ga;
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(packed + size_t(row_start) * row_bytes), (short)0, rows * row_bytes, 0x00020000);
@@ -571,14 +582,18 @@ __global__ __launch_bounds__(kQ4Threads) void cq_gemv_q4_kernel(
         load(k, k);
         __builtin_amdgcn_sched_barrier(0);
     }
-    for (int f = t; f < 256 * kQ4Repl; f += kQ4Threads)
-        rep[f] = *reinterpret_cast<const float2 *>(lut + (f / kQ4Repl) * 2);
+    // 16 replicas of entry t / 2 a thread, two a write, from a place of its own
+    // so that neighbouring threads' writes fall on different banks
+    float4 *rep4 = reinterpret_cast<float4 *>(rep) + t * (kQ4Repl / 4);
+#pragma unroll
+    for (int i = 0; i < kQ4Repl / 4; ++i)
+        rep4[(i + (t >> 1)) % (kQ4Repl / 4)] = make_float4(lv2.x, lv2.y, lv2.x, lv2.y);
     __syncthreads();
 
     // byte 0 of a lookup address: the lane's replica (8 bytes each)
     const uint32_t lb = uint32_t(lane & (kQ4Repl - 1)) * uint32_t(sizeof(float2));
     const char *repb = reinterpret_cast<const char *>(rep);
-    for (int it0 = 0; it0 < iters; it0 += D) {
+    for (int it0 = 0; it0 < (kOnce ? 1 : iters); it0 += D) {
 #pragma unroll
         for (int k = 0; k < D; ++k) {
             const int it = it0 + k;
@@ -604,9 +619,11 @@ __global__ __launch_bounds__(kQ4Threads) void cq_gemv_q4_kernel(
             float total = na[k] * ta + nb[k] * tb;
             total = row16_sum(total);
             stage[(it % kQ4Stage) * kQ4Rows + rg] = total;  // the row's 16 lanes agree
-            __builtin_amdgcn_sched_barrier(0);
-            load(it + D, k);
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!kOnce) {
+                __builtin_amdgcn_sched_barrier(0);
+                load(it + D, k);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if ((it + 1) % kQ4Stage == 0) flush_stage<kQ4Threads>(stage, kQ4Stage, kQ4Rows, it + 1, kQ4Stage, iters, rows, y);
         }
     }
@@ -1769,16 +1786,25 @@ int nd_cq_matvec_rows_prepared(nd_ctx *ctx, const nd_cq *w, const float *xh, siz
         const size_t tiles = (rows + kNibRows - 1) / kNibRows;
         const size_t blocks = tiles < slots ? tiles : slots;
         const int iters = int((tiles + blocks - 1) / blocks);
-#define ND_CQN(NDV)                                                                             \
-    hipLaunchKernelGGL((cq_gemv_nib_kernel<NDV>), dim3(unsigned(blocks)), dim3(kNibThreads), 0,  \
+#define ND_CQN_D(NDV, DV)                                                                             \
+    hipLaunchKernelGGL((cq_gemv_nib_kernel<NDV, DV>), dim3(unsigned(blocks)), dim3(kNibThreads), 0,  \
                        ctx->stream, w->packed, w->norms, w->lut, xh, y, int(row_start), int(rows), \
                        args_rb, ng, gr, iters)
+        // as many tiles held as a workgroup has, at most the pipeline's
+#define ND_CQN(NDV)                    \
+    if (iters == 1)                    \
+        ND_CQN_D(NDV, 1);              \
+    else if (iters == 2)               \
+        ND_CQN_D(NDV, 2);              \
+    else                               \
+        ND_CQN_D(NDV, kNibDepth)
         switch (row_dwords / 16) {
         case 1: ND_CQN(1); break;
         case 2: ND_CQN(2); break;
         default: ND_CQN(3); break;
         }
 #undef ND_CQN
+#undef ND_CQN_D
         return nd::check_launch("cq_gemv_nib");
     }
     if (stream && w->per_byte == 2 && row_dwords / 16 >= 4 && w->group % 32 == 0 && offsets32) {
@@ -1787,16 +1813,24 @@ int nd_cq_matvec_rows_prepared(nd_ctx *ctx, const nd_cq *w, const float *xh, siz
         const size_t tiles = (rows + kQ4Rows - 1) / kQ4Rows;
         const size_t blocks = tiles < slots ? tiles : slots;
         const int iters = int((tiles + blocks - 1) / blocks);
-#define ND_CQ4(NDV)                                                                             \
-    hipLaunchKernelGGL((cq_gemv_q4_kernel<NDV>), dim3(unsigned(blocks)), dim3(kQ4Threads), 0,    \
+#define ND_CQ4_D(NDV, DV)                                                                             \
+    hipLaunchKernelGGL((cq_gemv_q4_kernel<NDV, DV>), dim3(unsigned(blocks)), dim3(kQ4Threads), 0,    \
                        ctx->stream, w->packed, w->norms, w->lut, xh, y, int(row_start), int(rows), \
                        args_rb, ng, gr, iters)
+#define ND_CQ4(NDV)                    \
+    if (iters == 1)                    \
+        ND_CQ4_D(NDV, 1);              \
+    else if (iters == 2)               \
+        ND_CQ4_D(NDV, 2);              \
+    else                               \
+        ND_CQ4_D(NDV, kQ4Depth)
         switch (row_dwords / 16) {
         case 4: ND_CQ4(4); break;
         case 5: ND_CQ4(5); break;
         default: ND_CQ4(6); break;
         }
 #undef ND_CQ4
+#undef ND_CQ4_D
         return nd::check_launch("cq_gemv_q4");
     }
     if (stream) {
