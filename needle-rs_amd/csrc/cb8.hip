@@ -629,8 +629,9 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
 // lane-replicated codebook table (entry e, replica r in bank r: conflict-free
 // gathers; both groups' bf16 in one word) straight into MFMA B fragments; a
 // byte dot product forms an entry's address in one operation.  X is rounded to
-// bf16 as it is staged in LDS, double buffered.  Codes are loaded two steps
-// ahead, X three.  Both operands use physical k 16q..16q+7 for the first MFMA
+// bf16 as it is staged in LDS, double buffered.  Codes and X are
+// loaded two steps ahead; Y is stored past the caches (64 rows by 6080 x 512, 64
+// problems: 92 -> 76 us).  Both operands use physical k 16q..16q+7 for the first MFMA
 // of a half step and 16q+8..+15 for the second.  Without LINES a lane's codes
 // come eight at a time, at 8q of each 32 k: for codes aligned to 8 bytes, and
 // with the larger tiles' K order, bit for bit.  Past K (a last step of 32, 64
@@ -638,10 +639,12 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
 // Bound by LDS (gathers and X fragments) at 64 rows, by memory at few.
 // Measured, MI355X, a call (before: four waves of 32 columns, X rounded by a
 // launch of its own; widths not a multiple of 128 in 64x64 tiles): 20 problems
-// of 3072 x 768, 64 rows 23.8 -> 20.8 us, 16 rows 23.5 -> 12.6, 3 rows 22.9 ->
+// of 3072 x 768, 64 rows 22.8 -> 18.3 us, 16 rows 23.5 -> 12.6, 3 rows 22.9 ->
 // 11.9; 24 x 3 rows by 2624 x 2208 62.6 -> 25.3 (5.6 TB/s); 8 x 50 by 768 x
-// 3072 47.4 -> 31.3.  32 columns and half the step a wave: 21.2 and 14.7 for
-// 64 and 16 rows.
+// 3072 47.4 -> 31.3; 64 x 64 rows by 1024 x 3072 77.2 -> 55.1, by 3072 x 768
+// 69.4 -> 59.6, but 448 of these, far past the caches, 418 -> 432 (X rounded
+// beforehand: 422).  32 columns and half the step a wave: 21.2 and 14.7 us
+// for 20 problems of 64 and 16 rows.
 constexpr int kRN = 128;          // output columns (N) per block: two codebook groups
 constexpr int kRC = 128;          // K per step
 constexpr int kRXS = kRC + 8;     // padded X row in LDS (bf16)
@@ -679,8 +682,11 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     auto cload = [&](int slot, int c) {
         if constexpr (LINES) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-                cw[slot][h] = *reinterpret_cast<const u32x4_t *>(wp0 + min(c * kRC + 64 * h + k0, K - 16));
+            for (int h = 0; h < 2; ++h) {
+                // the second read of a line is its last
+                const u32x4_t *p = reinterpret_cast<const u32x4_t *>(wp0 + min(c * kRC + 64 * h + k0, K - 16));
+                cw[slot][h] = h ? __builtin_nontemporal_load(p) : *p;
+            }
         } else {
 #pragma unroll
             for (int h = 0; h < 4; ++h) {
@@ -691,26 +697,25 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
         }
     };
     // X of step c: 16 MT rows x 128, four columns a thread and piece
-    float4 xr[2][MT];
+    float4 xr[MT];
     const int xrow = t >> 5, xcol = (t & 31) * 4;
-    auto xload = [&](int slot, int c) {
+    auto xload = [&](int c) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-            xr[slot][i] = *reinterpret_cast<const float4 *>(X + size_t(min(xrow + 16 * i, M - 1)) * K +
+            xr[i] = *reinterpret_cast<const float4 *>(X + size_t(min(xrow + 16 * i, M - 1)) * K +
                                                             min(c * kRC + xcol, K - 4));
     };
-    auto xstore = [&](int slot, int buf, int c) {
+    auto xstore = [&](int buf, int c) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            const float4 v = xr[slot][i];
+            const float4 v = xr[i];
             uint2 h = make_uint2(f32x2_to_bf16x2_rne(v.x, v.y), f32x2_to_bf16x2_rne(v.z, v.w));
             if (xrow + 16 * i >= M || c * kRC + xcol >= K) h = make_uint2(0, 0);
             *reinterpret_cast<uint2 *>(&xs[buf][(xrow + 16 * i) * kRXS + xcol]) = h;
         }
     };
-    xload(0, 0);
+    xload(0);
     cload(0, 0);
-    xload(1, 1);
     cload(1, 1);
     {
         // the table, through a staging row in xs[1] so every write is
@@ -729,8 +734,8 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
         }
     }
     if (t < 32) tab[256 * 32 + t] = 0;
-    xstore(0, 0, 0);
-    xload(0, 2);
+    xstore(0, 0);
+    xload(1);
     __syncthreads();
     // waves 0-1 hold rows of the first group (low halves), 2-3 the second
     const uint32_t sel = w >= 4 ? 0x07060302u : 0x05040100u;
@@ -763,8 +768,8 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
             const int c = c0 + s;
             if (c < nc) {
                 // X of step c + 1 into the buffer that step c - 1 read
-                xstore(s ^ 1, s ^ 1, c + 1);
-                xload(s ^ 1, c + 3);
+                xstore(s ^ 1, c + 1);
+                xload(c + 2);
                 bf16x8_t b[4];
 #pragma unroll
                 for (int h = 0; h < 4; ++h)
@@ -787,7 +792,7 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int m = 16 * mt + 4 * q + i;
-            if (m < M && col < N) Y[size_t(m) * N + col] = acc[mt][i];
+            if (m < M && col < N) __builtin_nontemporal_store(acc[mt][i], Y + size_t(m) * N + col);
         }
 }
 
