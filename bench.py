@@ -485,7 +485,7 @@ def format_a_runs(torch, nd, steps):
             for tag, exact in (("tolerance_us", False), ("exact_us", True))}
         w.close()
     out["single_call_latency"] = lat
-    # prefill GEMM (matmul_rows_prepared, fp32 MFMA): 512 prepared rows
+    # prefill GEMM (matmul_rows_prepared, f16 matrix cores): 512 prepared rows
     # against the q projection's shape (2-bit) and the LM head's (4-bit)
     gemm = {}
     for name, rows, bits in (("q576x768_2bit", 576, 2), ("lm_head8192x768_4bit", 8192, 4)):
@@ -497,6 +497,7 @@ def format_a_runs(torch, nd, steps):
         ms = timed_loop(torch, lambda: w.matmul_rows_prepared(xh, M, 0, rows, y), max(20, steps), 5)
         tf = 2.0 * M * rows * inn / (ms * 1e-3) / 1e12
         gemm[name + "_m512"] = {"us": round(ms * 1e3, 2), "TFLOPs": round(tf, 2),
+                                "unit": "f16 matrix cores, fp32 operands as two f16 pieces",
                                 "frac_fp32_mfma_peak": round(tf / FP32_MFMA_TFLOPS, 4)}
         w.close()
     out["prefill_gemm_fp32_mfma"] = gemm
@@ -868,7 +869,7 @@ def main():
                 "ms_per_step": round(ms_dec, 4),
                 "attention_GBps": round(att_gbs, 2),
                 "attention_frac_hbm": round(att_gbs / HBM_PEAK_GBS, 4),
-                "attention_traffic_bytes": pmc_traffic("attn_i8_kernel<1,64,64,16>"),
+                "attention_traffic_bytes": pmc_traffic("attn_i8_kernel<64,64>"),
                 "attention_algorithmic_bytes": S * ATT_BYTES,
                 "bytes_per_session_decode": ATT_BYTES,
                 "single_session_attention_us": round(ms_att1 * 1e3, 2),
