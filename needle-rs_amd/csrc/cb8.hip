@@ -392,20 +392,21 @@ __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *
     const unsigned short *cbr = cbh[sr >> 6];
     uint4 xa[4];
     uint2 wc[4];
+    // a 32-column run past K reads the one before it and is zeroed at the LDS
+    // store: no load sits behind a branch
     auto load = [&](int k0) {
         const bool on = k0 + sc < K;
+        const int kc = on ? k0 + sc : K - 32;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            xa[q] = on && mrow ? *reinterpret_cast<const uint4 *>(xrow + k0 + sc + 8 * q)
-                               : make_uint4(0, 0, 0, 0);
+        for (int q = 0; q < 4; ++q) xa[q] = *reinterpret_cast<const uint4 *>(xrow + kc + 8 * q);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            wc[q] = on ? *reinterpret_cast<const uint2 *>(wrow + k0 + sc + 8 * q) : make_uint2(0, 0);
+        for (int q = 0; q < 4; ++q) wc[q] = *reinterpret_cast<const uint2 *>(wrow + kc + 8 * q);
         return on;
     };
     auto store = [&](bool on) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) *reinterpret_cast<uint4 *>(&As[sr][sc + 8 * q]) = xa[q];
+        for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<uint4 *>(&As[sr][sc + 8 * q]) = on && mrow ? xa[q] : make_uint4(0, 0, 0, 0);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const uint32_t d[2] = {wc[q].x, wc[q].y};
