@@ -630,22 +630,23 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
 // lane-replicated codebook table (entry e, replica r in bank r: conflict-free
 // gathers; both groups' bf16 in one word) straight into MFMA B fragments; a
 // byte dot product forms an entry's address in one operation.  X is rounded to
-// bf16 as it is staged in LDS, double buffered.  Codes and X are
-// loaded two steps ahead; Y is stored past the caches (64 rows by 6080 x 512, 64
-// problems: 92 -> 76 us).  Both operands use physical k 16q..16q+7 for the first MFMA
-// of a half step and 16q+8..+15 for the second.  Without LINES a lane's codes
-// come eight at a time, at 8q of each 32 k: for codes aligned to 8 bytes, and
-// with the larger tiles' K order, bit for bit.  Past K (a last step of 32, 64
-// or 96), X is zero and the codes are a zero entry behind the codebook.
+// bf16 as it is staged in LDS, double buffered.  Codes and X are loaded two
+// steps ahead.  Both operands use physical k 16q..16q+7 for the first MFMA of a
+// half step and 16q+8..+15 for the second.  Without LINES a lane's codes come
+// eight at a time, at 8q of each 32 k: for codes aligned to 8 bytes, and with
+// the larger tiles' K order, bit for bit.  Past K (a last step of 32, 64 or
+// 96), X is zero and the codes are a zero entry behind the codebook.
+// Y is stored past the caches (64 problems of 64 rows by 6080 x 512: 92 -> 76
+// us), whole lines through LDS (448 of 64 rows by 3072 x 768: 433 -> 416; half
+// lines were written 1.2 times).
 // Bound by LDS (gathers and X fragments) at 64 rows, by memory at few.
 // Measured, MI355X, a call (before: four waves of 32 columns, X rounded by a
 // launch of its own; widths not a multiple of 128 in 64x64 tiles): 20 problems
 // of 3072 x 768, 64 rows 22.8 -> 18.3 us, 16 rows 23.5 -> 12.6, 3 rows 22.9 ->
 // 11.9; 24 x 3 rows by 2624 x 2208 62.6 -> 25.3 (5.6 TB/s); 8 x 50 by 768 x
 // 3072 47.4 -> 31.3; 64 x 64 rows by 1024 x 3072 77.2 -> 55.1, by 3072 x 768
-// 69.4 -> 59.6, but 448 of these, far past the caches, 418 -> 432 (X rounded
-// beforehand: 422).  32 columns and half the step a wave: 21.2 and 14.7 us
-// for 20 problems of 64 and 16 rows.
+// 69.4 -> 57.6, 448 of these, far past the caches, 422 -> 416.  32 columns and
+// half the step a wave: 21.2 and 14.7 us for 20 problems of 64 and 16 rows.
 constexpr int kRN = 128;          // output columns (N) per block: two codebook groups
 constexpr int kRC = 128;          // K per step
 constexpr int kRXS = kRC + 8;     // padded X row in LDS (bf16)
@@ -755,8 +756,8 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
         uint32_t h[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const uint32_t v0 = *(lds_u32)(__builtin_amdgcn_udot4(dw[k >> 1], 0x80u << (16 * (k & 1)), at, false));
-            const uint32_t v1 = *(lds_u32)(__builtin_amdgcn_udot4(dw[k >> 1], 0x8000u << (16 * (k & 1)), at, false));
+            const uint32_t v0 = *(lds_u32)(uintptr_t(__builtin_amdgcn_udot4(dw[k >> 1], 0x80u << (16 * (k & 1)), at, false)));
+            const uint32_t v1 = *(lds_u32)(uintptr_t(__builtin_amdgcn_udot4(dw[k >> 1], 0x8000u << (16 * (k & 1)), at, false)));
             h[k] = __builtin_amdgcn_perm(v1, v0, sel);
         }
         return __builtin_bit_cast(bf16x8_t, make_uint4(h[0], h[1], h[2], h[3]));
@@ -788,13 +789,23 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
             }
         }
     }
+    // the tile through the table's LDS, so that whole lines are stored: columns
+    // of 16 exchanged by row so that a wave's writes fall on all banks
+    float *yt = reinterpret_cast<float *>(tab);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = 16 * mt + 4 * q + i;
-            if (m < M && col < N) __builtin_nontemporal_store(acc[mt][i], Y + size_t(m) * N + col);
-        }
+        for (int i = 0; i < 4; ++i)
+            yt[(16 * mt + 4 * q + i) * kRN + ((16 * w + r16) ^ (16 * q))] = acc[mt][i];
+    __syncthreads();
+    typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));  // Y is aligned as floats are
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int m = xrow + 16 * i;
+        const f32x4_any_t v = *reinterpret_cast<const f32x4_any_t *>(yt + m * kRN + (xcol ^ (16 * ((m >> 2) & 3))));
+        if (m < M && n0 + xcol < N)
+            __builtin_nontemporal_store(v, reinterpret_cast<f32x4_any_t *>(Y + size_t(m) * N + n0 + xcol));
+    }
 }
 
 int launch_gemv(nd_ctx *ctx, size_t count, const uint8_t *w, size_t w_stride, const float *cb,
