@@ -517,7 +517,7 @@ __global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
             a = fmaxf(a, ndl::wave_xor<32>(a));
             const float qs = a > 0.0f ? a / 127.0f : 1.0f;
             const float inv = 1.0f / qs;
-            float nan = 0.0f;  // NaN where a code is
+            float nan = 0.0f;  // NaN where a code is (an infinite y, of a subnormal scale, has one)
             uint32_t dw[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int e = 0; e < SL; ++e) {
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
                 // the float below a half, for every |y| < 2^22
                 const float y = v[e] * inv;
                 const float r = __builtin_amdgcn_fmed3f(y + copysignf(0.49999997f, y), -128.0f, 127.5f);
-                nan += y * 0.0f;
+                nan = y != y ? y : nan;
                 dw[e >> 2] |= (uint32_t(int32_t(r)) & 0xffu) << (8 * (e & 3));
             }
             nan += ndl::wave_xor<16>(nan);

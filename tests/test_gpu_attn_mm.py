@@ -128,3 +128,25 @@ def test_nan_query_stays_with_its_head(ctx):
                                          dev(np.full(3, 63, np.int32)), dev(q), quant_query=quant))
             bad = np.isnan(out.reshape(3, 12, 64)).all(-1)
             assert bad[1, 7] and bad.sum() == 1 and np.isnan(out).sum() == 64
+
+
+@pytest.mark.parametrize("H,KVH,QK", [(12, 2, 48), (8, 4, 64)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_quantised_query_of_subnormal_scale(ctx, shared, H, KVH, QK):
+    """Heads whose absmax / 127 is subnormal, so that its inverse is infinite:
+    every nonzero element has a code and the head is finite; a zero element
+    (0 * inf) makes its head NaN, no other; a scale that rounds to zero is a
+    query of zeros."""
+    rng = np.random.default_rng(QK + shared)
+    n = 5
+    g, blk, nb = _block(ctx, rng, H, KVH, QK, 64, 64, 1 if shared else n)
+    q = rng.uniform(0.2, 1.0, (n, H, QK)) * rng.choice([-1.0, 1.0], (n, H, QK))
+    q[0] *= 1e-38
+    q[1] *= 3.6e-37
+    q[2, ::2] *= 1e-38
+    q[3] *= 1e-38
+    q[3, 2, 7] = 0.0
+    q[4] *= 5e-44
+    q = q.astype(np.float32)
+    assert np.count_nonzero(q) == q.size - 1
+    _check(ctx, g, blk, nb, [0, 3, 0, 31, 10], [63, 40, 31, 63, 10], q.reshape(n, -1), True, shared)
