@@ -662,12 +662,14 @@ __global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
         if constexpr (QQ) {
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
+                // query scale before K scale: a dot times a large K scale would
+                // overflow where the reference's order, query codes scaled, does not
                 const intx4_t kf{int(kr[a][0]), int(kr[a][1]), int(kr[a][2]), KD == 3 ? 0 : int(kr[a][KD - 1])};
 #pragma unroll
                 for (int x = 0; x < NT; ++x) {
                     const intx4_t d = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qi[x], intx4_t{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s[x][4 * a + i] = (float(d[i]) * ks[a][i]) * cf[x];
+                    for (int i = 0; i < 4; ++i) s[x][4 * a + i] = (float(d[i]) * cf[x]) * ks[a][i];
                 }
             }
         } else {

@@ -21,13 +21,13 @@ pytestmark = pytest.mark.gpu
 TOL = 2e-5
 
 
-def _block(ctx, rng, H, KVH, QK, cap, npos, count=1):
+def _block(ctx, rng, H, KVH, QK, cap, npos, count=1, k_size=1.0):
     """Blocks whose every byte and scale is garbage (NaN) until written."""
     g = nd.kv_geom(H, KVH, QK, 64, cap)
     blk, nb = nd.kv_alloc(g, count)
     blk.fill_(0xff)
     for i in range(count):
-        k = rng.normal(size=(npos, KVH * QK)).astype(np.float32)
+        k = (rng.normal(size=(npos, KVH * QK)) * k_size).astype(np.float32)
         v = rng.normal(size=(npos, KVH * 64)).astype(np.float32)
         # the last `cap` positions only: earlier ones would race for a slot
         p0 = max(0, npos - cap)
@@ -150,3 +150,18 @@ def test_quantised_query_of_subnormal_scale(ctx, shared, H, KVH, QK):
     q = q.astype(np.float32)
     assert np.count_nonzero(q) == q.size - 1
     _check(ctx, g, blk, nb, [0, 3, 0, 31, 10], [63, 40, 31, 63, 10], q.reshape(n, -1), True, shared)
+
+
+@pytest.mark.parametrize("quant", [True])
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("k_size,q_size", [(6e36, 1.6e-37), (3e-34, 3e33)])
+def test_scores_of_unlike_sizes(ctx, shared, quant, k_size, q_size):
+    """Keys near the largest floats against a query near the smallest, and the
+    other way round: N(0, 1) scores whose factors lie far from 1, so a product
+    of two of the three (dot, K scale, query scale) can overflow or lose bits
+    where the reference's order does not."""
+    rng = np.random.default_rng(int(quant) + 2 * int(shared))
+    n = 5
+    g, blk, nb = _block(ctx, rng, 12, 2, 48, 64, 64, 1 if shared else n, k_size=k_size)
+    q = (rng.normal(size=(n, 12 * 48)) * q_size).astype(np.float32)
+    _check(ctx, g, blk, nb, [0, 3, 0, 31, 10], [63, 40, 31, 63, 10], q, quant, shared)
