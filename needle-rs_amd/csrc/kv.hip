@@ -397,7 +397,8 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 //           quant_query the query is int8 codes times one scale a head, so
 //           the dot is an exact integer (i32_16x16x64_i8, no conversion of
 //           K at all); else the fp32 query is three bf16 pieces whose sum is
-//           exactly the query and K's codes are exact in bf16.
+//           exactly the query (scaled by a power of two where it is so small
+//           that they would be subnormal) and K's codes are exact in bf16.
 //   values  O^T[v][col] = V^T P^T: a score tile's result layout (lane = column,
 //           four positions a lane) is the B layout the product needs, so the
 //           weights stay in their lanes, as three bf16 pieces whose sum is
@@ -405,7 +406,8 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 //           takes V columns 4 n + c, so a lane's V bytes come as one dword a
 //           position and no byte is moved between lanes.
 // Every product is exact and the sums are fp32 (or int32): nothing is held in
-// 16 bits.  What bounds it is the VALU work of the softmax (about 22
+// 16 bits.  (A weight's bits below 2^-126, of a value below 2^-119, are lost:
+// they are below a value's last bit where values are 2^-95 or more.)  What bounds it is the VALU work of the softmax (about 22
 // operations a score) and V's conversion (1.5 a byte, shared by the wave's
 // columns); the matrix cores need about a third of the time.
 // Measured, MI355X, against the per-position kernel that took these calls
@@ -533,9 +535,19 @@ __global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
             qi[x] = intx4_t{int(dw[0]), int(dw[1]), int(dw[2]), int(dw[3])};
             cf[x] = qs * scale2 + nan;
         } else {
+            // a bf16 piece has no bit below 2^-126: a head of small values goes
+            // in 2^100 times as large
+            float a = 0.0f;
 #pragma unroll
-            for (int e = 0; e < SL; e += 2) split3(v[e], v[e + 1], qp[x][0][e / 2], qp[x][1][e / 2], qp[x][2][e / 2]);
-            cf[x] = scale2;
+            for (int e = 0; e < SL; e += 2) a = max3(a, __builtin_fabsf(v[e]), __builtin_fabsf(v[e + 1]));
+            a = fmaxf(a, ndl::wave_xor<16>(a));
+            a = fmaxf(a, ndl::wave_xor<32>(a));
+            const bool small = a < 0x1p-100f;
+            const float up = small ? 0x1p100f : 1.0f;
+#pragma unroll
+            for (int e = 0; e < SL; e += 2)
+                split3(v[e] * up, v[e + 1] * up, qp[x][0][e / 2], qp[x][1][e / 2], qp[x][2][e / 2]);
+            cf[x] = small ? scale2 * 0x1p-100f : scale2;
         }
     }
     // the union of the columns' spans (the same in all four lane quarters)
@@ -699,7 +711,7 @@ __global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
                             k0, __builtin_bit_cast(bf16x8_t, u32x4_t{qq[0], qq[1], qq[2], qq[3]}), d, 0, 0, 0);
                     }
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s[x][4 * a + i] = (d[i] * ks[a][i]) * cf[x];
+                    for (int i = 0; i < 4; ++i) s[x][4 * a + i] = (d[i] * cf[x]) * ks[a][i];
                 }
             }
         }

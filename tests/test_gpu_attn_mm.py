@@ -152,14 +152,14 @@ def test_quantised_query_of_subnormal_scale(ctx, shared, H, KVH, QK):
     _check(ctx, g, blk, nb, [0, 3, 0, 31, 10], [63, 40, 31, 63, 10], q.reshape(n, -1), True, shared)
 
 
-@pytest.mark.parametrize("quant", [True])
+@pytest.mark.parametrize("quant", [False, True])
 @pytest.mark.parametrize("shared", [False, True])
 @pytest.mark.parametrize("k_size,q_size", [(6e36, 1.6e-37), (3e-34, 3e33)])
 def test_scores_of_unlike_sizes(ctx, shared, quant, k_size, q_size):
     """Keys near the largest floats against a query near the smallest, and the
     other way round: N(0, 1) scores whose factors lie far from 1, so a product
-    of two of the three (dot, K scale, query scale) can overflow or lose bits
-    where the reference's order does not."""
+    of two of the three (dot, K scale, query scale) can overflow, or a small
+    query's pieces lose bits, where the reference's order does not."""
     rng = np.random.default_rng(int(quant) + 2 * int(shared))
     n = 5
     g, blk, nb = _block(ctx, rng, 12, 2, 48, 64, 64, 1 if shared else n, k_size=k_size)
