@@ -647,6 +647,9 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
 // 3072 47.4 -> 31.3; 64 x 64 rows by 1024 x 3072 77.2 -> 55.1, by 3072 x 768
 // 69.4 -> 57.6, 448 of these, far past the caches, 422 -> 416.  32 columns and
 // half the step a wave: 21.2 and 14.7 us for 20 problems of 64 and 16 rows.
+// Blocks of 512 threads a launch may have: HIP counts the threads of a dimension
+// in 32 bits, and a launch of more leaves blocks out.
+constexpr size_t kMaxBlocks512 = 0xffffffffu / 512;
 constexpr int kRN = 128;          // output columns (N) per block: two codebook groups
 constexpr int kRC = 128;          // K per step
 constexpr int kRXS = kRC + 8;     // padded X row in LDS (bf16)
@@ -892,8 +895,8 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
     const size_t row_tiles_m = (m + 63) / 64;
     const size_t row_tiles = ((out + kRN - 1) / kRN) * row_tiles_m * count;
     const bool lines = m <= 64 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && w_stride % 16 == 0;
-    const bool use_rows = (m <= 64 || row_tiles <= 2 * cus) && row_tiles <= 0x7fffffff;
-    const bool use_256 = !use_rows && m >= 96 && out % kPN == 0 && big_tiles >= cus && big_tiles <= 0x7fffffff;
+    const bool use_rows = m <= 64 || row_tiles <= 2 * cus;
+    const bool use_256 = !use_rows && m >= 96 && out % kPN == 0 && big_tiles >= cus && big_tiles <= kMaxBlocks512;
     // X to bf16 once per call, into the context workspace, for the kernels
     // that stage bf16 X; the 256x256 and the row kernel round fp32 X as they
     // stage it
@@ -908,19 +911,28 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
         if (int rc = nd::check_launch("x_to_bf16")) return rc;
     }
     if (use_rows) {
-        const int run = row_tiles % 8 == 0 ? int(row_tiles / 8) : 0;
-#define ND_GEMM_ROWS(MT, LINES)                                                                     \
-    hipLaunchKernelGGL((cb8_gemm_rows_kernel<MT, LINES>), dim3(unsigned(row_tiles)), dim3(512), 0, ctx->stream, x, \
-                       x_stride, w, cb, y, int(m), int(out), int(in), w_stride, cb_stride, y_stride,    \
-                       int((out + kRN - 1) / kRN), int(row_tiles_m), run)
-        if (!lines)
-            ND_GEMM_ROWS(4, false);
-        else if (m <= 16)
-            ND_GEMM_ROWS(1, true);
-        else if (m <= 32)
-            ND_GEMM_ROWS(2, true);
-        else
-            ND_GEMM_ROWS(4, true);
+        // one launch, or as many problems a launch as its grid may hold (a
+        // problem has 2^17 tiles at most)
+        const size_t tiles_n = (out + kRN - 1) / kRN, tiles = tiles_n * row_tiles_m;
+        const size_t most = kMaxBlocks512 / tiles;
+        for (size_t z0 = 0; z0 < count; z0 += most) {
+            const size_t blocks = (count - z0 < most ? count - z0 : most) * tiles;
+            const int run = blocks % 8 == 0 ? int(blocks / 8) : 0;
+#define ND_GEMM_ROWS(MT, LINES)                                                                         \
+    hipLaunchKernelGGL((cb8_gemm_rows_kernel<MT, LINES>), dim3(unsigned(blocks)), dim3(512), 0, ctx->stream, \
+                       x + z0 * x_stride, x_stride, w + z0 * w_stride, cb + z0 * cb_stride,             \
+                       y + z0 * y_stride, int(m), int(out), int(in), w_stride, cb_stride, y_stride,     \
+                       int(tiles_n), int(row_tiles_m), run)
+            if (!lines)
+                ND_GEMM_ROWS(4, false);
+            else if (m <= 16)
+                ND_GEMM_ROWS(1, true);
+            else if (m <= 32)
+                ND_GEMM_ROWS(2, true);
+            else
+                ND_GEMM_ROWS(4, true);
+            if (int rc = nd::check_launch("cb8_gemm")) return rc;
+        }
 #undef ND_GEMM_ROWS
     } else if (use_256) {
         // at least one 256x256 tile per CU: below that the 128x128 tiles fill

@@ -295,3 +295,25 @@ def test_gemm_codes_aligned_to_eight_bytes(ctx):
     v = torch.gather(CB.bfloat16().double().repeat_interleave(64, 0), 1, W.long())
     x = X.bfloat16().double()
     assert torch.all((y - x @ v.T).abs() <= (x.abs() @ v.abs().T) * inn * 2.0 ** -23)
+
+
+def test_gemm_more_tiles_than_a_launch_holds(ctx):
+    """65,535 one-row problems over one weight of 129 column tiles: 8,454,015
+    row tiles, more than a grid of 512-thread blocks may have (8,388,607).
+    Problems on both sides of the cut have the bits of a call of their own,
+    and every one is within 32 roundings of the bf16 operands' product."""
+    count, out, inn = 65535, 129 * 128, 32
+    g = torch.Generator(device="cuda").manual_seed(9)
+    W = torch.randint(0, 256, (out, inn), generator=g, dtype=torch.uint8, device="cuda")
+    CB = torch.randn(out // 64, 256, generator=g, device="cuda") * 0.02
+    X = torch.randn(count, inn, generator=g, device="cuda")
+    Y = torch.full((count, out), 7.0, device="cuda")
+    nd._check(nd.lib().nd_cb8_gemm_batched(ctx.h, count, X.data_ptr(), inn, W.data_ptr(), 0, CB.data_ptr(), 0,
+                                           Y.data_ptr(), out, 1, out, inn))
+    cut = 8388607 // 129
+    for z in (0, cut - 1, cut, count - 1):
+        assert torch.equal(nd.cb8_gemm(ctx, X[z:z + 1], W, CB)[0], Y[z])
+    v = torch.gather(CB.bfloat16().double().repeat_interleave(64, 0), 1, W.long())
+    for z in range(0, count, 2048):
+        x = X[z:z + 2048].bfloat16().double()
+        assert torch.all((Y[z:z + 2048].double() - x @ v.T).abs() <= (x.abs() @ v.abs().T) * inn * 2.0 ** -23)
