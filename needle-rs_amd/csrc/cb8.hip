@@ -168,15 +168,15 @@ __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_kernel(
     if ((j & 3) == 0 && r < out) y[r] = s;
 }
 
-// Any `in` (multiple of 16).  Eight lanes share a row (128 contiguous bytes a
-// load; a wave's 16 rows take P = 2 passes), a step is U = 4 vectors of 16
-// codes a lane and row: eight loads of 16 bytes in flight, and the next step's
-// are issued before the current one's gathers.  The part step at a row's end
-// goes first, its loads together with the first full step's: a vector past the
-// end is read as the last one and left out of the sum.  The activations sit in
-// LDS, the quads of a vector rotated by its index so that the lanes' reads of
-// one quad fall on different banks; eight lanes a row read each once for two
-// rows.
+// Any `in` (multiple of 16).  L lanes share a row, a wave's 64 / L rows of a pass
+// take P passes; a step is U = 4 vectors of 16 codes a lane and row, and the
+// next step's are issued before the current one's gathers.  L = 8, P = 2: 128
+// contiguous bytes a row and load, eight loads of 16 bytes in flight.  The part
+// step at a row's end goes first, its loads together with the first full step's:
+// a vector past the end is read as the last one and left out of the sum.  The
+// activations sit in LDS, the quads of a vector rotated by its index so that the
+// lanes' reads of one quad fall on different banks; eight lanes a row read each
+// once for two rows.
 // Bound by HBM on stacks of wide rows, by filling the table for a tile on
 // narrow ones.  Measured, MI355X, stacks of 300 MB, codes' GB/s (before: one
 // load in flight a lane; 16 lanes a row): in = 64: 2289 (1122), 128: 3960
@@ -184,12 +184,18 @@ __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_kernel(
 // (1996), 4096: 5509 (1750).  Four lanes a row gain on 64 (2753) and lose
 // elsewhere (4124 at 1040); 16 gain on 208 to 400 (12 % at most) and lose
 // elsewhere (3701 at 4096).
+// A problem of few rows has only its lanes to share the work, and rows past the
+// end would repeat the last one's: 16 lanes a row up to 16 rows, a wave a row up
+// to four.  us, eight lanes / so: 1 x 16 rows by 8000 25.3 / 9.3, by 16384 48.7 /
+// 16.0; 2000 x 5 by 784 15.2 / 8.5; 1 x 3 by 16384 48.7 / 6.8 (16 lanes 15.8);
+// 2000 x 4 by 4112 56.8 / 18.1 (24.7).
+template <int L, int P>
 __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_any_kernel(
     const uint8_t *__restrict__ w, size_t w_stride, const float *__restrict__ cb,
     size_t cb_stride, const float *__restrict__ x, size_t x_stride, float *__restrict__ y,
     size_t y_stride, int out, int in)
 {
-    constexpr int L = 8, P = 2, U = 4, R = 64 / L;
+    constexpr int U = 4, R = 64 / L;
     __shared__ float4 rep4[256 * 32 / 4];  // 32 KB
     extern __shared__ float4 xs4[];        // [in / 4]
     const size_t prob = blockIdx.y;
@@ -198,7 +204,7 @@ __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_any_kernel(
     x += prob * x_stride;
     y += prob * y_stride;
     const int t = threadIdx.x, lane = t & 63, j = lane & (L - 1);
-    const int row0 = blockIdx.x * kTileRows + (t >> 6) * 16 + lane / L;
+    const int row0 = blockIdx.x * kTileRows + (t >> 6) * (R * P) + lane / L;
     const int nvec = in >> 4;
 
     const u32x4_t *wr[P];
@@ -235,7 +241,7 @@ __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_any_kernel(
     __syncthreads();
 
     const float *cbl = reinterpret_cast<const float *>(rep4) + (lane & 31);
-    float acc[P][8] = {};  // 64 partial sums a row
+    float acc[P][8] = {};  // 8 L partial sums a row
     auto block = [&](const u32x4_t (&c)[P][U], int u, int v) {
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
@@ -266,6 +272,11 @@ __global__ __launch_bounds__(kThreads, 4) void cb8_gemv_any_kernel(
     for (int p = 0; p < P; ++p) {
         float s = ((acc[p][0] + acc[p][1]) + (acc[p][2] + acc[p][3])) +
                   ((acc[p][4] + acc[p][5]) + (acc[p][6] + acc[p][7]));
+        if constexpr (L == 64) {
+            s += ndl::wave_xor<32>(s);
+            s += ndl::wave_xor<16>(s);
+        }
+        if constexpr (L >= 16) s += ndl::wave_xor<8>(s);
         s += ndl::wave_xor<4>(s);
         s += ndl::wave_xor<2>(s);
         s += ndl::wave_xor<1>(s);
@@ -840,8 +851,16 @@ int launch_gemv(nd_ctx *ctx, size_t count, const uint8_t *w, size_t w_stride, co
         }
     } else {
         ND_REQUIRE(in * sizeof(float) <= 64 * 1024, "in (%zu) too large", in);
-        hipLaunchKernelGGL(cb8_gemv_any_kernel, grid, dim3(kThreads), in * sizeof(float), ctx->stream, w,
-                           w_stride, cb, cb_stride, x, x_stride, y, y_stride, int(out), int(in));
+#define ND_GEMV_ANY(L, P)                                                                             \
+    hipLaunchKernelGGL((cb8_gemv_any_kernel<L, P>), grid, dim3(kThreads), in * sizeof(float), ctx->stream, w, \
+                       w_stride, cb, cb_stride, x, x_stride, y, y_stride, int(out), int(in))
+        if (out <= 4)
+            ND_GEMV_ANY(64, 1);
+        else if (out <= 16)
+            ND_GEMV_ANY(16, 1);
+        else
+            ND_GEMV_ANY(8, 2);
+#undef ND_GEMV_ANY
     }
 #undef ND_GEMV
     return nd::check_launch("cb8_gemv");

@@ -42,10 +42,12 @@ def test_gemv_ragged(ctx, out, inn):
 
 @pytest.mark.parametrize("count,out,inn", [(3, 1, 16), (2, 64, 112), (5, 65, 128), (2, 81, 496),
                                            (1, 130, 512), (2, 17, 528), (1, 100, 1008), (1, 64, 1536),
-                                           (2, 33, 2064), (1, 3, 16384)])
+                                           (2, 33, 2064), (1, 3, 16384), (2, 4, 4112), (3, 1, 4096),
+                                           (1, 2, 16368), (2, 5, 1040), (3, 16, 2064), (1, 16, 1008),
+                                           (2, 13, 48), (1, 17, 4096)])
 def test_gemv_part_steps(ctx, count, out, inn):
-    """Widths around the steps of 512 columns and their parts of 128, ragged
-    rows, padded strides; within inn rounding errors of the sum's magnitude
+    """Widths around the steps of 512 columns and their parts of 128 (1024 and
+    4096 for up to 16 and 4 rows), ragged rows, padded strides; within inn rounding errors of the sum's magnitude
     of the 64-bit result, and an infinite entry of an unused code stays out."""
     rng = np.random.default_rng(out + inn)
     tiles = (out + 63) // 64
