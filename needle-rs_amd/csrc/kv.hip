@@ -450,7 +450,7 @@ __device__ inline void split3(float x0, float x1, uint32_t &h, uint32_t &m, uint
 }
 
 template <int QK, bool QQ, int NT, int NW, bool SHARED>
-__global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
+__global__ __launch_bounds__(NW * 64, NT == 1 ? 4 : 1) void attn_mm_kernel(
     Geom g, const uint8_t *__restrict__ kv, size_t kv_stride, const int32_t *__restrict__ lo_a,
     const int32_t *__restrict__ hi_a, const float *__restrict__ q, float scale2, int rows, int splits,
     float *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml)
@@ -537,17 +537,20 @@ __global__ __launch_bounds__(NW * 64) void attn_mm_kernel(
         } else {
             // a bf16 piece has no bit below 2^-126: a head of small values goes
             // in 2^100 times as large
+            cf[x] = scale2;
             float a = 0.0f;
 #pragma unroll
-            for (int e = 0; e < SL; e += 2) a = max3(a, __builtin_fabsf(v[e]), __builtin_fabsf(v[e + 1]));
-            a = fmaxf(a, ndl::wave_xor<16>(a));
-            a = fmaxf(a, ndl::wave_xor<32>(a));
-            const bool small = a < 0x1p-100f;
-            const float up = small ? 0x1p100f : 1.0f;
+            for (int e = 0; e < SL; ++e) a += __builtin_fabsf(v[e]);
+            if (__any(a < 0x1p-100f)) {
+                a += ndl::wave_xor<16>(a);
+                a += ndl::wave_xor<32>(a);
+                const bool small = a < 0x1p-100f;
+                if (small) cf[x] = scale2 * 0x1p-100f;
 #pragma unroll
-            for (int e = 0; e < SL; e += 2)
-                split3(v[e] * up, v[e + 1] * up, qp[x][0][e / 2], qp[x][1][e / 2], qp[x][2][e / 2]);
-            cf[x] = small ? scale2 * 0x1p-100f : scale2;
+                for (int e = 0; e < SL; ++e) v[e] *= small ? 0x1p100f : 1.0f;
+            }
+#pragma unroll
+            for (int e = 0; e < SL; e += 2) split3(v[e], v[e + 1], qp[x][0][e / 2], qp[x][1][e / 2], qp[x][2][e / 2]);
         }
     }
     // the union of the columns' spans (the same in all four lane quarters)
