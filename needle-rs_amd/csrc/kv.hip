@@ -1089,8 +1089,9 @@ int attend_i8(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride
         // blocks below 8 waves a CU (64 sessions x 2 heads x 512: 7.4 against
         // 9.7 us with four waves and a merge launch), 4-wave blocks above
         // (256 x 2 x 1024: 15.3 against 17.3); no split leaves a wave without
-        // a chunk
-        const bool deep = pairs * 4 < cus * 8;
+        // a chunk, and a ring of up to four chunks has none for more waves
+        // (172 x 2 heads x 8 positions 10.2 against 8.8 us)
+        const bool deep = pairs * 4 < cus * 8 && g->cap > 128;
         const size_t nw = deep ? 16 : 4;
         const size_t fill = (cus * 8 + pairs * nw - 1) / (pairs * nw);
         const size_t most = (size_t(g->cap) + 32 * nw - 1) / (32 * nw);

@@ -89,3 +89,41 @@ def test_not_finite(ctx, bits):
             assert np.array_equal(got[r], want[r].astype(np.float32), equal_nan=True)
         else:
             assert np.all(np.abs(got[r] - want[r]) <= TOL * (np.abs(xh[r]).astype(np.float64) @ np.abs(w).T))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, TERNARY])
+@pytest.mark.parametrize("out,inn,group,batch", [(300, 768, 128, 70), (130, 700, 256, 5), (4100, 512, 512, 130),
+                                                 (8192, 256, 128, 200)])
+def test_rows_that_are_not_finite(ctx, bits, out, inn, group, batch):
+    """Infinities of one sign and both, across groups, in the last column, whole
+    groups of them, and NaN: the infinities and NaN of the product in 64 bits;
+    the finite rows beside them keep their bits."""
+    rng = np.random.default_rng(out + bits)
+    c = random_case(rng, out, inn, group, bits, CB)
+    gw = _weight(ctx, c)
+    xh = rng.normal(size=(batch, c.in_pad)).astype(np.float32)
+    run = lambda: host(gw.matmul_rows_prepared(dev(xh), batch, 0, out)).reshape(batch, out)
+    finite = run()
+    last, far = c.in_pad - 1, min(group + 3, c.in_pad - 2)
+    xh[0, 7] = np.inf
+    xh[1, last] = -np.inf
+    xh[2, [5, far]] = np.inf
+    xh[3, [5, far]] = np.inf, -np.inf
+    xh[4, far] = np.nan
+    odd = [0, 1, 2, 3, 4]
+    if batch > 5:
+        xh[17, :128] = np.where(rng.random(128) < 0.5, np.inf, -np.inf)
+        xh[batch - 1, last - 127:] = np.inf
+        odd += [17, batch - 1]
+    got = run()
+    w = _weights64(c)
+    with np.errstate(invalid="ignore"):
+        want = xh[odd].astype(np.float64)[:, None, :] * w[None] if out * c.in_pad < 300000 else None
+        if want is not None:
+            want = want.sum(-1)
+        else:  # the elements that are not finite decide
+            want = np.stack([(xh[r].astype(np.float64)[k] * w[:, k]).sum(-1)
+                             for r in odd for k in [~np.isfinite(xh[r])]])
+    assert np.array_equal(got[odd], want.astype(np.float32), equal_nan=True)
+    rest = np.setdiff1d(np.arange(batch), odd)
+    assert np.array_equal(got[rest].view(np.uint32), finite[rest].view(np.uint32))
