@@ -1090,7 +1090,7 @@ int attend_i8(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride
         // 9.7 us with four waves and a merge launch), 4-wave blocks above
         // (256 x 2 x 1024: 15.3 against 17.3); no split leaves a wave without
         // a chunk, and a ring of up to four chunks has none for more waves
-        // (172 x 2 heads x 8 positions 10.2 against 8.8 us)
+        // (172 x 2 heads x 8 positions: 10.5 us with 16 waves, 5.8 so)
         const bool deep = pairs * 4 < cus * 8 && g->cap > 128;
         const size_t nw = deep ? 16 : 4;
         const size_t fill = (cus * 8 + pairs * nw - 1) / (pairs * nw);

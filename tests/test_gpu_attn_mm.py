@@ -60,6 +60,7 @@ def _check(ctx, g, blk, nb, lo, hi, q, quant, shared):
 @pytest.mark.parametrize("H,KVH,QK", [(12, 2, 48), (16, 2, 64), (6, 2, 64), (8, 2, 48), (4, 2, 48)])
 @pytest.mark.parametrize("cap,spans", [
     (1, [(0, 0)]), (17, [(0, 16), (20, 36), (3, 3)]), (31, [(40, 70), (69, 70)]), (32, [(33, 64), (64, 64)]),
+    (128, [(0, 127), (100, 227), (127, 127)]), (129, [(0, 128), (100, 228), (5, 36)]),
     (2048, [(0, 2047), (1, 33), (100, 131), (2040, 2047)]), (1000, [(500, 1499), (999, 1001), (1480, 1499)])])
 def test_decode_grouped(ctx, H, KVH, QK, cap, spans, quant):
     """One row a block: ragged spans, wrapped rings, rings below a chunk."""
