@@ -307,8 +307,8 @@ __global__ __launch_bounds__(kThreads) void cq_gemv_stream_kernel(
 // nontemporal) every CAP tiles and at the end: a global store inside the
 // loop would put its write round trip under the next wait.  Rows past the
 // end reread the last row; the loop body has no branches.
-// A launch of one or two tiles a workgroup (rows up to 16384 at 2 bits, 16384
-// and 32768 at 4) holds just those: the pipeline of four computed and reread
+// A launch of one or two tiles a workgroup (on 256 CUs rows up to 32768 and
+// 65536 at 2 bits, 16384 and 32768 at 4) holds just those: the pipeline of four computed and reread
 // the last tile for each it did not have.  With the table of the 4-bit kernel
 // filled from one load a thread, one row by 8192 x 768 took 7.4 -> 5.0 us at 2
 // bits and 8.6 -> 5.0 at 4, by 16384 x 768 7.6 -> 5.2 and 13.0 -> 7.3.
@@ -1267,14 +1267,17 @@ __global__ __launch_bounds__(256) void cq_matmul_b_kernel(
 // multiples of 128, any width.
 //
 // An fp32 value times a power of two is h + l, two f16 values, to within
-// 2^-24 of itself (h keeps 11 bits, l the next 11 and its sign one more), so
-// x . lv = xh lh + xh ll + xl lh plus a term below 2^-24 of it: three f16
-// MFMAs in place of sixteen-fold slower fp32 ones, products exact, sums
-// fp32.  The activations are scaled by a power of two per (row, 128 columns)
-// and the levels by one per weight so that h uses f16's top binade; the
-// scales go back exactly, with the norm, once per 128 columns.  Against 64
-// bits the result is closer than the fp32 MFMA kernel's was (1.0e-7 against
-// 5.0e-7 at in 768: a sum of 32-wide dots is a shorter chain).
+// 2^-23 of itself (h keeps 11 bits, l the next 11 and its sign one more: a
+// quarter of all values are half a last bit off), so x . lv = xh lh + xh ll +
+// xl lh plus a term below 2^-22 of it: three f16 MFMAs in place of sixteen-fold
+// slower fp32 ones, their products exact, sums fp32.  The activations are scaled
+// by a power of two per (row, 128 columns) and the levels by one per weight so
+// that h uses f16's top binade; the scales go back exactly, with the norm, once
+// per 128 columns.  A piece ends at 2^-24 there, so a value far below its
+// group's largest is carried to 2^-39 of that (what a Hadamard transform leaves
+// in fp32 has lost more).  A product has fewer bits than in fp32; the result of
+// N(0, 1) rows is closer to 64 bits than the fp32 MFMA kernel's was (1.7e-7
+// against 5.0e-7 at in 768: sums of 32-wide dots are a shorter chain).
 //
 // Block: 16 MT batch rows x 16 NL weight rows a wave, NW waves side by side
 // along the weight rows, 128 columns a step.  X is split once per block into

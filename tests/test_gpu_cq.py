@@ -158,6 +158,31 @@ def test_matvec_streams_past_the_stage(ctx, bits):
     g.close()
 
 
+@pytest.mark.parametrize("bits,inn", [(2, 256), (2, 512), (2, 768), (TERNARY, 768), (4, 512), (4, 640), (4, 768)])
+def test_matvec_held_tiles(ctx, bits, inn):
+    """One, two and more tiles a workgroup (32,768 and 65,536 rows at 2 bits
+    and ternary, half as many at 4, on 256 CUs): row counts on both sides of
+    each change, from an odd row, bit for bit what the tallest launch gives
+    those rows, and that against the oracle."""
+    rng = np.random.default_rng(inn + bits)
+    width = 2 if bits == TERNARY else bits
+    edge = 32768 if width == 2 else 16384
+    out = 2 * edge + 600
+    packed = rng.integers(0, 256, size=out * inn * width // 8, dtype=np.uint8)
+    norms = (np.abs(rng.normal(0.0, 0.02, size=out * (inn // 128))) * np.sqrt(128.0))
+    blob = np.concatenate([packed, norms.astype(np.float16).view(np.uint8)])
+    g = nd.CqWeight(ctx, blob, out, inn, 128, bits, REAL_CB)
+    o = O.CqWeight(blob, out, inn, 128, bits, REAL_CB)
+    x = rng.normal(size=inn).astype(np.float32)
+    xh = g.prepare_input(dev(x))[0]
+    y = host(g.matvec_prepared(xh))
+    assert _close(y, o.matvec(x))
+    for rows in (1, 33, 64, edge - 1, edge, edge + 1, 2 * edge - 1, 2 * edge, 2 * edge + 1):
+        band = host(g.matvec_rows_prepared(xh, 5, rows))
+        assert np.array_equal(band.view(np.uint32), y[5:5 + rows].view(np.uint32)), rows
+    g.close()
+
+
 # A 2-bit slot that is neither monotone nor symmetric: the fp4 kernel's
 # plane coefficients are solved from the four levels, whatever they are.
 SKEW_CB = REAL_CB.copy()

@@ -1,11 +1,12 @@
 """The f16 matrix-core Cactus-Quants matmul at its tile edges, against the
 same product in 64 bits.
 
-Tolerance: both operands are carried to 2^-24 of themselves and one cross
-term below 2^-24 of the product is left out; a product sum adds at most 96
-fp32 roundings in a step of 32 columns' three products and one a step and a
-group after it.  Rounding errors of either sign add as their square root: 16
-units of 2^-24 of sum |x w| bound every draw here by a factor of ten or more.
+Tolerance: both operands are carried to 2^-23 of themselves and the cross term
+left out is below 2^-22 of the product: 2^-21 of it in all, 8 units of 2^-24, in
+the worst case.  A product sum adds at most 96 fp32 roundings in a step of 32
+columns' three products and one a step and a group after it; errors of either
+sign add as their square root.  16 units of sum |x w| bound every draw here: by
+a factor of two where one product makes most of a sum, of ten or more elsewhere.
 """
 import numpy as np
 import pytest
@@ -127,3 +128,22 @@ def test_rows_that_are_not_finite(ctx, bits, out, inn, group, batch):
     assert np.array_equal(got[odd], want.astype(np.float32), equal_nan=True)
     rest = np.setdiff1d(np.arange(batch), odd)
     assert np.array_equal(got[rest].view(np.uint32), finite[rest].view(np.uint32))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, TERNARY])
+@pytest.mark.parametrize("size", [2.0 ** 10, 2.0 ** 17, 2.0 ** 24, 2.0 ** 31])
+def test_one_large_value_in_a_group(ctx, bits, size):
+    """A piece ends at 2^-24 where a group's largest activation is 2^14 to
+    2^15: an element is carried to 2^-23 of itself or to 2^-39 of its group's
+    largest, whichever is more, and it shows where the largest meets a level of
+    zero."""
+    rng = np.random.default_rng(bits)
+    c = random_case(rng, 300, 512, 128, bits, CB)
+    xh = rng.normal(size=(40, 512)).astype(np.float32)
+    xh[:, [3, 200, 300, 400]] *= np.float32(size)
+    got = host(_weight(ctx, c).matmul_rows_prepared(dev(xh), 40, 0, 300)).reshape(40, 300)
+    w, x = _weights64(c), xh.astype(np.float64)
+    want, mag = x @ w.T, np.abs(x) @ np.abs(w).T
+    top = np.abs(x).reshape(40, 4, 128).max(-1)
+    floor = top @ np.abs(w).reshape(300, 4, 128).sum(-1).T
+    assert np.all(np.abs(got - want) <= TOL * mag + 2.0 ** -39 * floor)
