@@ -651,13 +651,16 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
 // us), whole lines through LDS (448 of 64 rows by 3072 x 768: 433 -> 416; half
 // lines were written 1.2 times).
 // Bound by LDS (gathers and X fragments) at 64 rows, by memory at few.
-// Measured, MI355X, a call (before: four waves of 32 columns, X rounded by a
-// launch of its own; widths not a multiple of 128 in 64x64 tiles): 20 problems
-// of 3072 x 768, 64 rows 22.8 -> 18.3 us, 16 rows 23.5 -> 12.6, 3 rows 22.9 ->
-// 11.9; 24 x 3 rows by 2624 x 2208 62.6 -> 25.3 (5.6 TB/s); 8 x 50 by 768 x
-// 3072 47.4 -> 31.3; 64 x 64 rows by 1024 x 3072 77.2 -> 55.1, by 3072 x 768
-// 69.4 -> 57.6, 448 of these, far past the caches, 422 -> 416.  32 columns and
-// half the step a wave: 21.2 and 14.7 us for 20 problems of 64 and 16 rows.
+// Measured, MI355X, calls back to back (before: four waves of 32 columns, X
+// rounded by a launch of its own; widths not a multiple of 128 in 64x64 tiles):
+// 20 problems of 3072 x 768, 64 rows 23.9 -> 19.5 us, 16 rows 23.4 -> 12.6, 3
+// rows 22.7 -> 12.1; 24 x 3 rows by 2624 x 2208 62.9 -> 25.0 (5.6 TB/s); 8 x 50
+// by 768 x 3072 48.9 -> 30.5; 64 x 64 rows by 1024 x 3072 78.0 -> 59.0, by 3072
+// x 768 63.3 -> 51.0, 448 of these, far past the caches, 409 -> 405.  32 columns
+// and half the step a wave: 21.2 and 14.7 us for 20 problems of 64 and 16 rows.
+// A tile fills a table of 32 KB first, which a K of 32 to 128 does not repay
+// once a launch has thousands of tiles: 200 x 64 rows by 1984 x 32 25.6 -> 31,
+// 2000 x 1 by 192 x 128 24.2 -> 28.
 // Blocks of 512 threads a launch may have: HIP counts the threads of a dimension
 // in 32 bits, and a launch of more leaves blocks out.
 constexpr size_t kMaxBlocks512 = 0xffffffffu / 512;
@@ -753,15 +756,13 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     xstore(0, 0);
     xload(1);
     __syncthreads();
-    // waves 0-1 hold rows of the first group (low halves), 2-3 the second
+    // waves 0-3 hold rows of the first group (low halves), 4-7 the second
     const uint32_t sel = w >= 4 ? 0x07060302u : 0x05040100u;
     typedef __attribute__((address_space(3))) uint32_t *lds_u32;
     const uint32_t base = uint32_t(reinterpret_cast<uintptr_t>((lds_u32)(tab + (lane & 31))));
     floatx4_t acc[MT];
 #pragma unroll
     for (int a = 0; a < MT; ++a) acc[a] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    // one dot product of bytes makes an entry's address; 16 codes past the end
-    // are the zero entry
     // one dot product of bytes makes an entry's address; codes past the end
     // are the zero entry
     auto decode = [&](uint32_t d0, uint32_t d1, bool in) {
@@ -908,8 +909,11 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
     // shorter there (us, rows / 128x128 tiles: 192 tiles of 1 x 512 by 3072 x
     // 768 14.0 / 22.1, 384 of 8 x 500 by 768 x 768 23.9 / 29.2, 512 of 4 x 1000
     // by 1024 x 256 14.5 / 15.6, 720 of 6 x 300 by 3072 x 768 34.7 / 33.1, 960
-    // of 20 x 80 by 3072 x 768 46.2 / 32.7).  Whole lines of codes need them
-    // 16-byte aligned.  Above 64 rows the K order is the larger tiles', so a
+    // of 20 x 80 by 3072 x 768 46.2 / 32.7).  (One to three groups of 64 columns
+    // leave up to half a 128x128 tile idle; 64x64 tiles would do 200 x 130 rows
+    // by 64 x 768 in 38.6 us against 42.6 and 64 x 2000 by 64 x 96 in 25.4
+    // against 27.8, not worth a kernel.)  Whole lines of codes need them 16-byte
+    // aligned.  Above 64 rows the K order is the larger tiles', so a
     // problem's bits do not depend on how many share its launch.
     const size_t row_tiles_m = (m + 63) / 64;
     const size_t row_tiles = ((out + kRN - 1) / kRN) * row_tiles_m * count;

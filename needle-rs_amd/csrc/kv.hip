@@ -7,11 +7,12 @@
 // round-half-away-from-zero as libm::roundf.  One wave per head vector.
 //
 // Attention (attend_step over Int8View, attention.rs:300-377) reads the int8
-// cache directly: a workgroup owns (query, kv head) -- every query head of
-// the GQA group, so a kv head's int8 rows are read once for all of them --
-// and walks its span in chunks with an online softmax (flash decoding).  The
-// span is split across workgroups, with a merge pass, only when there are
-// too few (query, kv head) pairs to fill the GPU (batch-1 decode).
+// cache directly, in chunks with an online softmax (flash decoding).  One query
+// head a kv head: attn_i8_kernel, a workgroup a (query, kv head).  Two or more,
+// and the rows of a prompt over one cache: attn_mm_kernel, on the matrix cores,
+// a wave 16 or 32 (row, head) columns of a kv head, so its int8 rows are read
+// once for all of them.  The span is split across workgroups, with a merge
+// pass, only when there are too few of them to fill the GPU (batch-1 decode).
 #include "nd_internal.h"
 #include "nd_kv_internal.h"
 
@@ -407,17 +408,23 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 //           position and no byte is moved between lanes.
 // Every product is exact and the sums are fp32 (or int32): nothing is held in
 // 16 bits.  (A weight's bits below 2^-126, of a value below 2^-119, are lost:
-// they are below a value's last bit where values are 2^-95 or more.)  What bounds it is the VALU work of the softmax (about 22
-// operations a score) and V's conversion (1.5 a byte, shared by the wave's
-// columns); the matrix cores need about a third of the time.
-// Measured, MI355X, against the per-position kernel that took these calls
-// before (K and V converted to fp32 and multiplied in the VALU for each query
-// head; a prompt's rows each walked their own span):
-//   prompt, 12 on 2 heads, qk 48, quant_query: 1000 rows 78 -> 12.7 us, 2000
-//   234 -> 29, 3000 470 -> 53 (12 x 64 MHA: 123 / 384 / 788 -> 13 / 29 / 50)
-//   decode, 12 on 2 heads: 64 sessions x 2048 29.6 -> 11.0 us, 256 x 1024
-//   41.4 -> 12.6, one session x 8192 24.7 -> 10.2; 8 on 4: 64 x 2048 26 -> 14;
-//   16 on 2: 256 x 1024 82 -> 13.8
+// they are below a value's last bit where values are 2^-95 or more.)
+// What bounds it is the VALU work of the softmax (about 22 operations a score)
+// and V's conversion (1.5 a byte, shared by the wave's columns); the matrix
+// cores need about a third of the time.
+// Measured, MI355X, kernel traces with the merge launch where there is one,
+// quant_query, against the per-position kernel that took these calls before (K
+// and V converted to fp32 and multiplied in the VALU for each query head; a
+// prompt's rows each walked their own span):
+//   prompt, 12 on 2 heads, qk 48: 500 rows 52.7 -> 8.8 us, 1000 81 -> 13.5,
+//   2000 236 -> 28.3, 3000 473 -> 49 (12 x 64 MHA: 50 / 128 / 389 / 802 -> 9.8
+//   / 13.9 / 27.9 / 49)
+//   decode, 12 on 2 heads: 64 sessions x 2048 32.8 -> 12.1 us (fp32 query 30.8
+//   -> 13.3), 256 x 1024 45.3 -> 13.7, one session x 8192 24.9 -> 10.8; 8 on 4:
+//   64 x 2048 27.9 -> 14.2; 16 on 2: 256 x 1024 86.8 -> 14.1
+// Four waves a SIMD for one column tile: with 129 registers instead of 128, many
+// short spans took up to a fifth longer (785 sessions of 31 positions, 8 on 4
+// heads: 12.9 and 15.5 us).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 typedef int intx4_t __attribute__((ext_vector_type(4)));

@@ -652,6 +652,9 @@ __global__ __launch_bounds__(kAttn2Threads, 4) void attn_exact2_kernel(
 // Bound by the VALU.  Measured (64 sessions x 32 rows at 512 positions,
 // MI355X): 253 us a layer as workgroups of one (row, head), 96 so over a
 // prompt (55 with six heads a wave on its short spans, 143 with three on its long).
+// Six heads a kv head, qk 48 and v 64 are the shipped geometry's and set the
+// lane layout; any other grouping, and the f32 cache, keep the workgroup a (row,
+// head) and its time.
 constexpr int kRowHeads = 6, kRowQk = 48, kRowVd = 64;
 // Where it pays (ms a pass of all 20 layers, this kernel / the workgroup a
 // (row, head)): a wave takes its spans in sequence, so it needs four of them

@@ -1574,7 +1574,10 @@ __global__ __launch_bounds__(1024) void k_post_hada(HadaArgs a, MhcIn mhc)
 // and t[k][.] never leaves the wave.  The operations of a row and their order
 // are those of k_post_hada.
 // Bound by LDS reads and the VALU; measured (2048 rows, MI355X): 128.8 us a
-// layer in workgroups of one row, 53.7 so.
+// layer in workgroups of one row, 53.7 so.  Eight rows take the 128 registers
+// that 1024 threads have and spill six (28 bytes a lane); four rows spill none,
+// but their chains take as long as those of eight: 64 sessions' prompt and 8
+// steps 30.86 ms against 30.44.
 typedef const __attribute__((address_space(4))) float *const_f32;
 
 template <int RB>
