@@ -353,24 +353,28 @@ __global__ __launch_bounds__(256) void x_to_bf16_kernel(const float *__restrict_
     }
 }
 
-// Y[M][N] = X[M][K] . decode(W[N][K])^T, X already bf16, on 128x128 tiles: 4
-// waves of 64x64 (4x4 MFMA tiles each), K steps of 64, each thread staging half
-// a row of A (32 bf16) and of B (32 codes): the next step's are loaded into
+// Y[M][N] = X[M][K] . decode(W[N][K])^T, X already bf16, on 128x128 tiles (NB =
+// 2): 4 waves of 64x64 (4x4 MFMA tiles each), K steps of 64, each thread staging
+// half a row of A (32 bf16) and of B (32 codes); or 128x64 (NB = 1): 4 waves of
+// 32x64, 16 codes a thread, the same order of K: the next step's are loaded into
 // registers while the current step's MFMAs run from LDS.  The codebooks sit in
 // LDS already rounded to bf16, so decoding a code is one LDS read.  With an odd
-// number of 64-column groups the last tile's second half repeats the last row
-// and is not stored.
-constexpr int kBM = 128, kBN = 128, kBK = 64;
+// number of 64-column groups the last 128-wide tile's second half repeats the
+// last row and is not stored.
+constexpr int kBM = 128, kBK = 64;
 
+template <int NB>
 __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *__restrict__ Xb,
                                                           const uint8_t *__restrict__ W,
                                                           const float *__restrict__ cb,
                                                           float *__restrict__ Y, int M, int N,
                                                           int K, size_t ws, size_t cs, size_t ys)
 {
-    __shared__ unsigned short cbh[2][256];
+    constexpr int BN = 64 * NB, MA = 2 * NB;  // columns; a wave's row tiles of 16
+    constexpr int BC = 16 * NB;               // codes a thread stages
+    __shared__ unsigned short cbh[NB][256];
     __shared__ __align__(16) unsigned short As[kBM][kBK + kLdsPad];
-    __shared__ __align__(16) unsigned short Bs[kBN][kBK + kLdsPad];
+    __shared__ __align__(16) unsigned short Bs[BN][kBK + kLdsPad];
 
     Xb += blockIdx.z * size_t(M) * K;
     W += blockIdx.z * ws;
@@ -380,55 +384,58 @@ __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = t >> 6;
-    const int n0 = blockIdx.x * kBN;
+    const int n0 = blockIdx.x * BN;
     const int m0 = blockIdx.y * kBM;
-    const int wm = (wave >> 1) * 64;
-    const int wn = (wave & 1) * 64;
+    const int wm = NB == 2 ? (wave >> 1) * 64 : wave * 32;
+    const int wn = NB == 2 ? (wave & 1) * 64 : 0;
 
-    // the tile's two 64-row codebooks, rounded to bf16
+    // the tile's codebooks, rounded to bf16
     cbh[0][t] = f32_to_bf16_rne(cb[size_t(n0 / 64) * 256 + t]);
-    cbh[1][t] = f32_to_bf16_rne(cb[size_t(min(n0 / 64 + 1, N / 64 - 1)) * 256 + t]);
+    if constexpr (NB == 2) cbh[1][t] = f32_to_bf16_rne(cb[size_t(min(n0 / 64 + 1, N / 64 - 1)) * 256 + t]);
 
-    floatx4_t acc[4][4];
+    floatx4_t acc[MA][4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < MA; ++a)
 #pragma unroll
         for (int b = 0; b < 4; ++b) acc[a][b] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int sr = t >> 1;          // staged row 0..127 (of A and of B)
-    const int sc = (t & 1) * 32;    // staged columns sc..sc+31 of the K step
+    const int sr = t >> 1;          // staged row 0..127 of A
+    const int sc = (t & 1) * 32;    // and columns sc..sc+31 of the K step
+    const int br = NB == 2 ? sr : t >> 2, bc = NB == 2 ? sc : (t & 3) * 16;  // of B, BC columns
     const bool mrow = m0 + sr < M;
     const unsigned short *xrow = Xb + size_t(mrow ? m0 + sr : 0) * K;
-    const uint8_t *wrow = W + size_t(min(n0 + sr, N - 1)) * K;  // N is a multiple of 64
-    const unsigned short *cbr = cbh[sr >> 6];
+    const uint8_t *wrow = W + size_t(min(n0 + br, N - 1)) * K;  // N is a multiple of 64
+    const unsigned short *cbr = cbh[br >> 6];
     uint4 xa[4];
-    uint2 wc[4];
-    // a 32-column run past K reads the one before it and is zeroed at the LDS
+    uint2 wc[BC / 8];
+    // a run of columns past K reads the one before it and is zeroed at the LDS
     // store: no load sits behind a branch
     auto load = [&](int k0) {
         const bool on = k0 + sc < K;
         const int kc = on ? k0 + sc : K - 32;
+        const int kb = NB == 2 ? kc : (k0 + bc < K ? k0 + bc : K - BC);
 #pragma unroll
         for (int q = 0; q < 4; ++q) xa[q] = *reinterpret_cast<const uint4 *>(xrow + kc + 8 * q);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) wc[q] = *reinterpret_cast<const uint2 *>(wrow + kc + 8 * q);
+        for (int q = 0; q < BC / 8; ++q) wc[q] = *reinterpret_cast<const uint2 *>(wrow + kb + 8 * q);
         return on;
     };
-    auto store = [&](bool on) {
+    auto store = [&](bool on, int k0) {
+        const bool onb = NB == 2 ? on : k0 + bc < K;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             *reinterpret_cast<uint4 *>(&As[sr][sc + 8 * q]) = on && mrow ? xa[q] : make_uint4(0, 0, 0, 0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < BC / 8; ++q) {
             const uint32_t d[2] = {wc[q].x, wc[q].y};
             uint32_t h[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const uint32_t lo = cbr[(d[e >> 1] >> (16 * (e & 1))) & 0xffu];
                 const uint32_t hi = cbr[(d[e >> 1] >> (16 * (e & 1) + 8)) & 0xffu];
-                h[e] = on ? lo | (hi << 16) : 0u;
+                h[e] = onb ? lo | (hi << 16) : 0u;
             }
-            *reinterpret_cast<uint4 *>(&Bs[sr][sc + 8 * q]) = make_uint4(h[0], h[1], h[2], h[3]);
+            *reinterpret_cast<uint4 *>(&Bs[br][bc + 8 * q]) = make_uint4(h[0], h[1], h[2], h[3]);
         }
     };
     __syncthreads();
@@ -436,20 +443,20 @@ __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *
     const int r16 = lane & 15;
     const int kq = (lane >> 4) * 8;
     for (int k0 = 0; k0 < K; k0 += kBK) {
-        store(on);
+        store(on, k0);
         __syncthreads();
         if (k0 + kBK < K) on = load(k0 + kBK);
         const int steps = (K - k0 < kBK ? K - k0 : kBK) / 32;
         for (int kk = 0; kk < steps; ++kk) {
-            bf16x8_t afrag[4], bfrag[4];
+            bf16x8_t afrag[MA], bfrag[4];
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < MA; ++a)
                 afrag[a] = *reinterpret_cast<const bf16x8_t *>(&As[wm + a * 16 + r16][kk * 32 + kq]);
 #pragma unroll
             for (int b = 0; b < 4; ++b)
                 bfrag[b] = *reinterpret_cast<const bf16x8_t *>(&Bs[wn + b * 16 + r16][kk * 32 + kq]);
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < MA; ++a)
 #pragma unroll
                 for (int b = 0; b < 4; ++b)
                     acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag[a], bfrag[b],
@@ -460,7 +467,7 @@ __global__ __launch_bounds__(256) void cb8_gemm128_kernel(const unsigned short *
     const int col = lane & 15;
     const int rb = (lane >> 4) * 4;
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < MA; ++a)
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
@@ -909,11 +916,8 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
     // shorter there (us, rows / 128x128 tiles: 192 tiles of 1 x 512 by 3072 x
     // 768 14.0 / 22.1, 384 of 8 x 500 by 768 x 768 23.9 / 29.2, 512 of 4 x 1000
     // by 1024 x 256 14.5 / 15.6, 720 of 6 x 300 by 3072 x 768 34.7 / 33.1, 960
-    // of 20 x 80 by 3072 x 768 46.2 / 32.7).  (One to three groups of 64 columns
-    // leave up to half a 128x128 tile idle; 64x64 tiles would do 200 x 130 rows
-    // by 64 x 768 in 38.6 us against 42.6 and 64 x 2000 by 64 x 96 in 25.4
-    // against 27.8, not worth a kernel.)  Whole lines of codes need them 16-byte
-    // aligned.  Above 64 rows the K order is the larger tiles', so a
+    // of 20 x 80 by 3072 x 768 46.2 / 32.7).  Whole lines of codes need them
+    // 16-byte aligned.  Above 64 rows the K order is the larger tiles', so a
     // problem's bits do not depend on how many share its launch.
     const size_t row_tiles_m = (m + 63) / 64;
     const size_t row_tiles = ((out + kRN - 1) / kRN) * row_tiles_m * count;
@@ -965,10 +969,22 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
                            x_stride, w, cb, y, int(m), int(out), int(in), w_stride, cb_stride, y_stride,
                            int(out / kPN), int((m + kPM - 1) / kPM), run);
     } else {
-        dim3 grid(static_cast<unsigned>((out + kBN - 1) / kBN), static_cast<unsigned>((m + kBM - 1) / kBM),
-                  static_cast<unsigned>(count));
-        hipLaunchKernelGGL(cb8_gemm128_kernel, grid, dim3(256), 0, ctx->stream, xb, w, cb, y,
-                           int(m), int(out), int(in), w_stride, cb_stride, y_stride);
+#define ND_GEMM128(NB)                                                                                 \
+    hipLaunchKernelGGL(cb8_gemm128_kernel<NB>,                                                           \
+                       dim3(unsigned((out + 64 * NB - 1) / (64 * NB)), unsigned((m + kBM - 1) / kBM), unsigned(count)), \
+                       dim3(256), 0, ctx->stream, xb, w, cb, y, int(m), int(out), int(in), w_stride, cb_stride, y_stride)
+        // 128x64 tiles for a small odd number of 64-column groups where half of
+        // the 128x128 tiles' area or more would be idle (us, 128x128 / 128x64: 200
+        // x 130 rows by 64 x 768 43.0 / 36.7, 46 x 2000 by 64 x 96 20.9 / 19.0,
+        // 250 x 130 by 192 x 96 23.9 / 19.3, 416 x 130 by 448 x 256 83.1 / 71.8);
+        // with less idle, or more columns, the wider tile is as fast or faster
+        // (49 x 130 by 4032 x 1408 240 / 287, 448 columns by 500 rows 1.09)
+        const size_t bm = (m + kBM - 1) / kBM * kBM, bn = (out + 127) / 128 * 128;
+        if (out % 128 != 0 && out <= 448 && 2 * m * out <= bm * bn)
+            ND_GEMM128(1);
+        else
+            ND_GEMM128(2);
+#undef ND_GEMM128
     }
     return nd::check_launch("cb8_gemm");
 }

@@ -263,10 +263,12 @@ def test_gemm_rows(ctx, count, m, out, inn):
 
 
 @pytest.mark.parametrize("one,many,m,out,inn", [(1, 30, 65, 2048, 96), (2, 33, 130, 704, 224), (1, 9, 200, 3072, 128),
-                                                (1, 20, 513, 192, 64), (3, 70, 96, 192, 1056)])
+                                                (1, 20, 513, 192, 64), (3, 70, 96, 192, 1056),
+                                                (1, 300, 130, 64, 96), (2, 130, 500, 64, 224),
+                                                (1, 100, 130, 448, 96), (1, 400, 70, 192, 32)])
 def test_gemm_problem_bits_do_not_depend_on_the_launch(ctx, one, many, m, out, inn):
-    """Few problems take 64-row tiles, many 128x128 or 256x256 ones (an odd
-    number of column groups among them): the same bits above 64 rows, and
+    """Few problems take 64-row tiles, many 128x128, 128x64 or 256x256 ones (an
+    odd number of column groups among them): the same bits above 64 rows, and
     within inn roundings of the products of the bf16 operands."""
     rng = np.random.default_rng(m + out)
     W = dev(rng.integers(0, 256, size=(many, out, inn), dtype=np.uint8))
