@@ -569,7 +569,7 @@ def attend_i8_prefill(ctx, num_heads, num_kv_heads, qk, vd, q, k, v, window=0, q
     seq = q.shape[0]
     g = kv_geom(num_heads, num_kv_heads, qk, vd, max(seq, 1))
     blk, _ = kv_alloc(g, 1, q.device.index or 0)
-    if window >= 0 and seq > 0:
+    if isinstance(window, int) and window >= 0 and seq > 0:
         # both ends of the spans in two operations: 1 - w .. seq - 1 clamped to
         # 0 holds every row's first position, then, w - 1 on, its last (its own)
         w = min(window, seq) if window else seq
@@ -577,7 +577,7 @@ def attend_i8_prefill(ctx, num_heads, num_kv_heads, qk, vd, q, k, v, window=0, q
         lo, hi = ends[:seq], ends[w - 1:]
     else:
         hi = torch.arange(seq, dtype=torch.int32, device=q.device)
-        lo = torch.clamp(hi + 1 - window, min=0) if window else torch.zeros_like(hi)
+        lo = torch.clamp(hi + 1 - window, min=0).to(torch.int32) if window else torch.zeros_like(hi)
     kv_write(ctx, g, blk, 0, hi, k.contiguous(), v.contiguous())
     scale = float(np.float32(1.0) / np.float32(math.sqrt(qk)))
     return attend_step_i8(ctx, g, blk, 0, lo, hi, q.contiguous(), scale, quant_query)

@@ -2,6 +2,8 @@
 does, and the spans of a prompt pass are every row's window (no GPU)."""
 import random
 
+import numpy as np
+import pytest
 import torch
 
 import needle_amd as nd
@@ -57,13 +59,19 @@ def test_layout_check_over_shapes_and_strides():
         assert got == want, (shape, strides, rows, numel)
 
 
-def test_prompt_spans(monkeypatch):
+@pytest.fixture
+def seen(monkeypatch):
+    """What a prompt pass would hand to the cache and the attention."""
     seen = {}
     monkeypatch.setattr(nd, "_torch", lambda: torch)
     monkeypatch.setattr(nd, "kv_alloc", lambda g, n, device: (torch.zeros(1, dtype=torch.uint8), 1))
     monkeypatch.setattr(nd, "kv_write", lambda ctx, g, kv, stride, pos, k, v: seen.update(pos=pos))
     monkeypatch.setattr(nd, "attend_step_i8",
                         lambda ctx, g, kv, stride, lo, hi, *rest: seen.update(lo=lo, hi=hi))
+    return seen
+
+
+def test_prompt_spans(seen):
     for seq in range(20):
         for window in (0, 1, 2, 5, 19, 20, 21, 64):
             x = torch.zeros(seq, 16)
@@ -73,3 +81,17 @@ def test_prompt_spans(monkeypatch):
             lo = torch.clamp(t + 1 - window, min=0) if window else torch.zeros_like(t)
             assert torch.equal(seen["lo"], lo) and seen["lo"].dtype == torch.int32
             assert seen["lo"].is_contiguous() and seen["hi"].is_contiguous()
+
+
+@pytest.mark.parametrize("window", [None, False, -1, -7, 5.0, 2.5, 64.0, -2.0, np.int64(5), np.float32(3.0),
+                                    torch.tensor(5), torch.tensor([3])])
+def test_prompt_spans_of_any_number(seen, window):
+    """A window is any number, or None for the whole prompt: spans as from
+    row + 1 - window, a fraction cut off."""
+    for seq in (1, 7, 20):
+        x = torch.zeros(seq, 16)
+        nd.attend_i8_prefill(None, 1, 1, 16, 16, x, x, x, window=window)
+        t = torch.arange(seq, dtype=torch.int32)
+        lo = torch.clamp(t + 1 - window, min=0).to(torch.int32) if window else torch.zeros_like(t)
+        assert torch.equal(seen["lo"], lo) and torch.equal(seen["hi"], t)
+        assert seen["lo"].dtype == seen["hi"].dtype == torch.int32
