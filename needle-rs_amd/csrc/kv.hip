@@ -407,8 +407,8 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 //           takes V columns 4 n + c, so a lane's V bytes come as one dword a
 //           position and no byte is moved between lanes.
 // Every product is exact and the sums are fp32 (or int32): nothing is held in
-// 16 bits.  (A weight's bits below 2^-126, of a value below 2^-119, are lost:
-// they are below a value's last bit where values are 2^-95 or more.)
+// 16 bits.  (A bf16 piece has no bit below 2^-126: a column that has met V
+// scales below 2^-64 only takes its softmax against a maximum 64 bits lower.)
 // What bounds it is the VALU work of the softmax (about 22 operations a score)
 // and V's conversion (1.5 a byte, shared by the wave's columns); the matrix
 // cores need about a third of the time.
@@ -422,6 +422,9 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 //   decode, 12 on 2 heads: 64 sessions x 2048 32.8 -> 12.1 us (fp32 query 30.8
 //   -> 13.3), 256 x 1024 45.3 -> 13.7, one session x 8192 24.9 -> 10.8; 8 on 4:
 //   64 x 2048 27.9 -> 14.2; 16 on 2: 256 x 1024 86.8 -> 14.1
+// Watching for small V scales costs 0.1 to 0.3 us of these (64 x 2048 11.6 -> 11.9
+// in calls back to back, 2000 rows of a window of 256 14.7 -> 15.0); told by a second
+// walk of the few columns that need it, 0.3 to 0.7 us on short spans.
 // Four waves a SIMD for one column tile: with 129 registers instead of 128, many
 // short spans took up to a fifth longer (785 sessions of 31 positions, 8 on 4
 // heads: 12.9 and 15.5 us).
@@ -665,9 +668,16 @@ __global__ __launch_bounds__(NW * 64, NT == 1 ? 4 : 1) void attn_mm_kernel(
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[x][c] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
+    // As long as every V scale of the column is below 2^-64 its sums are taken
+    // against a maximum 64 bits lower: its weights' pieces are normal numbers.
+    bool low[NT], any_low = true;
+#pragma unroll
+    for (int x = 0; x < NT; ++x) low[x] = true;
 
     while (more) {
         const uint32_t pc = p0;
+        // positions of the chunk whose V scale is 2^-64 or more
+        const uint32_t normal = uint32_t(__ballot(!(__builtin_fabsf(scr) < 0x1p-64f)) >> 32);
         // the chunk's scales, from position order to the score tiles' rows
         sc_s[w][lane] = scr;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -754,10 +764,29 @@ __global__ __launch_bounds__(NW * 64, NT == 1 ? 4 : 1) void attn_mm_kernel(
             m_new[x] = max3(__uint_as_float(s32[0]), __uint_as_float(s32[1]), m16);
             grew = grew || m_new[x] > m_run[x];
         }
+        bool up[NT];
+#pragma unroll
+        for (int x = 0; x < NT; ++x) up[x] = false;
+        if (any_low) {
+            bool still = false;
+#pragma unroll
+            for (int x = 0; x < NT; ++x) {
+                // the column's own of them, from its first position to its last (one
+                // span for all columns of a row: scalar)
+                const uint32_t first = max(SHARED ? lo[x] : ulo, pc), last = min(SHARED ? hi[x] : uhi, pc + 31u);
+                const uint32_t own = (normal >> ((first - pc) & 31u)) << ((first - last - 1u) & 31u);
+                up[x] = low[x] && ((SHARED && bad[x]) || (first <= last && own != 0));
+                low[x] = low[x] && !up[x];
+                grew = grew || up[x];
+                still = still || low[x];
+            }
+            any_low = __any(still);
+        }
         if (__any(grew)) {
 #pragma unroll
             for (int x = 0; x < NT; ++x) {
-                const float al = m_new[x] > m_run[x] ? __builtin_amdgcn_exp2f(m_run[x] - m_new[x]) : 1.0f;
+                float al = m_new[x] > m_run[x] ? __builtin_amdgcn_exp2f(m_run[x] - m_new[x]) : 1.0f;
+                al = up[x] ? al * 0x1p-64f : al;
                 m_run[x] = m_new[x];
                 l_run[x] *= al;
 #pragma unroll
@@ -767,7 +796,7 @@ __global__ __launch_bounds__(NW * 64, NT == 1 ? 4 : 1) void attn_mm_kernel(
         uint32_t pp[NT][3][4];
 #pragma unroll
         for (int x = 0; x < NT; ++x) {
-            const float mu = m_run[x] == -INFINITY ? 0.0f : m_run[x];
+            const float mu = (m_run[x] == -INFINITY ? 0.0f : m_run[x]) - (low[x] ? 64.0f : 0.0f);
             float wt[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -814,7 +843,7 @@ __global__ __launch_bounds__(NW * 64, NT == 1 ? 4 : 1) void attn_mm_kernel(
         const int col = 16 * x + n;
         if (col < COLS) {
             if (qd == 0) {
-                mm[w][col] = bad[x] ? NAN : m_run[x];
+                mm[w][col] = bad[x] ? NAN : m_run[x] - (low[x] ? 64.0f : 0.0f);
                 ml[w][col] = l;
             }
             // lane (n, qd) holds V columns 16 qd + 4 i + c
