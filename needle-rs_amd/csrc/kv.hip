@@ -962,8 +962,9 @@ bool attn_shape(int rep, int qk, int vd)
     return r && (qk == 48 || qk == 64) && vd == 64;
 }
 
-// The matrix-core kernel takes every prompt, and every decode call with two
-// or more query heads a kv head (figures at the kernel).  One query head a kv
+// The matrix-core kernel takes every prompt but the shortest of one query head a
+// kv head (figures at the rule), and every decode call with two or more query
+// heads a kv head (figures at the kernel).  One query head a kv
 // head stays with attn_i8_kernel: its column tile would be 1/16 full, and
 // where the caches stream from HBM it is the faster of the two (12 x 64, 256
 // sessions x 1024: 70 against 77-85 us; 64 x 512: 11.5 against 11.6-13.1).
@@ -1103,7 +1104,13 @@ int attend_i8(nd_ctx *ctx, const nd_kv_geom *g, const void *kv, size_t kv_stride
     bool base2 = true;
     AttnFn fn;
     dim3 grid;
-    if (kv_stride == 0 && count > 1) {
+    // A short prompt with one query head a kv head, in blocks of one row: as long
+    // as each has a CU of its own, a tile of 16 rows only waits longer (us, 12
+    // heads, matrix cores / rows: 8 rows 5.0 / 4.3, 20 rows 5.5 / 4.4, 17 rows in a
+    // ring of 243 4.9 / 4.5, 10 in one of 776 7.8 / 7.0; 26 rows 5.4 / 5.5, 46 rows
+    // 5.2 / 6.3, 16 in a ring of 1995 7.4 / 8.4, 12 in one of 3445 7.4 / 9.1)
+    const bool few_rows = rep < kMmMinRep && pairs * max_splits <= cus;
+    if (kv_stride == 0 && count > 1 && !few_rows) {
         // A prompt's rows over one block.  Two column tiles a wave share V's
         // conversion once that leaves four blocks a CU (3000 rows, 12 on 2:
         // 53 against 57 us; 2000: 31 against 29); with fewer than two

@@ -103,6 +103,23 @@ def test_prompt_rows(ctx, H, KVH, QK, seq, window, quant):
 
 
 @pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("H,QK", [(12, 64), (32, 48)])
+@pytest.mark.parametrize("cap", [30, 512, 513])
+@pytest.mark.parametrize("over", [0, 1])
+def test_few_rows_of_one_head_each(ctx, H, QK, cap, over, quant):
+    """One query head a kv head, as many (row, head) pairs as CUs and a row
+    more, rings on both sides of a split: wrapped, windowed and bad spans."""
+    rng = np.random.default_rng(cap + H)
+    rows = torch.cuda.get_device_properties(0).multi_processor_count // H + over
+    g, blk, nb = _block(ctx, rng, H, H, QK, cap, 2 * cap)
+    hi = 2 * cap - 1 - np.arange(rows) % cap
+    lo = np.maximum(hi + 1 - rng.integers(1, cap + 1, rows), cap)
+    lo[0], hi[0], lo[1] = cap, 2 * cap - 1, hi[1] + 1
+    q = rng.normal(size=(rows, H * QK)).astype(np.float32)
+    _check(ctx, g, blk, nb, lo, hi, q, quant, True)
+
+
+@pytest.mark.parametrize("quant", [False, True])
 def test_shared_block_any_spans(ctx, quant):
     """Rows over one ring in any order with spans that share nothing, among
     them bad ones (NaN, that row alone) and positions far apart."""
