@@ -899,33 +899,45 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(Geom g, int nchunks,
                                                                const float *__restrict__ part_ml,
                                                                float *__restrict__ out)
 {
-    // the partials' factors, 64 at a time in the lanes, then one column a lane
+    // a lane a column (v is 64 wherever attention is split); the partials'
+    // factors 64 at a time in the lanes, four partials loaded ahead
     const size_t qi = blockIdx.y;
     const int head = blockIdx.x, lane = threadIdx.x;
     const size_t base = (qi * g.H + head) * size_t(nchunks);
-    __shared__ float fs[64], ls[64];
-    float M = -INFINITY;
-    for (int c = lane; c < nchunks; c += 64) M = fmaxf(M, part_ml[(base + c) * 2]);
+    const float *po = part_o + base * 64 + lane;
+    const float2 *mls = reinterpret_cast<const float2 *>(part_ml) + base;
+    auto load_ml = [&](int c) { return c < nchunks ? mls[c] : make_float2(-INFINITY, 0.0f); };
+    float2 ml = load_ml(lane);
+    float o[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) o[u] = po[size_t(min(u, nchunks - 1)) * 64];
+    float M = ml.x;
+    for (int c = lane + 64; c < nchunks; c += 64) M = fmaxf(M, mls[c].x);
     M = wave_max(M);
-    for (int col = lane; col < g.VD; col += 64) {
-        float O = 0.0f, L = 0.0f;
-        for (int c0 = 0; c0 < nchunks; c0 += 64) {
-            const int nc = min(64, nchunks - c0);
-            __syncthreads();
-            if (lane < nc) {
-                const float m = part_ml[(base + c0 + lane) * 2];
-                fs[lane] = m == -INFINITY ? 0.0f : (BASE2 ? exp2f(m - M) : expf(m - M));
-                ls[lane] = m == -INFINITY ? 0.0f : part_ml[(base + c0 + lane) * 2 + 1];
-            }
-            __syncthreads();
-#pragma unroll 4
-            for (int c = 0; c < nc; ++c) {
-                O += part_o[(base + c0 + c) * g.VD + col] * fs[c];
-                L += ls[c] * fs[c];
+    float O = 0.0f, L = 0.0f;
+    for (int c0 = 0; c0 < nchunks; c0 += 64) {
+        if (c0) ml = load_ml(c0 + lane);
+        const float f = ml.x == -INFINITY ? 0.0f : (BASE2 ? exp2f(ml.x - M) : expf(ml.x - M));
+        const float l = ml.x == -INFINITY ? 0.0f : ml.y;
+        const int nc = min(64, nchunks - c0);
+        for (int c = 0; c < nc; c += 4) {
+            float next[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) next[u] = po[size_t(min(c0 + c + 4 + u, nchunks - 1)) * 64];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                // past the end: lane 63's or -inf's factor, left out
+                const float fc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), min(c + u, 63)));
+                const float lc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(l), min(c + u, 63)));
+                if (c + u < nc) {
+                    O += o[u] * fc;
+                    L += lc * fc;
+                }
+                o[u] = next[u];
             }
         }
-        out[qi * size_t(g.H) * g.VD + size_t(head) * g.VD + col] = O / L;
     }
+    out[(qi * size_t(g.H) + head) * 64 + lane] = O / L;
 }
 
 using AttnFn = void (*)(dim3, hipStream_t, Geom, const uint8_t *, size_t, const int32_t *,

@@ -119,6 +119,18 @@ def test_few_rows_of_one_head_each(ctx, H, QK, cap, over, quant):
     _check(ctx, g, blk, nb, lo, hi, q, quant, True)
 
 
+@pytest.mark.parametrize("H,KVH,QK,cap", [(12, 12, 64, 40000), (8, 1, 64, 34000), (12, 12, 64, 1100),
+                                          (12, 12, 64, 2700), (12, 2, 48, 1100), (8, 1, 64, 1500)])
+def test_merge_of_split_spans(ctx, H, KVH, QK, cap):
+    """One session, its span split over two to more than 64 blocks: whole, a few
+    positions (most partials empty), an end, and a bad one."""
+    rng = np.random.default_rng(cap + KVH)
+    g, blk, nb = _block(ctx, rng, H, KVH, QK, cap, cap)
+    for lo, hi in [(0, cap - 1), (5, 7), (cap - 300, cap - 1), (cap // 3, cap // 2), (9, 8)]:
+        q = rng.normal(size=(1, H * QK)).astype(np.float32)
+        _check(ctx, g, blk, nb, [lo], [hi], q, False, False)
+
+
 @pytest.mark.parametrize("quant", [False, True])
 def test_shared_block_any_spans(ctx, quant):
     """Rows over one ring in any order with spans that share nothing, among
