@@ -665,9 +665,12 @@ __global__ __launch_bounds__(512) void cb8_gemm256_kernel(const float *__restric
 // by 768 x 3072 48.9 -> 30.5; 64 x 64 rows by 1024 x 3072 78.0 -> 59.0, by 3072
 // x 768 63.3 -> 51.0, 448 of these, far past the caches, 409 -> 405.  32 columns
 // and half the step a wave: 21.2 and 14.7 us for 20 problems of 64 and 16 rows.
-// A tile fills a table of 32 KB first, which a K of 32 to 128 does not repay
-// once a launch has thousands of tiles: 200 x 64 rows by 1984 x 32 25.6 -> 31,
-// 2000 x 1 by 192 x 128 24.2 -> 28.
+// Up to a K of 128 (ONE) there is one step: nothing is loaded ahead, pieces past
+// K are left out, and without a second buffer of X three blocks of 64 rows share
+// a CU where two did.  us, 64x64 tiles before / with the steps' loop / so: 200 x
+// 64 rows by 1984 x 32 26.7 / 33.2 / 21.0, 104 x 56 by 5312 x 96 37.6 / 43.5 /
+// 30.7, 158 x 46 by 5440 x 128 71.9 / 76.7 / 47.0, 2000 x 1 by 192 x 128 24.4 /
+// 28.5 / 15.5.
 // Blocks of 512 threads a launch may have: HIP counts the threads of a dimension
 // in 32 bits, and a launch of more leaves blocks out.
 constexpr size_t kMaxBlocks512 = 0xffffffffu / 512;
@@ -675,8 +678,8 @@ constexpr int kRN = 128;          // output columns (N) per block: two codebook 
 constexpr int kRC = 128;          // K per step
 constexpr int kRXS = kRC + 8;     // padded X row in LDS (bf16)
 
-template <int MT, bool LINES>
-__global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__restrict__ X, size_t xstride,
+template <int MT, bool LINES, bool ONE>
+__global__ __launch_bounds__(512, ONE ? 6 : 4) void cb8_gemm_rows_kernel(const float *__restrict__ X, size_t xstride,
                                                                const uint8_t *__restrict__ W,
                                                                const float *__restrict__ cb,
                                                                float *__restrict__ Y, int M, int N, int K,
@@ -684,7 +687,8 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
                                                                int tiles_m, int xcd_run)
 {
     __shared__ __align__(16) uint32_t tab[257 * 32];  // a zero entry behind the codebook
-    __shared__ __align__(16) unsigned short xs[2][16 * MT * kRXS];
+    __shared__ __align__(16) unsigned short xs[ONE ? 1 : 2][16 * MT * kRXS];
+    __shared__ uint32_t one_vals[ONE ? 256 : 1];
     // the column tiles of one problem are consecutive in u and land on one
     // XCD (workgroups are dealt to the 8 XCDs round-robin), sharing X in L2
     const int id = blockIdx.x;
@@ -742,11 +746,12 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     };
     xload(0);
     cload(0, 0);
-    cload(1, 1);
+    if constexpr (!ONE) cload(1, 1);
     {
-        // the table, through a staging row in xs[1] so every write is
-        // conflict-free: word e of the staging row, then 4 x 16 bytes a thread
-        uint32_t *vals = reinterpret_cast<uint32_t *>(&xs[1][0]);
+        // the table, through a staging row (in xs[1] where there is one) so
+        // every write is conflict-free: word e of the row, then 4 x 16 bytes a
+        // thread
+        uint32_t *vals = ONE ? one_vals : reinterpret_cast<uint32_t *>(&xs[ONE ? 0 : 1][0]);
         const int ng = N / 64 - 1;
         if (t < 256)
             vals[t] = f32_to_bf16_rne(cb[size_t(n0 / 64) * 256 + t]) |
@@ -761,7 +766,7 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     }
     if (t < 32) tab[256 * 32 + t] = 0;
     xstore(0, 0);
-    xload(1);
+    if constexpr (!ONE) xload(1);
     __syncthreads();
     // waves 0-3 hold rows of the first group (low halves), 4-7 the second
     const uint32_t sel = w >= 4 ? 0x07060302u : 0x05040100u;
@@ -786,13 +791,26 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
     };
     // piece h of a step, eight codes: where its k start for this lane
     auto piece = [&](int h) { return LINES ? 64 * (h >> 1) + 8 * (h & 1) + k0 : 32 * h + k0; };
-    for (int c0 = 0; c0 < nc; c0 += 2) {
+    if constexpr (ONE) {
+        // pieces wholly past K are left out
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+            if ((LINES ? 64 * (h >> 1) : 32 * h) < K) {
+                const bf16x8_t b = decode(cw[0][h >> 1][2 * (h & 1)], cw[0][h >> 1][2 * (h & 1) + 1], piece(h) < K);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        *reinterpret_cast<const bf16x8_t *>(&xs[0][(16 * mt + r16) * kRXS + piece(h)]), b, acc[mt], 0, 0, 0);
+            }
+        __syncthreads();
+    }
+    for (int c0 = 0; !ONE && c0 < nc; c0 += 2) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int c = c0 + s;
             if (c < nc) {
                 // X of step c + 1 into the buffer that step c - 1 read
-                xstore(s ^ 1, c + 1);
+                xstore(ONE ? 0 : s ^ 1, c + 1);
                 xload(c + 2);
                 bf16x8_t b[4];
 #pragma unroll
@@ -805,7 +823,7 @@ __global__ __launch_bounds__(512, 4) void cb8_gemm_rows_kernel(const float *__re
 #pragma unroll
                     for (int h = 0; h < 4; ++h)
                         acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            *reinterpret_cast<const bf16x8_t *>(&xs[s][(16 * mt + r16) * kRXS + piece(h)]), b[h],
+                            *reinterpret_cast<const bf16x8_t *>(&xs[ONE ? 0 : s][(16 * mt + r16) * kRXS + piece(h)]), b[h],
                             acc[mt], 0, 0, 0);
                 __syncthreads();
             }
@@ -945,22 +963,29 @@ int nd_cb8_gemm_batched(nd_ctx *ctx, size_t count, const float *x, size_t x_stri
         for (size_t z0 = 0; z0 < count; z0 += most) {
             const size_t blocks = (count - z0 < most ? count - z0 : most) * tiles;
             const int run = blocks % 8 == 0 ? int(blocks / 8) : 0;
-#define ND_GEMM_ROWS(MT, LINES)                                                                         \
-    hipLaunchKernelGGL((cb8_gemm_rows_kernel<MT, LINES>), dim3(unsigned(blocks)), dim3(512), 0, ctx->stream, \
+#define ND_GEMM_ROWS(MT, LINES)              \
+    if (in <= size_t(kRC))                   \
+        ND_GEMM_ROWS_ONE(MT, LINES, true);   \
+    else                                     \
+        ND_GEMM_ROWS_ONE(MT, LINES, false)
+#define ND_GEMM_ROWS_ONE(MT, LINES, ONE)                                                                \
+    hipLaunchKernelGGL((cb8_gemm_rows_kernel<MT, LINES, ONE>), dim3(unsigned(blocks)), dim3(512), 0, ctx->stream, \
                        x + z0 * x_stride, x_stride, w + z0 * w_stride, cb + z0 * cb_stride,             \
                        y + z0 * y_stride, int(m), int(out), int(in), w_stride, cb_stride, y_stride,     \
                        int(tiles_n), int(row_tiles_m), run)
-            if (!lines)
+            if (!lines) {
                 ND_GEMM_ROWS(4, false);
-            else if (m <= 16)
+            } else if (m <= 16) {
                 ND_GEMM_ROWS(1, true);
-            else if (m <= 32)
+            } else if (m <= 32) {
                 ND_GEMM_ROWS(2, true);
-            else
+            } else {
                 ND_GEMM_ROWS(4, true);
+            }
             if (int rc = nd::check_launch("cb8_gemm")) return rc;
         }
 #undef ND_GEMM_ROWS
+#undef ND_GEMM_ROWS_ONE
     } else if (use_256) {
         // at least one 256x256 tile per CU: below that the 128x128 tiles fill
         // the chip better

@@ -301,6 +301,39 @@ def test_gemm_codes_aligned_to_eight_bytes(ctx):
     assert torch.all((y - x @ v.T).abs() <= (x.abs() @ v.abs().T) * inn * 2.0 ** -23)
 
 
+@pytest.mark.parametrize("m", [1, 17, 33, 64])
+@pytest.mark.parametrize("out", [64, 192])
+@pytest.mark.parametrize("shift", [0, 8])
+@pytest.mark.parametrize("inn", [32, 64, 96, 128])
+def test_gemm_of_one_step(ctx, inn, shift, out, m):
+    """K up to 128 takes one step: bit for bit the product with X continued by
+    zeros to a K of several, and within inn roundings of the 64-bit one."""
+    rng = np.random.default_rng(inn + out + m)
+    wide = 288
+
+    def codes(w):
+        raw = torch.zeros(w.size + shift, dtype=torch.uint8, device="cuda")
+        view = raw[shift:].view(w.shape)
+        view.copy_(dev(w))
+        assert view.data_ptr() % 16 == shift
+        return view
+
+    W = rng.integers(0, 256, size=(2, out, wide), dtype=np.uint8)
+    CB = dev(rng.normal(0, 0.02, size=(2, out // 64, 256)).astype(np.float32))
+    X = rng.normal(size=(2, m, wide)).astype(np.float32)
+    X[:, :, inn:] = 0.0
+    Y, Z = (torch.full((2, m, out), 7.0, device="cuda") for _ in range(2))
+    Wn = codes(np.ascontiguousarray(W[:, :, :inn]))
+    Xn = dev(np.ascontiguousarray(X[:, :, :inn]))
+    nd.cb8_gemm_batched(ctx, Xn, Wn, CB, Y)
+    nd.cb8_gemm_batched(ctx, dev(X), codes(W), CB, Z)
+    assert torch.equal(Y, Z)
+    for i in range(2):
+        v = torch.gather(CB[i].bfloat16().double().repeat_interleave(64, 0), 1, Wn[i].long())
+        x = Xn[i].bfloat16().double()
+        assert torch.all((Y[i].double() - x @ v.T).abs() <= (x.abs() @ v.abs().T) * inn * 2.0 ** -23)
+
+
 def test_gemm_more_tiles_than_a_launch_holds(ctx):
     """65,535 one-row problems over one weight of 129 column tiles: 8,454,015
     row tiles, more than a grid of 512-thread blocks may have (8,388,607).
