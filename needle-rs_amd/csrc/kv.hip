@@ -416,15 +416,16 @@ __global__ __launch_bounds__(kThreads) void attn_i8_kernel(
 // quant_query, against the per-position kernel that took these calls before (K
 // and V converted to fp32 and multiplied in the VALU for each query head; a
 // prompt's rows each walked their own span):
-//   prompt, 12 on 2 heads, qk 48: 500 rows 52.7 -> 8.8 us, 1000 81 -> 13.5,
-//   2000 236 -> 28.3, 3000 473 -> 49 (12 x 64 MHA: 50 / 128 / 389 / 802 -> 9.8
-//   / 13.9 / 27.9 / 49)
-//   decode, 12 on 2 heads: 64 sessions x 2048 32.8 -> 12.1 us (fp32 query 30.8
-//   -> 13.3), 256 x 1024 45.3 -> 13.7, one session x 8192 24.9 -> 10.8; 8 on 4:
-//   64 x 2048 27.9 -> 14.2; 16 on 2: 256 x 1024 86.8 -> 14.1
-// Watching for small V scales costs 0.1 to 0.3 us of these (64 x 2048 11.6 -> 11.9
-// in calls back to back, 2000 rows of a window of 256 14.7 -> 15.0); told by a second
-// walk of the few columns that need it, 0.3 to 0.7 us on short spans.
+//   prompt, 12 on 2 heads, qk 48: 500 rows 52.7 -> 8.7 us, 1000 81 -> 13.2,
+//   2000 236 -> 29.9, 3000 473 -> 55 (12 x 64 MHA: 50 / 128 / 389 / 802 -> 9.5
+//   / 14.2 / 30.2 / 57)
+//   decode, 12 on 2 heads: 64 sessions x 2048 32.8 -> 12.0 us (fp32 query 30.8
+//   -> 13.2), 256 x 1024 45.3 -> 13.6, one session x 8192 24.9 -> 10.4; 8 on 4:
+//   64 x 2048 27.9 -> 14.4; 16 on 2: 256 x 1024 86.8 -> 14.2
+// Watching for small V scales costs 2 % of these and 0.1 us of the shortest (calls
+// back to back: 64 sessions x 2048 11.6 -> 11.9 us, 2000 rows 26.3 -> 27.0, 3000 47.6
+// -> 49.0).  Found out afterwards, by a second walk of the columns that need it,
+// it costs half as much of long prompts, and 0.5 us of short spans in 16-wave blocks.
 // Four waves a SIMD for one column tile: with 129 registers instead of 128, many
 // short spans took up to a fifth longer (785 sessions of 31 positions, 8 on 4
 // heads: 12.9 and 15.5 us).
